@@ -22,6 +22,16 @@
 #define AKMC_ZONE_FULL32 2
 #define AKMC_ZONE_FULL64 4
 #define AKMC_ZONE_RESET 8
+// the walker's searches run in the resident kernel (search_resident.hip);
+// its FULL bits then ask the chain of list and pair kernels for one
+// evaluation of all its atoms in that precision
+#define AKMC_ZONE_RES 16
+// capacities of a resident walker: free atoms, zone atoms, atoms of the
+// cell, candidates of its list build
+#define AKMC_RES_FREE 256
+#define AKMC_RES_SLOTS 2048
+#define AKMC_RES_ATOMS 16383
+#define AKMC_RES_CAND 4096
 // cells per axis are capped so a walker's grid fits one workgroup's LDS
 #define AKMC_MAX_CELLS_AXIS 16
 #define AKMC_MAX_WALKER_CELLS (AKMC_MAX_CELLS_AXIS * AKMC_MAX_CELLS_AXIS * AKMC_MAX_CELLS_AXIS)
@@ -120,6 +130,26 @@ struct WalkerOut {
     double stress[6];
 };
 
+// Resident search walkers (search_resident.hip): the atoms their free atoms
+// reach and the short lists a search evaluation runs over, per walker
+struct ResidentDev {
+    int on;
+    int fcap;                  // entries per free atom's list
+    int *n;                    // [W] zone atoms (slots), -1: lists to be built
+    uint16_t *slot;            // [W][RES_SLOTS] slot -> local atom, ascending
+    unsigned long long *mask;  // [W][RES_SLOTS][4] free atoms in reach of a frozen
+                               // slot: free atom f is bit f / 4 of word f % 4
+    uint16_t *fslot;           // [W][RES_FREE] free atom -> slot
+    uint16_t *flist;           // [W][RES_FREE][fcap] neighbours (slots) of a free atom
+    int *fcnt;                 // [W][RES_FREE]
+    double *ref;               // [W][3][RES_FREE] free positions at the list build
+    double *eout;              // [W][2][2] energies of the atoms outside the zone
+                               // (precision; embedding, pair)
+    int *eok;                  // [W] bit 0 / 1: the FP32 / FP64 ones are current
+    double *base_rho[2];       // [A] density from frozen neighbours (precision)
+    double *base_ep[2];        // [A] half pair energies with frozen neighbours
+};
+
 struct BatchDev {
     int A, W, maxnb, ncells_total, nk_total, G1, maxnk;
     int lpa;              // lanes per atom of the Sutton-Chen pair kernels (1, 2, 4)
@@ -200,6 +230,9 @@ struct BatchDev {
     int *wl_count;        // [4] chunks per list
     int wl_grid_staged;   // persistent grids of those kernels (multiples of 8)
     int wl_grid_plain;
+    int zone_off;         // zones are off: every evaluation covers all atoms (resident
+                          // walkers are then served by the chain on every step)
+    ResidentDev r;
 };
 
 // entry k of atom i's neighbour list in the 32-bit form (local index and
@@ -296,6 +329,7 @@ struct WalkerState {
     // status, force calls and iterations of its relax
     double eb2, eb2_64, b2_maxd2;
     int b2_new, b2_status, b2_calls, b2_iters;
+    int too_big;  // the walker does not fit the resident kernel's capacities
 };
 
 struct SearchDev {
@@ -324,6 +358,18 @@ struct SearchDev {
     int final64;                      // relaxes end with one FP64 energy evaluation
 };
 
+// after pass 1 of the chain: what frozen neighbours contribute to the
+// density and pair energy of every atom of the resident walkers it serves
+void akmc_launch_res_base(const BatchDev &b, const FieldDev &hf, hipStream_t st);
+// up to nsteps micro-steps of every resident walker (evaluation and state
+// machine); logic 0: one evaluation each, nothing else
+void akmc_launch_search_resident(const BatchDev &b, const FieldDev &hf, const SearchDev &s, int nsteps, int logic,
+                                 hipStream_t st);
+// every resident walker goes over to the chain (fresh zone, full evaluations)
+void akmc_launch_leave_resident(const BatchDev &b, hipStream_t st);
+// 0 general pair table, 1 one species pair with n = 9, m = 6, 2 every
+// species pair present with n = 9, m = 6
+int akmc_sc_kind(const FieldDev &hf);
 void akmc_launch_search_logic(const BatchDev &b, const SearchDev &s, hipStream_t st);
 // the same state machines in 1024-thread workgroups (large walkers)
 void akmc_launch_search_logic_wide(const BatchDev &b, const SearchDev &s, hipStream_t st);
@@ -346,9 +392,9 @@ struct StartItem {
     WalkerState ws;
 };
 // scatters the starts and asks each started walker for a list rebuild on
-// its first micro-step (zflag and harvested may be null)
+// its first micro-step (zflag, harvested and res_n may be null)
 void akmc_launch_start_walkers(const BatchDev &b, const SearchDev &s, const StartItem *items, int nitems, int *zflag,
-                               int *harvested, hipStream_t st);
+                               int *harvested, int *res_n, hipStream_t st);
 // copies the positions X of every walker that has ended and is not yet
 // harvested into out ([3][A], host memory mapped for the device) and marks it
 void akmc_launch_harvest_pack(const BatchDev &b, const SearchDev &s, int *harvested, double *out, hipStream_t st);

@@ -158,6 +158,13 @@ struct akmc_batch_s {
     bool logic_wide = false;
     int *zflag = nullptr, *zmark = nullptr, *zlist = nullptr, *nz = nullptr;
     std::vector<int> hzflag;
+    // resident searches (search_resident.hip): their lists, off for good once
+    // a walker has not fit them, and whether the captured graph is for a batch
+    // whose running walkers are all resident
+    ResidentDev r{};
+    bool res_off = false;
+    int nmax = 0;
+    int graph_res = 0;
     // kernel variants of the search micro-steps' Sutton-Chen passes:
     // (lanes, unroll, staged) of pass 1, of pass 2, then of the FP64 passes
     // of mixed steps; lanes 0: the default
@@ -707,6 +714,7 @@ int batch_build(akmc_field_t f, int W, const int *natoms, const double *lat, akm
         int nmax = 0;
         for (int w = 0; w < W; ++w) nmax = std::max(nmax, natoms[w]);
         d.nb16 = (f->kind == 0 && f->min_image && nmax <= 65535) ? 1 : 0;
+        b->nmax = nmax;
         // above this size a 256-thread workgroup loops 64 times over a
         // walker's atoms per vector operation of its state machine
         constexpr int kWideLogicAtoms = 16384;
@@ -1086,7 +1094,68 @@ void drop_graph(akmc_batch_t b)
 bool zone_usable(akmc_batch_t b)
 {
     const FieldDev &h = b->f->host;
-    return b->zone_on && b->zflag && h.kind == 0 && !h.eam && h.min_image;
+    return b->zflag && h.kind == 0 && !h.eam && h.min_image;
+}
+
+// bytes of a resident walker's lists
+size_t resident_bytes(akmc_batch_t b)
+{
+    return AKMC_RES_SLOTS * 34 + AKMC_RES_FREE * (30 + 2 * (size_t)b->d.maxnb) + 64;
+}
+
+// searches may run in the resident kernel: zones apply, and the walkers,
+// the field's pair table and the lists' memory are within its capacities
+bool resident_usable(akmc_batch_t b)
+{
+    constexpr size_t kMaxBytes = (size_t)8 << 30;
+    return zone_usable(b) && !b->res_off && b->f->host.nspec <= 4 && b->nmax <= AKMC_RES_ATOMS &&
+           resident_bytes(b) * b->W <= kMaxBytes;
+}
+
+// a search of m free atoms of the walker w runs there
+bool resident_walker(akmc_batch_t b, int w)
+{
+    const int m = b->hnact[w];
+    return m > 0 && m < b->hw[w].n && m <= AKMC_RES_FREE && resident_usable(b);
+}
+
+int ensure_resident(akmc_batch_t b)
+{
+    if (b->r.on) return AKMC_SUCCESS;
+    const size_t W = b->W, A = b->A;
+    ResidentDev r{};
+    r.fcap = b->d.maxnb;
+    TRY(dalloc(b, &r.n, W));
+    TRY(dalloc(b, &r.slot, W * AKMC_RES_SLOTS));
+    TRY(dalloc(b, &r.mask, W * AKMC_RES_SLOTS * 4));
+    TRY(dalloc(b, &r.fslot, W * AKMC_RES_FREE));
+    TRY(dalloc(b, &r.flist, W * AKMC_RES_FREE * r.fcap));
+    TRY(dalloc(b, &r.fcnt, W * AKMC_RES_FREE));
+    TRY(dalloc(b, &r.ref, W * 3 * AKMC_RES_FREE));
+    TRY(dalloc(b, &r.eout, W * 4));
+    TRY(dalloc(b, &r.eok, W));
+    for (int p = 0; p < 2; ++p) {
+        TRY(dalloc(b, &r.base_rho[p], A));
+        TRY(dalloc(b, &r.base_ep[p], A));
+    }
+    r.on = 1;
+    b->r = r;
+    return AKMC_SUCCESS;
+}
+
+// how the running walkers' micro-steps run: 0 the chain alone, 1 the chain
+// and the resident kernel, 2 every running walker is resident
+int resident_mode(akmc_batch_t b)
+{
+    if (!b->r.on || b->res_off) return 0;
+    int res = 0, other = 0;
+    for (int w = 0; w < b->W; ++w) {
+        const WalkerState &ws = b->hws[w];
+        if (ws.kind == WK_IDLE || ws.state == ST_DONE) continue;
+        if (b->hzflag[w] & AKMC_ZONE_RES) ++res;
+        else ++other;
+    }
+    return res == 0 ? 0 : other ? 1 : 2;
 }
 
 // the batch view of the search micro-steps: the plain one plus the pair
@@ -1117,7 +1186,9 @@ BatchDev step_dev(akmc_batch_t b)
             d.staged64 = b->sv[8];
         }
     }
-    if (zone_usable(b)) {
+    if (zone_usable(b) && (b->zone_on || b->r.on)) {
+        d.zone_off = b->zone_on ? 0 : 1;
+        if (!b->res_off) d.r = b->r;
         d.zfrozen = b->s.frozen;
         d.zflag = b->zflag;
         d.zmark = b->zmark;
@@ -1129,26 +1200,50 @@ BatchDev step_dev(akmc_batch_t b)
     return d;
 }
 
-// one micro-step; step j of a run chunk records the kernel-timer events
-void enqueue_micro_step(akmc_batch_t b, int j)
+// the kernels of one force evaluation of the chain, with the fixed parts of
+// the resident walkers it serves; j >= 0: the kernel timer's events of a
+// chunk's step j
+void enqueue_chain(akmc_batch_t b, const BatchDev &d, int res, int j)
 {
     // FP64 pair terms run when a walker may ask for them: verification or
     // the closing FP64 energy of a relax
-    int prec = batch_mode(b) | ((b->s.verify_nl > 0 || b->s.final64) ? 2 : 0);
-    const BatchDev d = step_dev(b);
-    if (b->ktimer && (prec & 1) && b->f->host.kind == 0) {
-        for (int ph = 0; ph < 2; ++ph) akmc_launch_phase(d, b->f->host, prec, 0, ph, b->stream);
+    const int prec = batch_mode(b) | ((b->s.verify_nl > 0 || b->s.final64) ? 2 : 0);
+    const FieldDev &hf = b->f->host;
+    for (int ph = 0; ph < 2; ++ph) akmc_launch_phase(d, hf, prec, 0, ph, b->stream);
+    if (res) akmc_launch_res_base(d, hf, b->stream);
+    if (j >= 0 && b->ktimer && (prec & 1) && hf.kind == 0) {
         (void)hipEventRecord(b->kev[0][j], b->stream);
-        akmc_launch_phase(d, b->f->host, 1, 0, 2, b->stream);
+        akmc_launch_phase(d, hf, 1, 0, 2, b->stream);
         (void)hipEventRecord(b->kev[1][j], b->stream);
-        if (prec & 2) akmc_launch_phase(d, b->f->host, 2 | 4, 0, 2, b->stream);  // FP64 part of a mixed step
-        akmc_launch_phase(d, b->f->host, prec, 0, 3, b->stream);
+        if (prec & 2) akmc_launch_phase(d, hf, 2 | 4, 0, 2, b->stream);  // FP64 part of a mixed step
     } else {
-        akmc_launch_forces_impl(d, b->f->host, prec, 0, b->stream);
+        akmc_launch_phase(d, hf, prec, 0, 2, b->stream);
     }
-    // walkers of tens of thousands of atoms: 1024-thread state machines
-    if (b->logic_wide) akmc_launch_search_logic_wide(d, b->s, b->stream);
-    else akmc_launch_search_logic(d, b->s, b->stream);
+    if (res < 2) akmc_launch_phase(d, hf, prec, 0, 3, b->stream);
+}
+
+// Micro-steps between two runs of the chain when every running walker is
+// resident.  The chain is ten kernels that then have nothing to do (about
+// 40 us); a search waits for it once, at the start of its FP64 verification.
+constexpr int kResidentSteps = 9;
+
+// the kernels of a chunk of micro-steps, res as resident_mode
+void enqueue_steps(akmc_batch_t b, int steps, int res)
+{
+    const BatchDev d = step_dev(b);
+    // zones off, or walkers that need the chain, take it on every step
+    const int runs = res == 2 && b->zone_on && !b->ktimer ? (steps + kResidentSteps - 1) / kResidentSteps : steps;
+    for (int j = 0, done = 0; j < runs; ++j) {
+        const int k = (steps - done) / (runs - j);
+        done += k;
+        enqueue_chain(b, d, res, j);
+        if (res) akmc_launch_search_resident(d, b->f->host, b->s, k, 1, b->stream);
+        // walkers of tens of thousands of atoms: 1024-thread state machines
+        if (res < 2) {
+            if (b->logic_wide) akmc_launch_search_logic_wide(d, b->s, b->stream);
+            else akmc_launch_search_logic(d, b->s, b->stream);
+        }
+    }
 }
 
 int fetch_states(akmc_batch_t b)
@@ -1214,6 +1309,10 @@ int start_walkers(akmc_batch_t b, const int *walkers, int kind, double dt0, doub
         it.walker = w;
         it.zflag = (m > 0 && m < b->hw[w].n) ? (AKMC_ZONE_ON | AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64 | AKMC_ZONE_RESET)
                                              : 0;
+        if (resident_walker(b, w)) {
+            TRY(ensure_resident(b));
+            it.zflag |= AKMC_ZONE_RES;
+        }
         it.active = batch_mode(b);
         it.pad = 0;
         it.ws = ws;
@@ -1224,7 +1323,8 @@ int start_walkers(akmc_batch_t b, const int *walkers, int kind, double dt0, doub
     HIPCHK(hipMemcpyAsync(b->st_dev, b->st_pin, k * sizeof(StartItem), hipMemcpyHostToDevice, b->stream));
     HIPCHK(hipEventRecord(b->st_ev, b->stream));
     b->st_pending = true;
-    akmc_launch_start_walkers(b->d, b->s, b->st_dev, k, b->zflag, b->hv_on ? b->harvested : nullptr, b->stream);
+    akmc_launch_start_walkers(b->d, b->s, b->st_dev, k, b->zflag, b->hv_on ? b->harvested : nullptr, b->r.on ? b->r.n : nullptr,
+                              b->stream);
     akmc_launch_probe_init(b->d, b->s, b->stream);
     HIPCHK(hipGetLastError());
     if (!b->inflight) HIPCHK(hipStreamSynchronize(b->stream));
@@ -1329,17 +1429,18 @@ int load_walkers(akmc_batch_t b, const int *walkers, const double *x0, const dou
 int copy_walkers_out(akmc_batch_t b, const double *src, int nw, const int *walkers, double *out);
 int copy_walkers_out3(akmc_batch_t b, const double *const src[3], int nw, const int *walkers, double *out);
 
-int capture_graph(akmc_batch_t b, int steps)
+int capture_graph(akmc_batch_t b, int steps, int res)
 {
     drop_graph(b);
     HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    for (int k = 0; k < steps; ++k) enqueue_micro_step(b, k);
+    enqueue_steps(b, steps, res);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(b->stream, &g);
     if (e != hipSuccess) return fail(AKMC_EHIP, "graph capture failed: %s", hipGetErrorString(e));
     b->graph = g;
     HIPCHK(hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0));
     b->graph_steps = steps;
+    b->graph_res = res;
     b->graph_args = b->s;
     b->graph_d = step_dev(b);
     b->graph_prec = batch_mode(b);
@@ -1824,15 +1925,16 @@ int launch_chunk(akmc_batch_t b, int steps, int running)
     }
     // HIP events recorded inside a replayed graph cannot be timed, so the
     // kernel timer launches the micro-steps one by one
+    const int res = resident_mode(b);
     if (b->use_graphs && !b->ktimer) {
         const BatchDev bd = step_dev(b);
-        if (!b->gexec || b->graph_steps != steps || b->graph_prec != batch_mode(b) ||
+        if (!b->gexec || b->graph_steps != steps || b->graph_res != res || b->graph_prec != batch_mode(b) ||
             std::memcmp(&b->graph_args, &b->s, sizeof(SearchDev)) != 0 ||
             std::memcmp(&b->graph_d, &bd, sizeof(BatchDev)) != 0)
-            TRY(capture_graph(b, steps));
+            TRY(capture_graph(b, steps, res));
         HIPCHK(hipGraphLaunch(b->gexec, b->stream));
     } else {
-        for (int j = 0; j < steps; ++j) enqueue_micro_step(b, j);
+        enqueue_steps(b, steps, res);
         HIPCHK(hipGetLastError());
     }
     if (b->hv_on) {
@@ -1899,6 +2001,16 @@ int akmc_batch_run_wait(akmc_batch_t b, int *steps_done, int *running)
     // walkers started behind the chunk have not run yet
     for (const auto &p : b->started_inflight) b->hws[p.first] = p.second;
     b->started_inflight.clear();
+    // a walker that does not fit the resident kernel takes every walker of
+    // the batch back to the chain
+    bool too_big = false;
+    for (int w = 0; w < b->W; ++w) too_big |= b->hws[w].too_big != 0;
+    if (too_big && !b->res_off) {
+        akmc_launch_leave_resident(step_dev(b), b->stream);
+        HIPCHK(hipGetLastError());
+        b->res_off = true;
+        for (int &f : b->hzflag) f &= ~AKMC_ZONE_RES;
+    }
     for (int w = 0; w < b->W; ++w) run += b->hws[w].kind != WK_IDLE && b->hws[w].state != ST_DONE;
     if (steps_done) *steps_done = k;
     if (running) *running = run;
@@ -2275,11 +2387,17 @@ static int time_search_phases_prec(akmc_batch_t b, int prec, int nrep, double ms
     for (auto &e : b->evp)
         if (!e) HIPCHK(hipEventCreate(&e));
     const BatchDev d = step_dev(b);
+    const int res = resident_mode(b);
     for (int ph = 0; ph < 4; ++ph) ms[ph] = 0.0;
     for (int r = 0; r < nrep; ++r) {
         HIPCHK(hipEventRecord(b->evp[0], b->stream));
         for (int ph = 0; ph < 4; ++ph) {
             akmc_launch_phase(d, b->f->host, prec, 0, ph, b->stream);
+            // resident walkers: their whole evaluation is timed with pass 1
+            if (ph == 1 && res) {
+                akmc_launch_res_base(d, b->f->host, b->stream);
+                akmc_launch_search_resident(d, b->f->host, b->s, 1, 0, b->stream);
+            }
             HIPCHK(hipEventRecord(b->evp[ph + 1], b->stream));
         }
         HIPCHK(hipEventSynchronize(b->evp[4]));

@@ -9,6 +9,7 @@
 // are FP64; pair physics is T (float on the fast path, double for FP64
 // verification); per-atom force/energy sums are FP64.
 #include "akmc_internal.h"
+#include "sc_pair.h"
 
 #include <math.h>
 
@@ -56,147 +57,19 @@ __device__ inline double *energy_b(const BatchDev &b)
 template <typename T>
 __device__ inline bool zoned(const BatchDev &b, int w)
 {
-    if (!b.zflag) return false;
+    if (!b.zflag || b.zone_off) return false;
     const int f = b.zflag[w];
+    if (f & AKMC_ZONE_RES) return false;  // the chain evaluates all atoms of a resident walker
     return (f & AKMC_ZONE_ON) && !(f & (sizeof(T) == 8 ? AKMC_ZONE_FULL64 : AKMC_ZONE_FULL32));
 }
 
-template <typename T>
-__device__ inline const SCCoef<T> &sc_coef(const SCPairDev &p);
-template <>
-__device__ inline const SCCoef<float> &sc_coef<float>(const SCPairDev &p) { return p.f; }
-template <>
-__device__ inline const SCCoef<double> &sc_coef<double>(const SCPairDev &p) { return p.d; }
-
-// 1/x: the hardware reciprocal (1 ulp) on the FP32 path, an exact division
-// on the FP64 verification path
-template <typename T>
-__device__ inline T recip(T x) { return T(1) / x; }
-template <>
-__device__ inline float recip<float>(float x) { return __builtin_amdgcn_rcpf(x); }
-
-// u^x for non-integer exponents: libm pow on the FP64 path; on the FP32
-// path the integer part of x by squaring and the fraction by libm log2f /
-// exp2f (relative-accurate near u = 1, where (a/r)^2 lives), which keeps
-// the error of u^x at a few ulp without the cost of a full powf
-__device__ inline double pow_general(double u, double x) { return pow(u, x); }
-__device__ inline float pow_general(float u, float x)
+// a resident search walker that asks the chain for nothing on this step: no
+// evaluation of all its atoms is pending in its precision
+__device__ inline bool resident_idle(const BatchDev &b, int w)
 {
-    if (!(x >= 0.0f && x < 64.0f)) return exp2f(x * log2f(u));  // outside the split's range
-    const float xi = floorf(x);
-    float r = 1.0f, base = u;
-    for (int p = int(xi); p > 0; p >>= 1) {
-        if (p & 1) r *= base;
-        base *= base;
-    }
-    return r * exp2f((x - xi) * log2f(u));
-}
-
-// u2^(k/2) for an integer k >= 0 by repeated squaring; with k uniform across
-// the wavefront the loop is scalar control flow around the multiplications
-template <typename T>
-__device__ inline T pow_int(T u2, int k)
-{
-    T r = T(1), base = u2;
-    int p = k >> 1;
-    while (p) {
-        if (p & 1) r *= base;
-        base *= base;
-        p >>= 1;
-    }
-    if (k & 1) r *= sqrt(u2);
-    return r;
-}
-
-// square root for the integer powers: the hardware instruction (1 ulp) on
-// the FP32 path, whose arguments (a/r)^2 are normal numbers far from the
-// denormal range the correctly rounded expansion guards; libm on FP64
-__device__ inline double root(double x) { return sqrt(x); }
-__device__ inline float root(float x) { return __builtin_amdgcn_sqrtf(x); }
-
-// 1/sqrt(x) in FP64 for normal x > 0: the hardware estimate refined by two
-// Newton steps y += y (1 - x y^2) / 2 (quadratic convergence), a few ulp
-// from the correctly rounded value at a third of the cost of a division and
-// a square root
-__device__ inline double rsqrt_fp64(double x)
-{
-    double y = __builtin_amdgcn_rsq(x);
-    double r = fma(-(x * y), y, 1.0);
-    y = fma(0.5 * y, r, y);
-    r = fma(-(x * y), y, 1.0);
-    return fma(0.5 * y, r, y);
-}
-
-// The single-species power inputs of U pairs: ir2 = 1/r^2, u2 = (a/r)^2 and,
-// in FP64, rt = a/r.  FP32: hardware reciprocal (the power takes sqrt(u2)
-// from the hardware square root for odd exponents).  FP64: one refined 1/r,
-// so that neither a division nor a square root is needed.
-template <typename T, int U>
-__device__ inline void sc_powers_in(const double (&r2)[U], T a, T (&ir2)[U], T (&u2)[U], T (&rt)[U])
-{
-    if constexpr (sizeof(T) == 8) {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const double ir = rsqrt_fp64(r2[u]);
-            ir2[u] = ir * ir;
-            u2[u] = a * a * ir2[u];
-            rt[u] = a * ir;
-        }
-    } else {
-#pragma unroll
-        for (int u = 0; u < U; ++u) {
-            ir2[u] = recip<T>(T(r2[u]));
-            u2[u] = a * a * ir2[u];
-            rt[u] = T(0);  // the FP32 power takes its root from u2 itself
-        }
-    }
-}
-
-// (a/r)^9 and (a/r)^6 of the single-pair kernels from u2 = (a/r)^2, with
-// the compile-time exponents of the Sutton-Chen pairs they serve: the
-// products of the repeated squaring, u8 sqrt(u2) and u2 u4, without its
-// loop
-template <typename T, int U>
-__device__ inline void pow_9_6(const T (&u2)[U], const T (&rt)[U], T (&u9)[U], T (&u6)[U])
-{
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-        const T u4 = u2[u] * u2[u];
-        const T u8 = u4 * u4;
-        u9[u] = u8 * (sizeof(T) == 8 ? rt[u] : root(u2[u]));
-        u6[u] = u2[u] * u4;
-    }
-}
-template <typename T, int U>
-__device__ inline void pow_6(const T (&u2)[U], T (&u6)[U])
-{
-#pragma unroll
-    for (int u = 0; u < U; ++u) u6[u] = u2[u] * (u2[u] * u2[u]);
-}
-
-template <typename T>
-__device__ inline T pow_half(T u2, int k, T e)
-{
-    // u2^(e/2) with u2 = (a/r)^2; exact repeated squaring when e is an integer
-    if (k >= 0) {
-        T r = T(1), base = u2;
-        int p = k >> 1;
-        while (p) {
-            if (p & 1) r *= base;
-            base *= base;
-            p >>= 1;
-        }
-        if (k & 1) r *= sqrt(u2);
-        return r;
-    }
-    return pow_general(u2, e * T(0.5));
-}
-
-__device__ inline void min_image(double &dx, double &dy, double &dz, const WalkerDev &w)
-{
-    dx -= w.L[0] * rint(dx * w.invL[0]);
-    dy -= w.L[1] * rint(dy * w.invL[1]);
-    dz -= w.L[2] * rint(dz * w.invL[2]);
+    if (!b.r.on || b.zone_off) return false;
+    const int f = b.zflag[w];
+    return (f & AKMC_ZONE_RES) && !(f & (b.active[w] == 2 ? AKMC_ZONE_FULL64 : AKMC_ZONE_FULL32));
 }
 
 __device__ inline void entry_disp(uint32_t e, double &dx, double &dy, double &dz, const WalkerDev &w,
@@ -246,10 +119,11 @@ __global__ void __launch_bounds__(kPackBlock) k_pack_check_zoned(BatchDev b)
 {
     if (blockIdx.x == 0 && threadIdx.x == 0) *b.cell_work_n = 0;  // k_cell_bin queues this step's cells
     const int w = blockIdx.x;
-    if (skipped(b, w)) return;
+    if (skipped(b, w) || resident_idle(b, w)) return;
     const WalkerDev W = b.walkers[w];
     const int f = b.zflag[w];
-    const bool zoned = (f & (AKMC_ZONE_ON | AKMC_ZONE_RESET)) == AKMC_ZONE_ON;
+    const bool res = b.r.on && (f & AKMC_ZONE_RES);
+    const bool zoned = !b.zone_off && !res && (f & (AKMC_ZONE_ON | AKMC_ZONE_RESET)) == AKMC_ZONE_ON;
     const int n = zoned ? b.nz[w] : W.n;
     const double h2 = b.field->half_skin2;
     bool moved = false;
@@ -262,7 +136,8 @@ __global__ void __launch_bounds__(kPackBlock) k_pack_check_zoned(BatchDev b)
     }
     // a walker's fresh zone is marked by its list build (its start already
     // asks for one)
-    if (moved || (f & AKMC_ZONE_RESET)) b.rebuild[w] = 1;
+    // (a resident walker's lists are those of its last full evaluation)
+    if (moved || (f & AKMC_ZONE_RESET) || (res && !b.zone_off)) b.rebuild[w] = 1;
 }
 
 // record the positions the lists are built from (positions are never
@@ -345,7 +220,7 @@ __global__ void __launch_bounds__(kBinBlock) k_cell_bin(BatchDev b)
     const int tid = threadIdx.x;
     for (int c = tid; c < nc; c += kBinBlock) fill[c] = 0;
     // a restarted walker's zone starts empty (the list build marks it)
-    if (b.zflag && (b.zflag[w] & AKMC_ZONE_RESET))
+    if (b.zflag && (b.zflag[w] & (AKMC_ZONE_RESET | AKMC_ZONE_RES)) == AKMC_ZONE_RESET)
         for (int l = tid; l < W.n; l += kBinBlock) b.zmark[W.off + l] = 0;
     __syncthreads();
     const bool keep = W.n <= kBinAtoms;
@@ -582,7 +457,8 @@ __device__ void nbr_build_item(const BatchDev &b, int cg, int chunk, double *sx,
     static_assert(kNbLanes == 16, "the hit ballot is split in 16-bit fields");
     // a free atom of a zoned walker puts itself and every atom of its list
     // within rc + skin/2 in the walker's zone
-    const bool mark = have && b.zflag && (b.zflag[w] & AKMC_ZONE_ON) && b.zfrozen[i] == 0;
+    const bool mark = have && b.zflag && (b.zflag[w] & (AKMC_ZONE_ON | AKMC_ZONE_RES)) == AKMC_ZONE_ON &&
+                      b.zfrozen[i] == 0;
     if (mark && lane == 0) b.zmark[i] = 1;
     int cnt = 0, nnear = 0;
     int ms = 0;  // candidates staged in LDS
@@ -826,8 +702,9 @@ __global__ void __launch_bounds__(kBlock) k_zone_build(BatchDev b, unsigned long
     if (!b.rebuild[w]) return;
     const int f = b.zflag[w];
     // the walker's rebuild is done (k_rebuild_done's bookkeeping)
-    if (!(f & AKMC_ZONE_ON)) {
+    if (!(f & AKMC_ZONE_ON) || (f & AKMC_ZONE_RES)) {
         if (threadIdx.x == 0) {
+            b.zflag[w] = f & ~AKMC_ZONE_RESET;
             b.rebuild[w] = 0;
             atomicAdd(count, 1ull);
         }
@@ -888,11 +765,12 @@ __global__ void __launch_bounds__(1024) k_work_list(BatchDev b, int4 apc)
             for (int w0 = 0; w0 < b.W; w0 += 1024) {
                 const int w = w0 + tid;
                 int k = 0;
-                if (w < b.W && b.active[w] == mode) {
+                if (w < b.W && b.active[w] == mode && !resident_idle(b, w)) {
                     int len = b.walkers[w].n;
-                    if (b.zflag) {
+                    if (b.zflag && !b.zone_off) {
                         const int f = b.zflag[w];
-                        if ((f & AKMC_ZONE_ON) && !(f & full)) len = pass == 1 ? b.nz[w] : b.znact[w];
+                        if ((f & (AKMC_ZONE_ON | AKMC_ZONE_RES)) == AKMC_ZONE_ON && !(f & full))
+                            len = pass == 1 ? b.nz[w] : b.znact[w];
                     }
                     k = (len + a - 1) / a;
                 }
@@ -936,28 +814,6 @@ __device__ inline int xcd_thread(int nblocks)
     const int logical = (blockIdx.x % kXCD) * per + blockIdx.x / kXCD;
     return logical < nblocks ? logical * blockDim.x + threadIdx.x : -1;
 }
-
-// sum over the LPA consecutive lanes that share one atom
-template <int LPA>
-__device__ inline double lane_group_sum(double v)
-{
-    for (int o = LPA / 2; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
-// The Sutton-Chen pair table (nspec^2 entries) staged in LDS by every
-// workgroup before any thread leaves, so the coefficient lookup of a pair is
-// an LDS read instead of a third dependent global load.
-__device__ inline void stage_sc_table(const FieldDev &F, SCPairDev *tab)
-{
-    static_assert(sizeof(SCPairDev) % 4 == 0, "table staged in 4-byte words");
-    const int nw = F.nspec * F.nspec * int(sizeof(SCPairDev) / 4);
-    const uint32_t *src = reinterpret_cast<const uint32_t *>(F.sc);
-    uint32_t *dst = reinterpret_cast<uint32_t *>(tab);
-    for (int w = threadIdx.x; w < nw; w += blockDim.x) dst[w] = src[w];
-    __syncthreads();
-}
-
 
 // The neighbour loops below hold U list entries, fetch the next U entries
 // while gathering the current U neighbours' positions (and densities), then
@@ -2013,7 +1869,7 @@ __global__ void __launch_bounds__(kReduceBlock) k_walker_reduce_many(BatchDev b)
 {
     __shared__ double sh[kReduceBlock];
     const int w = blockIdx.x;
-    if (skipped(b, w)) return;
+    if (skipped(b, w) || (b.r.on && (b.zflag[w] & AKMC_ZONE_RES))) return;
     const WalkerDev W = b.walkers[w];
     const bool e64 = b.active[w] == 2 && b.e_a64;
     const double *ea = e64 ? b.e_a64 : b.e_a, *eb = e64 ? b.e_b64 : b.e_b;
@@ -2152,6 +2008,14 @@ static void launch_lists(const BatchDev &b, const FieldDev &hf, hipStream_t s)
 static bool sc_one(const FieldDev &hf)
 {
     return hf.nspec == 1 && hf.sc[0].on && hf.sc[0].n_int == 9 && hf.sc[0].m_int == 6;
+}
+
+int akmc_sc_kind(const FieldDev &hf)
+{
+    if (sc_one(hf)) return 1;
+    for (int k = 0; k < hf.nspec * hf.nspec; ++k)
+        if (!hf.sc[k].on || hf.sc[k].n_int != 9 || hf.sc[k].m_int != 6) return 0;
+    return 2;
 }
 
 // grid, workgroup size and dynamic LDS of a Sutton-Chen pair launch
