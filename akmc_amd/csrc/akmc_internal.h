@@ -139,6 +139,7 @@ struct ResidentDev {
     uint16_t *slot;            // [W][RES_SLOTS] slot -> local atom, ascending
     unsigned long long *mask;  // [W][RES_SLOTS][4] free atoms in reach of a frozen
                                // slot: free atom f is bit f / 4 of word f % 4
+    uint16_t *task;            // [W][RES_SLOTS] frozen slots in the order they are served
     uint16_t *fslot;           // [W][RES_FREE] free atom -> slot
     uint16_t *flist;           // [W][RES_FREE][fcap] neighbours (slots) of a free atom
     int *fcnt;                 // [W][RES_FREE]
@@ -362,9 +363,15 @@ struct SearchDev {
 // density and pair energy of every atom of the resident walkers it serves
 void akmc_launch_res_base(const BatchDev &b, const FieldDev &hf, hipStream_t st);
 // up to nsteps micro-steps of every resident walker (evaluation and state
-// machine); logic 0: one evaluation each, nothing else
-void akmc_launch_search_resident(const BatchDev &b, const FieldDev &hf, const SearchDev &s, int nsteps, int logic,
-                                 hipStream_t st);
+// machine), those waiting for the chain's full evaluation among them when
+// service is set; logic 0: one evaluation each, nothing else
+// (args: a device copy of the batch's and searches' descriptors)
+struct ResArgs {
+    BatchDev b;
+    SearchDev s;
+};
+void akmc_launch_search_resident(int nwalkers, const FieldDev &hf, const ResArgs *args, int nsteps, int logic,
+                                 int service, hipStream_t st);
 // every resident walker goes over to the chain (fresh zone, full evaluations)
 void akmc_launch_leave_resident(const BatchDev &b, hipStream_t st);
 // 0 general pair table, 1 one species pair with n = 9, m = 6, 2 every

@@ -163,6 +163,8 @@ struct akmc_batch_s {
     // whose running walkers are all resident
     ResidentDev r{};
     bool res_off = false;
+    ResArgs *res_args = nullptr;      // device copy of the descriptors its kernel
+    ResArgs res_host{};               // reads, and what it holds
     int nmax = 0;
     int graph_res = 0;
     // kernel variants of the search micro-steps' Sutton-Chen passes:
@@ -1100,7 +1102,7 @@ bool zone_usable(akmc_batch_t b)
 // bytes of a resident walker's lists
 size_t resident_bytes(akmc_batch_t b)
 {
-    return AKMC_RES_SLOTS * 34 + AKMC_RES_FREE * (30 + 2 * (size_t)b->d.maxnb) + 64;
+    return AKMC_RES_SLOTS * 36 + AKMC_RES_FREE * (30 + 2 * (size_t)b->d.maxnb) + 64;
 }
 
 // searches may run in the resident kernel: zones apply, and the walkers,
@@ -1128,6 +1130,7 @@ int ensure_resident(akmc_batch_t b)
     TRY(dalloc(b, &r.n, W));
     TRY(dalloc(b, &r.slot, W * AKMC_RES_SLOTS));
     TRY(dalloc(b, &r.mask, W * AKMC_RES_SLOTS * 4));
+    TRY(dalloc(b, &r.task, W * AKMC_RES_SLOTS));
     TRY(dalloc(b, &r.fslot, W * AKMC_RES_FREE));
     TRY(dalloc(b, &r.flist, W * AKMC_RES_FREE * r.fcap));
     TRY(dalloc(b, &r.fcnt, W * AKMC_RES_FREE));
@@ -1138,8 +1141,26 @@ int ensure_resident(akmc_batch_t b)
         TRY(dalloc(b, &r.base_rho[p], A));
         TRY(dalloc(b, &r.base_ep[p], A));
     }
+    TRY(dalloc(b, &b->res_args, 1));
     r.on = 1;
     b->r = r;
+    return AKMC_SUCCESS;
+}
+
+BatchDev step_dev(akmc_batch_t b);
+
+// brings the resident kernel's descriptors up to date (in stream order: a
+// chunk in flight keeps the ones it was launched with)
+int sync_res_args(akmc_batch_t b)
+{
+    if (!b->r.on) return AKMC_SUCCESS;
+    ResArgs a;
+    std::memset((void *)&a, 0, sizeof a);
+    a.b = step_dev(b);
+    a.s = b->s;
+    if (std::memcmp(&a, &b->res_host, sizeof a) == 0) return AKMC_SUCCESS;
+    b->res_host = a;
+    HIPCHK(hipMemcpyAsync((void *)b->res_args, &b->res_host, sizeof a, hipMemcpyHostToDevice, b->stream));
     return AKMC_SUCCESS;
 }
 
@@ -1231,18 +1252,23 @@ constexpr int kResidentSteps = 9;
 void enqueue_steps(akmc_batch_t b, int steps, int res)
 {
     const BatchDev d = step_dev(b);
-    // zones off, or walkers that need the chain, take it on every step
-    const int runs = res == 2 && b->zone_on && !b->ktimer ? (steps + kResidentSteps - 1) / kResidentSteps : steps;
+    // walkers that need the chain take it on every step; with zones off the
+    // chain evaluates every atom on every step, and a search still waits as
+    // it does with zones on
+    const int runs = res == 2 && !b->ktimer ? (steps + kResidentSteps - 1) / kResidentSteps : steps;
     for (int j = 0, done = 0; j < runs; ++j) {
-        const int k = (steps - done) / (runs - j);
-        done += k;
-        enqueue_chain(b, d, res, j);
-        if (res) akmc_launch_search_resident(d, b->f->host, b->s, k, 1, b->stream);
-        // walkers of tens of thousands of atoms: 1024-thread state machines
-        if (res < 2) {
-            if (b->logic_wide) akmc_launch_search_logic_wide(d, b->s, b->stream);
-            else akmc_launch_search_logic(d, b->s, b->stream);
+        const int k = (steps - done) / (runs - j), launches = b->zone_on ? 1 : k;
+        for (int l = 0; l < launches; ++l) {
+            enqueue_chain(b, d, res, done + l);
+            if (res)
+                akmc_launch_search_resident(b->W, b->f->host, b->res_args, k / launches, 1, l == 0, b->stream);
+            // walkers of tens of thousands of atoms: 1024-thread state machines
+            if (res < 2) {
+                if (b->logic_wide) akmc_launch_search_logic_wide(d, b->s, b->stream);
+                else akmc_launch_search_logic(d, b->s, b->stream);
+            }
         }
+        done += k;
     }
 }
 
@@ -1926,6 +1952,7 @@ int launch_chunk(akmc_batch_t b, int steps, int running)
     // HIP events recorded inside a replayed graph cannot be timed, so the
     // kernel timer launches the micro-steps one by one
     const int res = resident_mode(b);
+    TRY(sync_res_args(b));
     if (b->use_graphs && !b->ktimer) {
         const BatchDev bd = step_dev(b);
         if (!b->gexec || b->graph_steps != steps || b->graph_res != res || b->graph_prec != batch_mode(b) ||
@@ -2388,6 +2415,7 @@ static int time_search_phases_prec(akmc_batch_t b, int prec, int nrep, double ms
         if (!e) HIPCHK(hipEventCreate(&e));
     const BatchDev d = step_dev(b);
     const int res = resident_mode(b);
+    TRY(sync_res_args(b));
     for (int ph = 0; ph < 4; ++ph) ms[ph] = 0.0;
     for (int r = 0; r < nrep; ++r) {
         HIPCHK(hipEventRecord(b->evp[0], b->stream));
@@ -2396,7 +2424,7 @@ static int time_search_phases_prec(akmc_batch_t b, int prec, int nrep, double ms
             // resident walkers: their whole evaluation is timed with pass 1
             if (ph == 1 && res) {
                 akmc_launch_res_base(d, b->f->host, b->stream);
-                akmc_launch_search_resident(d, b->f->host, b->s, 1, 0, b->stream);
+                akmc_launch_search_resident(b->W, b->f->host, b->res_args, 1, 0, 1, b->stream);
             }
             HIPCHK(hipEventRecord(b->evp[ph + 1], b->stream));
         }

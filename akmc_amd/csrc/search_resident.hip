@@ -14,12 +14,14 @@
 // for the zone's whole lists.  The energy is the sum over the zone's atoms
 // plus that of the atoms outside it, which changes only with the zone.
 //
-// What bounds it: one walker's chain of dependent phases (lists, masks,
-// reductions), with at most two workgroups of four wavefronts per CU to
-// hide it.  512 walkers of 500-4000 atoms: 91 us per micro-step for
-// evaluations and state machines, where the chain's kernels took 293 us; 12
-// walkers: 60 us against 104 us; 128 alloy cells of 3600 atoms, searches
-// with verification and basin 2: 86 us against 286 us.
+// What bounds it: one walker's chain of dependent phases (gathers, pair
+// terms, sums, the state machine's reductions; one walker alone runs at 60%
+// of the rate of two on a CU), so a workgroup has eight wavefronts, two fit
+// a CU, the functions are out of line for 128 registers each, lists and
+// records are in LDS, and sums go by DPP moves.  512 walkers of 500-4000
+// atoms: 63 us per micro-step for evaluations and state machines, where the
+// chain's kernels took 293 us (91 us with four wavefronts and lists in
+// global memory); 12 walkers: 41 us against 104 us.
 //
 // Results do not depend on the batch or on when the lists were built.  The
 // FP32 terms summed here span fewer than 2^29 in magnitude and count, so
@@ -27,18 +29,22 @@
 // twice the working precision.  With zones off the chain evaluates every
 // atom on every step and the same kernel follows, so both modes agree bit
 // for bit.
+#define AKMC_LOGIC_BLOCK 512
 #include "search_logic.h"
 #include "sc_pair.h"
 
 namespace {
 
 constexpr int kFree = AKMC_RES_FREE, kSlots = AKMC_RES_SLOTS, kCand = AKMC_RES_CAND;
-constexpr int kBitWords = 7168;  // hit words of a list build: free atoms x candidate wavefronts
+constexpr int kBitWords = 6784;  // hit words of a list build: free atoms x candidate wavefronts
 constexpr int kFreeLanes = 16;   // lanes per free atom's list
-constexpr int kFreeIlp = 4;      // list entries in flight per lane
+constexpr int kFreeIlp = 5;      // list entries in flight per lane: two batches for a bulk list of 155
 constexpr int kFzLanes = 4;      // lanes (mask words) per frozen slot
+constexpr int kFzIlp = 2;        // free atoms of a mask word in flight per lane
+constexpr int kClass = 8;        // frozen slots are served in classes of similar reach
 constexpr int kResSpec = 4;      // species of a resident walker's field
-static_assert(kCand * sizeof(uint16_t) + kBitWords * 8 == kLzLds * sizeof(double), "the build fits the pool");
+static_assert(kCand * sizeof(uint16_t) + kBitWords * 8 + 3 * kFree * sizeof(float) == kLzLds * sizeof(double),
+              "the build fits the pool");
 static_assert(4 * kSlots == kLzLds, "four doubles of the pool per slot");
 
 // a resident workgroup's LDS
@@ -46,13 +52,68 @@ template <int KIND>
 struct ResLds {
     double pool[kLzLds];                 // records of the zone, build scratch, Lanczos vectors
     double fx[kFree], fy[kFree], fz[kFree];  // free atoms
+    int fofs[kFree + 1];                 // start of each free atom's list among all of them
     uint16_t fid[kFree], fslot[kFree];   // their local indices and slots
-    uint8_t zt[kSlots];                  // per slot: species, bit 7: free
+    uint8_t zt[kSlots];                  // per slot: species
     SCPairDev tab[KIND == 1 ? 1 : kResSpec * kResSpec];  // pair table (general and table kinds)
     double sh[4 * kWaves];
     int wsum[2 * kWaves];
     WalkerState ws;
 };
+
+// the workgroup's LDS; one variable, so that the functions below, kept out
+// of line for their own register allocations, address it directly
+template <int KIND>
+__device__ __forceinline__ ResLds<KIND> &res_lds()
+{
+    __shared__ ResLds<KIND> L;
+    return L;
+}
+
+// an object every thread of the wavefront reads at one address, through
+// scalar loads (it does not change while the kernel runs)
+template <typename T>
+__device__ __forceinline__ T load_uniform(const T *p)
+{
+    const unsigned long long v = reinterpret_cast<unsigned long long>(p);
+    const unsigned lo = __builtin_amdgcn_readfirstlane(unsigned(v)), hi = __builtin_amdgcn_readfirstlane(unsigned(v >> 32));
+    typedef const __attribute__((address_space(4))) T CT;
+    T out;
+    __builtin_memcpy(&out, (CT *)((unsigned long long)hi << 32 | lo), sizeof(T));
+    return out;
+}
+
+// v of the lane that CTRL (a DPP row operation) pairs this one with
+template <int CTRL>
+__device__ __forceinline__ double dpp_of(double v)
+{
+    const long long w = __double_as_longlong(v);
+    const int lo = __builtin_amdgcn_update_dpp(0, int(w), CTRL, 0xF, 0xF, true);
+    const int hi = __builtin_amdgcn_update_dpp(0, int(w >> 32), CTRL, 0xF, 0xF, true);
+    return __longlong_as_double((long long)(unsigned)lo | (long long)hi << 32);
+}
+
+// sum over the LPA (4 or 16) consecutive lanes of a group, the same bits on
+// all of them: neighbours, pairs (quad permutes), quads and halves of a row
+// (mirrors); register moves instead of the LDS shuffles of lane_group_sum
+template <int LPA>
+__device__ __forceinline__ double row_sum(double v)
+{
+    static_assert(LPA == 4 || LPA == 16, "quads or rows");
+    v += dpp_of<0xB1>(v);  // quad_perm [1,0,3,2]
+    v += dpp_of<0x4E>(v);  // quad_perm [2,3,0,1]
+    if constexpr (LPA == 16) {
+        v += dpp_of<0x141>(v);  // row_half_mirror
+        v += dpp_of<0x140>(v);  // row_mirror
+    }
+    return v;
+}
+
+// During evaluations the pool holds x, y, z and 1/sqrt(rho) per zone slot,
+// S doubles each, then the free atoms' lists when they fit (75 free atoms:
+// 28 KB and 24 KB of the 64 KB)
+__device__ inline int slot_stride(int nz) { return (nz + 15) & ~15; }
+__device__ inline bool lists_fit(int entries, int S) { return entries <= 4 * (kLzLds - 4 * S); }
 
 // sqrt(x) to within half a unit in the last place or so: the hardware
 // estimate and one Newton step (the general kernels' table pairs take the
@@ -140,13 +201,6 @@ __device__ inline void add_density(const WalkerDev &W, double rc2, const SCCoef<
     }
 }
 
-// 1/sqrt(rho) for the force pass (-1: no density)
-template <typename T>
-__device__ inline T inv_root(double rho)
-{
-    return rho < 1.0e-8 ? T(-1) : T(1.0 / sqrt(rho));
-}
-
 // exclusive prefix over the workgroup of a flag, in thread order; total gets
 // the sum.  slot alternates between two scratch rows, so one barrier does.
 __device__ inline int flag_prefix(bool v, int *wsum, int row, int &total)
@@ -172,13 +226,17 @@ __device__ inline int flag_prefix(bool v, int *wsum, int row, int &total)
 // ones within rc + skin), all in ascending index order.  Candidates are the
 // atoms within rc + skin of the free atoms' box.  false: past a capacity.
 template <int KIND>
-__device__ __forceinline__ bool res_build(const BatchDev &b, const SearchDev &s, const WalkerDev &W, ResLds<KIND> &L,
-                                          int nf)
+__device__ __attribute__((noinline)) bool res_build(const ResArgs *args, int nf)
 {
+    ResLds<KIND> &L = res_lds<KIND>();
+    const BatchDev b = load_uniform(&args->b);
+    const SearchDev s = load_uniform(&args->s);
+    const WalkerDev W = load_uniform(b.walkers + blockIdx.x);
     const int w = blockIdx.x, tid = threadIdx.x, lane = tid & 63, wave = tid >> 6;
     const ResidentDev &R = b.r;
     uint16_t *cand = reinterpret_cast<uint16_t *>(L.pool);
     unsigned long long *bits = reinterpret_cast<unsigned long long *>(L.pool + kCand / 4);
+    float *gx = reinterpret_cast<float *>(bits + kBitWords), *gy = gx + kFree, *gz = gy + kFree;  // from the box centre
     const double rl2 = b.field->rlist2, rz2 = b.field->rzone2;
     // the free atoms' box: an arc of the cell per axis around the first one
     double lo[3] = {0, 0, 0}, hi[3] = {0, 0, 0};
@@ -219,23 +277,42 @@ __device__ __forceinline__ bool res_build(const BatchDev &b, const SearchDev &s,
     __syncthreads();
     if (nc > kCand || nf * ncw > kBitWords) return false;
     // every candidate against every free atom: its mask (frozen candidates)
-    // and, by ballot, the free atoms' hit words over the candidates
+    // and, by ballot, the free atoms' hit words over the candidates.  FP32
+    // distances with a margin above their rounding (coordinates of up to L/2,
+    // 2^-24 of that each, so 2 r sqrt(3) L 2^-24 = 2e-7 r L on a square): an
+    // entry past its radius adds nothing, the evaluation tests every pair in
+    // FP64
+    for (int f = tid; f < nf; f += kBlock) {
+        double dx = L.fx[f] - bc[0], dy = L.fy[f] - bc[1], dz = L.fz[f] - bc[2];
+        min_image(dx, dy, dz, W);
+        gx[f] = float(dx);
+        gy[f] = float(dy);
+        gz[f] = float(dz);
+    }
+    __syncthreads();
+    const float L0 = float(W.L[0]), L1 = float(W.L[1]), L2 = float(W.L[2]);
+    const float i0 = float(W.invL[0]), i1 = float(W.invL[1]), i2 = float(W.invL[2]);
+    const float margin = 1.0e-6f * float(sqrt(rl2)) * fmaxf(fmaxf(L0, L1), fmaxf(L2, 16.0f));
     int nz = 0, nfree = 0;
     for (int c0 = 0; c0 < nc; c0 += kBlock) {
         const int c = c0 + tid;
         const bool has = c < nc;
         const int j = has ? cand[c] : 0, i = W.off + j;
-        const double x = b.x[i], y = b.y[i], z = b.z[i];
+        double xd = b.x[i] - bc[0], yd = b.y[i] - bc[1], zd = b.z[i] - bc[2];
+        min_image(xd, yd, zd, W);
+        const float x = float(xd), y = float(yd), z = float(zd);
         const bool fr = s.frozen[i] != 0;
-        const double lim = fr ? rz2 : rl2;
+        const float lim = float(fr ? rz2 : rl2) + margin;
         unsigned long long m[kFzLanes] = {};
         const int word = (c0 >> 6) + wave;
         for (int f0 = 0; f0 < nf; f0 += kFzLanes) {
 #pragma unroll
             for (int q = 0; q < kFzLanes; ++q) {
                 const int f = f0 + q < nf ? f0 + q : 0;
-                double dx = x - L.fx[f], dy = y - L.fy[f], dz = z - L.fz[f];
-                min_image(dx, dy, dz, W);
+                float dx = x - gx[f], dy = y - gy[f], dz = z - gz[f];
+                dx -= L0 * rintf(dx * i0);
+                dy -= L1 * rintf(dy * i1);
+                dz -= L2 * rintf(dz * i2);
                 const bool hit = has && f0 + q < nf && dx * dx + dy * dy + dz * dz <= lim && L.fid[f] != j;
                 const unsigned long long bal = __ballot(hit);
                 if (lane == 0 && word < ncw && f0 + q < nf) bits[f * ncw + word] = bal;
@@ -276,6 +353,41 @@ __device__ __forceinline__ bool res_build(const BatchDev &b, const SearchDev &s,
             if (at > R.fcap) atomicOr(b.overflow, AKMC_OV_LIST);
         }
     }
+    // the order frozen slots are served in: classes of the number of free
+    // atoms in reach, ascending slots within a class, so that the lanes of a
+    // wavefront loop about equally long
+    {
+        unsigned long long *mask = R.mask + (size_t)w * kSlots * kFzLanes;
+        constexpr int kRounds = kSlots / kBlock;
+        int *cnt = reinterpret_cast<int *>(L.pool);  // [kRounds][kWaves][kClass], the candidates are done
+        int cls[kRounds], rank[kRounds];
+        __syncthreads();
+#pragma unroll
+        for (int r = 0; r < kRounds; ++r) {
+            const int k = r * kBlock + tid;
+            int c = -1;
+            if (k < nz) {
+                int pc = 0;
+                for (int q = 0; q < kFzLanes; ++q) pc += __popcll(mask[(size_t)k * kFzLanes + q]);
+                c = pc == 0 ? -1 : min(kClass - 1, pc / 6);  // no bits: a free slot
+            }
+            cls[r] = c;
+            for (int v = 0; v < kClass; ++v) {
+                const unsigned long long bal = __ballot(c == v);
+                if (lane == 0) cnt[(r * kWaves + wave) * kClass + v] = __popcll(bal);
+                if (c == v) rank[r] = __popcll(bal & ((1ull << lane) - 1ull));
+            }
+        }
+        __syncthreads();
+        for (int r = 0; r < kRounds; ++r) {
+            if (cls[r] < 0) continue;
+            int at = rank[r];
+            for (int g = 0; g < kRounds * kWaves; ++g)
+                for (int v = 0; v < kClass; ++v)
+                    if (v < cls[r] || (v == cls[r] && g < r * kWaves + wave)) at += cnt[g * kClass + v];
+            R.task[(size_t)w * kSlots + at] = uint16_t(r * kBlock + tid);
+        }
+    }
     for (int f = tid; f < nf; f += kBlock) {
         R.ref[((size_t)w * 3 + 0) * kFree + f] = L.fx[f];
         R.ref[((size_t)w * 3 + 1) * kFree + f] = L.fy[f];
@@ -283,7 +395,6 @@ __device__ __forceinline__ bool res_build(const BatchDev &b, const SearchDev &s,
     }
     if (tid == 0) {
         R.n[w] = nz;
-        R.eok[w] = 0;
         b.nz[w] = nz;
         atomicAdd(b.rebuild_count, 1ull);
     }
@@ -291,11 +402,35 @@ __device__ __forceinline__ bool res_build(const BatchDev &b, const SearchDev &s,
     return true;
 }
 
+// starts of the free atoms' lists from their lengths (one wavefront)
+template <int KIND>
+__device__ inline void res_offsets(const int *fcnt, int nf)
+{
+    ResLds<KIND> &L = res_lds<KIND>();
+    if (threadIdx.x >= 64) return;
+    const int lane = threadIdx.x;
+    int before = 0;
+    for (int f0 = 0; f0 < nf; f0 += 64) {
+        const int v = f0 + lane < nf ? fcnt[f0 + lane] : 0;
+        int x = v;
+        for (int o = 1; o < 64; o <<= 1) {
+            const int t = __shfl_up(x, o);
+            if (lane >= o) x += t;
+        }
+        if (f0 + lane < nf) L.fofs[f0 + lane] = before + x - v;
+        before += __shfl(x, 63);
+    }
+    if (lane == 0) L.fofs[nf] = before;
+}
+
 // energies of the atoms outside the zone (fixed parts only: no free atom is
 // in their reach), in index order per thread
 template <int KIND>
-__device__ __forceinline__ void res_outside(const BatchDev &b, const WalkerDev &W, ResLds<KIND> &L, int nz, int prec)
+__device__ __attribute__((noinline)) void res_outside(const ResArgs *args, int nz, int prec)
 {
+    ResLds<KIND> &L = res_lds<KIND>();
+    const BatchDev b = load_uniform(&args->b);
+    const WalkerDev W = load_uniform(b.walkers + blockIdx.x);
     const int w = blockIdx.x, tid = threadIdx.x;
     uint32_t *in = reinterpret_cast<uint32_t *>(L.pool);
     for (int k = tid; k < (AKMC_RES_ATOMS + 32) / 32; k += kBlock) in[k] = 0u;
@@ -316,7 +451,6 @@ __device__ __forceinline__ void res_outside(const BatchDev &b, const WalkerDev &
         double *e = b.r.eout + ((size_t)w * 2 + prec) * 2;
         e[0] = v[0];
         e[1] = v[1];
-        b.r.eok[w] |= 1 << prec;
     }
     __syncthreads();
 }
@@ -324,174 +458,169 @@ __device__ __forceinline__ void res_outside(const BatchDev &b, const WalkerDev &
 // one evaluation at the free positions in LDS: forces of the free atoms and
 // the walker's energy record
 template <typename T, int KIND>
-__device__ __forceinline__ void res_eval(const BatchDev &b, const WalkerDev &W, ResLds<KIND> &L, int nf, int nz)
+__device__ __attribute__((noinline)) void res_eval(const ResArgs *args, int nf, int nz)
 {
+    ResLds<KIND> &L = res_lds<KIND>();
+    const BatchDev b = load_uniform(&args->b);
+    const WalkerDev W = load_uniform(b.walkers + blockIdx.x);
     constexpr int prec = sizeof(T) == 8 ? 1 : 0;
     const int w = blockIdx.x, tid = threadIdx.x;
-    const FieldDev &F = *b.field;
-    const SCCoef<T> c1 = sc_coef<T>(F.sc[0]);
-    const double rc2 = F.rc2;
-    const int ns = F.nspec;
+    const SCCoef<T> c1 = sc_coef<T>(load_uniform(&b.field->sc[0]));
+    const double rc2 = load_uniform(&b.field->rc2);
+    const int ns = load_uniform(&b.field->nspec);
     const ResidentDev &R = b.r;
-    const double *rx = L.pool, *ry = rx + kSlots, *rz = ry + kSlots;
-    T *rw = reinterpret_cast<T *>(L.pool + 3 * kSlots);  // 1/sqrt(rho) per slot
+    const int S = slot_stride(nz);
+    const double *rx = L.pool, *ry = rx + S, *rz = ry + S;
+    double *rd = L.pool + 3 * S;       // density per slot, then 1/sqrt(rho)
+    T *rw = reinterpret_cast<T *>(rd);  // in the low half for FP32
+    constexpr int kRw = 8 / sizeof(T);
     double many = 0.0, pair = 0.0;
-    // frozen slots: four lanes each, one mask word per lane, two of its free
-    // atoms at a time; the next slot's loads go out before this one's pairs
+    // frozen slots: four lanes each, one mask word per lane, kFzIlp of its
+    // free atoms at a time; the next slot's loads go out before this one's
     const unsigned long long *mask = R.mask + (size_t)w * kSlots * kFzLanes;
-    const uint16_t *slot = R.slot + (size_t)w * kSlots;
+    const uint16_t *task = R.task + (size_t)w * kSlots, *slot = R.slot + (size_t)w * kSlots;
     {
-        int t = tid;
-        unsigned long long mn = t < kFzLanes * nz ? mask[t] : 0ull;
-        int jn = t < kFzLanes * nz ? slot[t / kFzLanes] : 0;
-        for (; t < kFzLanes * nz; t += kBlock) {
+        constexpr int kPer = kBlock / kFzLanes;
+        const int nt = nz - nf, q = tid % kFzLanes;
+        int t = tid / kFzLanes;
+        int sn = t < nt ? task[t] : 0, s2 = t + kPer < nt ? task[t + kPer] : 0;
+        unsigned long long mn = mask[sn * kFzLanes + q];
+        int in = W.off + slot[sn];
+        for (; t < nt; t += kPer) {
             unsigned long long m = mn;
-            const int i = W.off + jn, sl = t / kFzLanes, q = t % kFzLanes;
+            const int i = in, sl = sn;
             const double brho = R.base_rho[prec][i], bep = R.base_ep[prec][i];
-            if (t + kBlock < kFzLanes * nz) {
-                mn = mask[t + kBlock];
-                jn = slot[(t + kBlock) / kFzLanes];
-            }
-            const int zt = L.zt[sl];
-            if (zt & 128) continue;  // a free slot (all four lanes)
+            sn = s2;
+            mn = mask[sn * kFzLanes + q];
+            in = W.off + slot[sn];
+            s2 = t + 2 * kPer < nt ? task[t + 2 * kPer] : 0;
             const double xi = rx[sl], yi = ry[sl], zi = rz[sl];
             double rho = 0.0, ep = 0.0;
             while (m) {
-                double px[2], py[2], pz[2];
-                bool ok[2];
-                const SCPairDev *p[2];
+                double px[kFzIlp], py[kFzIlp], pz[kFzIlp];
+                bool ok[kFzIlp];
+                const SCPairDev *p[kFzIlp];
 #pragma unroll
-                for (int u = 0; u < 2; ++u) {
+                for (int u = 0; u < kFzIlp; ++u) {
                     ok[u] = m != 0ull;
                     const int f = ok[u] ? kFzLanes * (__ffsll((long long)m) - 1) + q : 0;
                     m &= m - 1ull;
                     px[u] = L.fx[f];
                     py[u] = L.fy[f];
                     pz[u] = L.fz[f];
-                    p[u] = KIND == 1 ? nullptr : L.tab + (zt & 127) * ns + (L.zt[L.fslot[f]] & 127);
+                    p[u] = KIND == 1 ? nullptr : L.tab + L.zt[sl] * ns + L.zt[L.fslot[f]];
                 }
-                add_density<T, KIND, 2>(W, rc2, c1, p, xi, yi, zi, px, py, pz, ok, rho, ep);
+                add_density<T, KIND, kFzIlp>(W, rc2, c1, p, xi, yi, zi, px, py, pz, ok, rho, ep);
             }
-            rho = lane_group_sum<kFzLanes>(rho) + brho;
-            ep = lane_group_sum<kFzLanes>(ep) + bep;
+            rho = row_sum<kFzLanes>(rho) + brho;
+            ep = row_sum<kFzLanes>(ep) + bep;
             if (q == 0) {
-                rw[sl] = inv_root<T>(rho);
-                many -= sqrt(rho);
+                rd[sl] = rho;
                 pair += ep;
             }
         }
     }
-    // free atoms: kFreeLanes lanes per list, entries strided over the lanes,
-    // the next batch (of this atom or the next) in flight during a batch
+    // free atoms: kFreeLanes lanes per list, entries strided over the lanes
     const int g = tid / kFreeLanes, sub = tid % kFreeLanes;
     constexpr int kGroups = kBlock / kFreeLanes, kBatch = kFreeLanes * kFreeIlp;
-    const int *fcnt = R.fcnt + w * kFree;
-    const uint16_t *flist = R.flist + (size_t)w * kFree * R.fcap;
+    const uint16_t *glist = R.flist + (size_t)w * kFree * R.fcap;
+    const uint16_t *llist = reinterpret_cast<const uint16_t *>(L.pool + 4 * S);
+    const bool lists = lists_fit(L.fofs[nf], S);
+    // the slots of entries k, k + kFreeLanes, ... of free atom f (-1: none)
     auto fetch = [&](int f, int k, int cnt, int (&e)[kFreeIlp]) {
 #pragma unroll
         for (int u = 0; u < kFreeIlp; ++u) {
             const int kk = k + u * kFreeLanes;
-            e[u] = kk < cnt ? int(flist[(size_t)f * R.fcap + kk]) : -1;
+            e[u] = -1;
+            if (kk < cnt) e[u] = lists ? int(llist[L.fofs[f] + kk]) : int(glist[(size_t)f * R.fcap + kk]);
         }
     };
-    {
-        int f = g, cnt = f < nf ? fcnt[f] : 0, en[kFreeIlp];
-        if (f < nf) fetch(f, sub, cnt, en);
-        while (f < nf) {
-            const int fn = f + kGroups, cn = fn < nf ? fcnt[fn] : 0;
-            const int sl = L.fslot[f], zt = L.zt[sl] & 127;
-            const double xi = L.fx[f], yi = L.fy[f], zi = L.fz[f];
-            double rho = 0.0, ep = 0.0;
-            for (int k = sub; k < cnt || k == sub; k += kBatch) {
-                int e[kFreeIlp];
+    for (int f = g; f < nf; f += kGroups) {
+        const int cnt = L.fofs[f + 1] - L.fofs[f];
+        const int sl = L.fslot[f], zt = L.zt[sl];
+        const double xi = L.fx[f], yi = L.fy[f], zi = L.fz[f];
+        double rho = 0.0, ep = 0.0;
+        for (int k = sub; k < cnt; k += kBatch) {
+            int e[kFreeIlp];
+            fetch(f, k, cnt, e);
+            double px[kFreeIlp], py[kFreeIlp], pz[kFreeIlp];
+            bool ok[kFreeIlp];
+            const SCPairDev *p[kFreeIlp];
 #pragma unroll
-                for (int u = 0; u < kFreeIlp; ++u) e[u] = en[u];
-                if (k + kBatch < cnt) fetch(f, k + kBatch, cnt, en);
-                else if (fn < nf) fetch(fn, sub, cn, en);
-                double px[kFreeIlp], py[kFreeIlp], pz[kFreeIlp];
-                bool ok[kFreeIlp];
-                const SCPairDev *p[kFreeIlp];
-#pragma unroll
-                for (int u = 0; u < kFreeIlp; ++u) {
-                    ok[u] = e[u] >= 0;
-                    const int j = ok[u] ? e[u] : sl;
-                    px[u] = rx[j];
-                    py[u] = ry[j];
-                    pz[u] = rz[j];
-                    p[u] = KIND == 1 ? nullptr : L.tab + zt * ns + (L.zt[j] & 127);
-                }
-                add_density<T, KIND, kFreeIlp>(W, rc2, c1, p, xi, yi, zi, px, py, pz, ok, rho, ep);
+            for (int u = 0; u < kFreeIlp; ++u) {
+                ok[u] = e[u] >= 0;
+                const int j = ok[u] ? e[u] : sl;
+                px[u] = rx[j];
+                py[u] = ry[j];
+                pz[u] = rz[j];
+                p[u] = KIND == 1 ? nullptr : L.tab + zt * ns + L.zt[j];
             }
-            rho = lane_group_sum<kFreeLanes>(rho);
-            ep = lane_group_sum<kFreeLanes>(ep);
-            if (sub == 0) {
-                rw[sl] = inv_root<T>(rho);
-                many -= sqrt(rho);
-                pair += ep;
-            }
-            f = fn;
-            cnt = cn;
+            add_density<T, KIND, kFreeIlp>(W, rc2, c1, p, xi, yi, zi, px, py, pz, ok, rho, ep);
+        }
+        rho = row_sum<kFreeLanes>(rho);
+        ep = row_sum<kFreeLanes>(ep);
+        if (sub == 0) {
+            rd[sl] = rho;
+            pair += ep;
         }
     }
     __syncthreads();
+    // embedding energies and 1/sqrt(rho), a slot per thread
+    for (int k = tid; k < nz; k += kBlock) {
+        const double rho = rd[k], r = sqrt(rho);
+        many -= r;
+        rw[kRw * k] = rho < 1.0e-8 ? T(-1) : T(1.0 / r);
+    }
+    __syncthreads();
     // forces of the free atoms (the expressions of the chain's pass 2)
-    {
-        int f = g, cnt = f < nf ? fcnt[f] : 0, en[kFreeIlp];
-        if (f < nf) fetch(f, sub, cnt, en);
-        while (f < nf) {
-            const int fn = f + kGroups, cn = fn < nf ? fcnt[fn] : 0;
-            const int sl = L.fslot[f], zt = L.zt[sl] & 127;
-            const double xi = L.fx[f], yi = L.fy[f], zi = L.fz[f];
-            const T isi = rw[sl];
-            double fx = 0.0, fy = 0.0, fz = 0.0;
-            for (int k = sub; k < cnt || k == sub; k += kBatch) {
-                int e[kFreeIlp];
+    for (int f = g; f < nf; f += kGroups) {
+        const int cnt = L.fofs[f + 1] - L.fofs[f];
+        const int sl = L.fslot[f], zt = L.zt[sl];
+        const double xi = L.fx[f], yi = L.fy[f], zi = L.fz[f];
+        const T isi = rw[kRw * sl];
+        double fx = 0.0, fy = 0.0, fz = 0.0;
+        for (int k = sub; k < cnt; k += kBatch) {
+            int e[kFreeIlp];
+            fetch(f, k, cnt, e);
+            double dx[kFreeIlp], dy[kFreeIlp], dz[kFreeIlp], r2[kFreeIlp];
+            T isj[kFreeIlp];
+            bool in[kFreeIlp];
+            const SCPairDev *p[kFreeIlp];
 #pragma unroll
-                for (int u = 0; u < kFreeIlp; ++u) e[u] = en[u];
-                if (k + kBatch < cnt) fetch(f, k + kBatch, cnt, en);
-                else if (fn < nf) fetch(fn, sub, cn, en);
-                double dx[kFreeIlp], dy[kFreeIlp], dz[kFreeIlp], r2[kFreeIlp];
-                T isj[kFreeIlp];
-                bool in[kFreeIlp];
-                const SCPairDev *p[kFreeIlp];
-#pragma unroll
-                for (int u = 0; u < kFreeIlp; ++u) {
-                    const int j = e[u] >= 0 ? e[u] : sl;
-                    dx[u] = xi - rx[j];
-                    dy[u] = yi - ry[j];
-                    dz[u] = zi - rz[j];
-                    isj[u] = rw[j];
-                    p[u] = KIND == 1 ? nullptr : L.tab + zt * ns + (L.zt[j] & 127);
-                    min_image(dx[u], dy[u], dz[u], W);
-                    r2[u] = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
-                    in[u] = e[u] >= 0 && r2[u] <= rc2 && r2[u] > 1.0e-16;
-                }
-                T ir2[kFreeIlp], un[kFreeIlp], um[kFreeIlp];
-                pair_terms<T, KIND, kFreeIlp>(r2, in, c1, p, ir2, un, um);
-#pragma unroll
-                for (int u = 0; u < kFreeIlp; ++u) {
-                    const SCCoef<T> &c = coef_of<T, KIND>(c1, p[u]);
-                    const T fs = c.fs_coef * un[u];
-                    const T fm = (isi >= T(0) && isj[u] >= T(0)) ? c.fm_coef * (isi + isj[u]) * um[u] : T(0);
-                    T ft = in[u] ? (fs - fm) * ir2[u] : T(0);
-                    if constexpr (sizeof(T) == 4) asm("" : "+v"(ft));
-                    const double dft = double(ft);
-                    fx += dft * dx[u];
-                    fy += dft * dy[u];
-                    fz += dft * dz[u];
-                }
+            for (int u = 0; u < kFreeIlp; ++u) {
+                const int j = e[u] >= 0 ? e[u] : sl;
+                dx[u] = xi - rx[j];
+                dy[u] = yi - ry[j];
+                dz[u] = zi - rz[j];
+                isj[u] = rw[kRw * j];
+                p[u] = KIND == 1 ? nullptr : L.tab + zt * ns + L.zt[j];
+                min_image(dx[u], dy[u], dz[u], W);
+                r2[u] = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
+                in[u] = e[u] >= 0 && r2[u] <= rc2 && r2[u] > 1.0e-16;
             }
-            fx = lane_group_sum<kFreeLanes>(fx);
-            fy = lane_group_sum<kFreeLanes>(fy);
-            fz = lane_group_sum<kFreeLanes>(fz);
-            if (sub == 0) {
-                const int i = W.off + L.fid[f];
-                b.fx[i] = fx;
-                b.fy[i] = fy;
-                b.fz[i] = fz;
+            T ir2[kFreeIlp], un[kFreeIlp], um[kFreeIlp];
+            pair_terms<T, KIND, kFreeIlp>(r2, in, c1, p, ir2, un, um);
+#pragma unroll
+            for (int u = 0; u < kFreeIlp; ++u) {
+                const SCCoef<T> &c = coef_of<T, KIND>(c1, p[u]);
+                const T fs = c.fs_coef * un[u];
+                const T fm = (isi >= T(0) && isj[u] >= T(0)) ? c.fm_coef * (isi + isj[u]) * um[u] : T(0);
+                T ft = in[u] ? (fs - fm) * ir2[u] : T(0);
+                if constexpr (sizeof(T) == 4) asm("" : "+v"(ft));
+                const double dft = double(ft);
+                fx += dft * dx[u];
+                fy += dft * dy[u];
+                fz += dft * dz[u];
             }
-            f = fn;
-            cnt = cn;
+        }
+        fx = row_sum<kFreeLanes>(fx);
+        fy = row_sum<kFreeLanes>(fy);
+        fz = row_sum<kFreeLanes>(fz);
+        if (sub == 0) {
+            const int i = W.off + L.fid[f];
+            b.fx[i] = fx;
+            b.fy[i] = fy;
+            b.fz[i] = fz;
         }
     }
     double v[2] = {many, pair};
@@ -509,14 +638,33 @@ __device__ __forceinline__ void res_eval(const BatchDev &b, const WalkerDev &W, 
     __syncthreads();
 }
 
+// the walker's state machine
+template <int KIND>
+__device__ __attribute__((noinline)) void res_step(const ResArgs *args, int nf)
+{
+    ResLds<KIND> &L = res_lds<KIND>();
+    const BatchDev b = load_uniform(&args->b);
+    const SearchDev s = load_uniform(&args->s);
+    const WalkerDev *W = b.walkers + blockIdx.x;
+    Ctx C_{b, s, load_uniform(&W->off), load_uniform(&W->n), b.A, nf, L.pool};
+    // the walker's scalars are private to each thread during its step (all
+    // threads take the same branches) and in LDS during the evaluations
+    WalkerState w = L.ws;
+    walker_step(C_, w, L.sh);
+    __syncthreads();
+    if (threadIdx.x == 0) L.ws = w;
+}
+
 // Micro-steps of resident walkers, one workgroup each.  A walker whose full
 // evaluation in its precision is pending has had it from the chain that ran
-// before this launch when the launch begins; one that comes to need it later
-// (a search entering FP64 verification) waits for the next launch.
+// before a service launch; one that comes to need it later (a search
+// entering FP64 verification) waits for the next service launch.
 template <int KIND>
-__global__ void __launch_bounds__(kBlock, 2) k_search_resident(BatchDev b, SearchDev s, int nsteps, int logic)
+__global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *args, int nsteps, int logic, int service)
 {
-    __shared__ ResLds<KIND> L;
+    ResLds<KIND> &L = res_lds<KIND>();
+    const BatchDev b = load_uniform(&args->b);
+    const SearchDev s = load_uniform(&args->s);
     const int wid = blockIdx.x, tid = threadIdx.x;
     int flags = b.zflag[wid];
     if (!(flags & AKMC_ZONE_RES) || b.active[wid] == 0) return;
@@ -524,24 +672,28 @@ __global__ void __launch_bounds__(kBlock, 2) k_search_resident(BatchDev b, Searc
     if constexpr (KIND != 1) stage_sc_table(*b.field, L.tab);
     __syncthreads();
     if (L.ws.kind == WK_IDLE || L.ws.state == ST_DONE) return;
-    const WalkerDev W = b.walkers[wid];
+    const WalkerDev W = load_uniform(b.walkers + wid);
     const int nf = s.nact[wid];
-    Ctx C_{b, s, W.off, W.n, b.A, nf, L.pool};
     const double h2 = b.field->half_skin2;
-    int nz = b.r.n[wid], evals32 = 0;
-    if (nz >= 0)
+    int nz = b.r.n[wid], evals32 = 0, eok = b.r.eok[wid];
+    if (nz >= 0) {
         for (int f = tid; f < nf; f += kBlock) L.fslot[f] = b.r.fslot[wid * kFree + f];
+        res_offsets<KIND>(b.r.fcnt + wid * kFree, nf);
+    }
     for (int f = tid; f < nf; f += kBlock) L.fid[f] = uint16_t(s.act[W.off + f] - W.off);
     bool loaded = false, too_big = false;  // loaded: the zone's records are in the pool
     for (int step = 0; step < nsteps; ++step) {
         __syncthreads();
         if (L.ws.state == ST_DONE) break;
-        const int mode = b.active[wid], prec = mode == 2 ? 1 : 0;
+        // the mode the state machine left the walker in (BatchDev.active)
+        const int mode = step == 0 ? b.active[wid]
+                                   : (L.ws.kind == WK_VERIFY || L.ws.state == ST_R_E64) ? 2 : s.default_mode;
+        const int prec = mode == 2 ? 1 : 0;
         const int full = prec ? AKMC_ZONE_FULL64 : AKMC_ZONE_FULL32;
         if (flags & full) {
-            if (step > 0) break;
+            if (step > 0 || !service) break;
             flags &= ~full;
-            if (tid == 0) b.r.eok[wid] &= ~(1 << prec);
+            eok &= ~(1 << prec);
         }
         bool moved = nz < 0;
         for (int f = tid; f < nf; f += kBlock) {
@@ -557,50 +709,60 @@ __global__ void __launch_bounds__(kBlock, 2) k_search_resident(BatchDev b, Searc
             }
         }
         if (__syncthreads_or(moved)) {
-            if (!res_build(b, s, W, L, nf)) {
+            if (!res_build<KIND>(args, nf)) {
                 too_big = true;
                 break;
             }
             nz = b.r.n[wid];
+            res_offsets<KIND>(b.r.fcnt + wid * kFree, nf);
+            __syncthreads();
+            eok = 0;
             loaded = false;
         }
-        if (!(b.r.eok[wid] & (1 << prec))) {
-            res_outside(b, W, L, nz, prec);
+        if (!(eok & (1 << prec))) {
+            res_outside<KIND>(args, nz, prec);
+            eok |= 1 << prec;
             loaded = false;
         }
+        const int S = slot_stride(nz);
         if (!loaded) {
             for (int k = tid; k < nz; k += kBlock) {
                 const int i = W.off + b.r.slot[(size_t)wid * kSlots + k];
                 L.pool[k] = b.x[i];
-                L.pool[kSlots + k] = b.y[i];
-                L.pool[2 * kSlots + k] = b.z[i];
-                L.zt[k] = uint8_t(b.type[i] | (s.frozen[i] ? 0 : 128));
+                L.pool[S + k] = b.y[i];
+                L.pool[2 * S + k] = b.z[i];
+                L.zt[k] = uint8_t(b.type[i]);
+            }
+            if (lists_fit(L.fofs[nf], S)) {
+                uint16_t *llist = reinterpret_cast<uint16_t *>(L.pool + 4 * S);
+                const int lane = tid & 63;
+                for (int f = tid >> 6; f < nf; f += kWaves) {
+                    const uint16_t *gl = b.r.flist + ((size_t)wid * kFree + f) * b.r.fcap;
+                    const int o = L.fofs[f], n = L.fofs[f + 1] - o;
+                    for (int k = lane; k < n; k += 64) llist[o + k] = gl[k];
+                }
             }
             loaded = true;
         } else {
             for (int f = tid; f < nf; f += kBlock) {
                 const int k = L.fslot[f];
                 L.pool[k] = L.fx[f];
-                L.pool[kSlots + k] = L.fy[f];
-                L.pool[2 * kSlots + k] = L.fz[f];
+                L.pool[S + k] = L.fy[f];
+                L.pool[2 * S + k] = L.fz[f];
             }
         }
         __syncthreads();
-        if (prec) res_eval<double, KIND>(b, W, L, nf, nz);
-        else res_eval<float, KIND>(b, W, L, nf, nz);
+        if (prec) res_eval<double, KIND>(args, nf, nz);
+        else res_eval<float, KIND>(args, nf, nz);
         if (!logic) break;
         evals32 += mode == 1;
-        // the walker's scalars are private to each thread during its step (all
-        // threads take the same branches) and in LDS during the evaluations
-        WalkerState w = L.ws;
-        if (w.kind == WK_VERIFY) loaded = false;  // its Lanczos vectors take the pool
-        walker_step(C_, w, L.sh);
-        __syncthreads();
-        if (tid == 0) L.ws = w;
+        if (L.ws.kind == WK_VERIFY) loaded = false;  // its Lanczos vectors take the pool
+        res_step<KIND>(args, nf);
     }
     __syncthreads();
     if (tid == 0) {
         b.zflag[wid] = flags;
+        b.r.eok[wid] = eok;
         if (too_big) L.ws.too_big = 1;
         if (logic || too_big) s.ws[wid] = L.ws;
         s.evals32[wid] += evals32;
@@ -693,13 +855,13 @@ void akmc_launch_res_base(const BatchDev &b, const FieldDev &hf, hipStream_t st)
     }
 }
 
-void akmc_launch_search_resident(const BatchDev &b, const FieldDev &hf, const SearchDev &s, int nsteps, int logic,
-                                 hipStream_t st)
+void akmc_launch_search_resident(int nwalkers, const FieldDev &hf, const ResArgs *args, int nsteps, int logic,
+                                 int service, hipStream_t st)
 {
     switch (akmc_sc_kind(hf)) {
-    case 1: k_search_resident<1><<<b.W, kBlock, 0, st>>>(b, s, nsteps, logic); break;
-    case 2: k_search_resident<2><<<b.W, kBlock, 0, st>>>(b, s, nsteps, logic); break;
-    default: k_search_resident<0><<<b.W, kBlock, 0, st>>>(b, s, nsteps, logic);
+    case 1: k_search_resident<1><<<nwalkers, kBlock, 0, st>>>(args, nsteps, logic, service); break;
+    case 2: k_search_resident<2><<<nwalkers, kBlock, 0, st>>>(args, nsteps, logic, service); break;
+    default: k_search_resident<0><<<nwalkers, kBlock, 0, st>>>(args, nsteps, logic, service);
     }
 }
 
