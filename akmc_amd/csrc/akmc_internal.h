@@ -409,14 +409,27 @@ void akmc_launch_harvest_pack(const BatchDev &b, const SearchDev &s, int *harves
 // learned proposal (mlp_kernels.hip)
 void akmc_mlp_launch_weights(const float *p, uint16_t *w1t, uint16_t *w2t, uint16_t *w3t, uint16_t *w2r,
                              uint16_t *w3r, hipStream_t s);
+#define AKMC_MLP_PARAMS 23171
+#define AKMC_MLP_MAXBLOCKS 256  // workgroups of the gradient kernel at most
+// rows of X standardised in place: (X - mean) * scale
+void akmc_mlp_launch_standardize(float *X, long long rows, const float *mean, const float *scale, hipStream_t s);
+// Y [M][3] of the rows X [M][48]
 void akmc_mlp_launch_forward(const float *X, int M, const float *p, const uint16_t *w1t, const uint16_t *w2t,
-                             const uint16_t *w3t, float *Z1, float *H1, float *Z2, float *H2, float *Y, hipStream_t s);
-void akmc_mlp_launch_backward(const float *X, const float *T, int M, const uint16_t *w2r, const uint16_t *w3r,
-                              const float *Z1, const float *H1, const float *Z2, const float *H2, const float *Y,
-                              float *dY, float *dZ2, float *dZ1, double *loss_part, float *P, int rows_per_chunk,
-                              float *grad, hipStream_t s);
-void akmc_mlp_launch_adam(float *p, const float *g, float *m1, float *m2, int n, float lr, int t, hipStream_t s);
-void akmc_mlp_launch_gather(const float *src, int width, const int *idx, int M, float *dst, hipStream_t s);
-void akmc_mlp_launch_loss_accum(const double *part, int nb, double scale, double *acc, hipStream_t s);
-void akmc_mlp_launch_descriptors(const BatchDev &b, int nq, const int *qatom, const double *qvac,
-                                 const double *qmov, float *X, hipStream_t s);
+                             const uint16_t *w3t, float *Y, hipStream_t s);
+// gradient sums of rows idx[0 .. M) (null: rows 0 .. M) per workgroup into P
+// [blocks][AKMC_MLP_PARAMS], squared errors into part [blocks]
+int akmc_mlp_grad_blocks(int M);
+void akmc_mlp_launch_grad(const float *X, const float *T, const int *idx, int M, const float *p, const uint16_t *w1t,
+                          const uint16_t *w2t, const uint16_t *w3t, const uint16_t *w2r, const uint16_t *w3r, float *P,
+                          double *part, hipStream_t s);
+// the gradient g from P; step: Adam step t and the BF16 weights too; the mean
+// loss of the M rows is added to acc (device, may be null)
+void akmc_mlp_launch_update(const float *P, int M, float *g, float *p, float *m1, float *m2, uint16_t *w1t,
+                            uint16_t *w2t, uint16_t *w3t, uint16_t *w2r, uint16_t *w3r, int step, float lr, int t,
+                            const double *part, double *acc, hipStream_t s);
+// descriptors of nq queries (atom, site, mover): the terms of the na distinct
+// atoms into G [na][32], then the rows X [nq][48] (qslot: a query's atom in
+// the list of distinct ones)
+void akmc_mlp_launch_descriptors(const BatchDev &b, int na, const int *atoms, int nq, const int *qatom,
+                                 const int *qslot, const double *qvac, const double *qmov, float *G, float *X,
+                                 hipStream_t s);

@@ -183,6 +183,8 @@ struct akmc_batch_s {
     size_t gat_n = 0;
     int inflight = 0;           // a chunk launched by akmc_batch_run_async awaits its wait
     int inflight_steps = 0;
+    char *desc_dev = nullptr;   // device buffer of akmc_batch_descriptors (grows to the largest call)
+    size_t desc_n = 0;
     void *stage_pin = nullptr;  // pinned host / device staging of walker starts
     void *stage_dev = nullptr;
     size_t stage_n = 0;
@@ -879,6 +881,7 @@ void batch_free(akmc_batch_t b)
     if (b->ov_pin) (void)hipHostFree(b->ov_pin);
     if (b->gat_pin) (void)hipHostFree(b->gat_pin);
     if (b->gat_dev) (void)hipFree(b->gat_dev);
+    if (b->desc_dev) (void)hipFree(b->desc_dev);
     if (b->stage_pin) (void)hipHostFree(b->stage_pin);
     if (b->stage_dev) (void)hipFree(b->stage_dev);
     if (b->st_pin) (void)hipHostFree(b->st_pin);
@@ -2604,11 +2607,9 @@ struct akmc_mlp_s {
     std::vector<void *> allocs;
     float *p = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr;
     uint16_t *w1t = nullptr, *w2t = nullptr, *w3t = nullptr, *w2r = nullptr, *w3r = nullptr;
-    float *X = nullptr, *T = nullptr, *Z1 = nullptr, *H1 = nullptr, *Z2 = nullptr, *H2 = nullptr, *Y = nullptr,
-          *dY = nullptr, *dZ2 = nullptr, *dZ1 = nullptr, *P = nullptr;
+    float *X = nullptr, *T = nullptr, *Y = nullptr, *P = nullptr, *ms = nullptr;  // ms: mean and scale of the inputs
     double *lpart = nullptr;
     int adam_t = 0;
-    static constexpr int kChunk = 256;
 };
 
 namespace {
@@ -2636,22 +2637,24 @@ int mlp_refresh_weights(akmc_mlp_t m)
     return AKMC_SUCCESS;
 }
 
-// forward + loss/gradient of rows [0, M) already in m->X / m->T
-int mlp_loss_grad_dev(akmc_mlp_t m, int M, double *loss)
+// the inputs' mean and scale on the device (null: none)
+int mlp_scaling(akmc_mlp_t m, const float *mean, const float *scale)
 {
-    akmc_mlp_launch_forward(m->X, M, m->p, m->w1t, m->w2t, m->w3t, m->Z1, m->H1, m->Z2, m->H2, m->Y, m->stream);
-    akmc_mlp_launch_backward(m->X, m->T, M, m->w2r, m->w3r, m->Z1, m->H1, m->Z2, m->H2, m->Y, m->dY, m->dZ2,
-                             m->dZ1, m->lpart, m->P, akmc_mlp_s::kChunk, m->g, m->stream);
+    if (!mean) return AKMC_SUCCESS;
+    HIPCHK(hipMemcpyAsync(m->ms, mean, 48 * sizeof(float), hipMemcpyHostToDevice, m->stream));
+    HIPCHK(hipMemcpyAsync(m->ms + 48, scale, 48 * sizeof(float), hipMemcpyHostToDevice, m->stream));
+    return AKMC_SUCCESS;
+}
+
+// gradient sums of rows idx of (X, T), then the gradient (and, with step, the
+// Adam step); acc: where the rows' mean loss is added, or null
+int mlp_grad(akmc_mlp_t m, const float *X, const float *T, const int *idx, int M, int step, float lr, double *acc)
+{
+    akmc_mlp_launch_grad(X, T, idx, M, m->p, m->w1t, m->w2t, m->w3t, m->w2r, m->w3r, m->P, m->lpart, m->stream);
+    if (step) ++m->adam_t;
+    akmc_mlp_launch_update(m->P, M, m->g, m->p, m->m1, m->m2, m->w1t, m->w2t, m->w3t, m->w2r, m->w3r, step, lr,
+                           std::max(m->adam_t, 1), m->lpart, acc, m->stream);
     HIPCHK(hipGetLastError());
-    if (loss) {
-        int nb = (M + 255) / 256;
-        std::vector<double> part(nb);
-        HIPCHK(hipMemcpyAsync(part.data(), m->lpart, nb * sizeof(double), hipMemcpyDeviceToHost, m->stream));
-        HIPCHK(hipStreamSynchronize(m->stream));
-        double s = 0.0;
-        for (double v : part) s += v;
-        *loss = s / M;
-    }
     return AKMC_SUCCESS;
 }
 }  // namespace
@@ -2677,12 +2680,9 @@ int akmc_mlp_create(int max_rows, unsigned seed, akmc_mlp_t *out)
         (rc = malloc_m(m, &m->w2t, 128 * 128)) || (rc = malloc_m(m, &m->w3t, 16 * 128)) ||
         (rc = malloc_m(m, &m->w2r, 128 * 128)) || (rc = malloc_m(m, &m->w3r, 128 * 16)) ||
         (rc = malloc_m(m, &m->X, R * 48)) || (rc = malloc_m(m, &m->T, R * 3)) ||
-        (rc = malloc_m(m, &m->Z1, R * 128)) || (rc = malloc_m(m, &m->H1, R * 128)) ||
-        (rc = malloc_m(m, &m->Z2, R * 128)) || (rc = malloc_m(m, &m->H2, R * 128)) ||
-        (rc = malloc_m(m, &m->Y, R * 16)) || (rc = malloc_m(m, &m->dY, R * 16)) ||
-        (rc = malloc_m(m, &m->dZ2, R * 128)) || (rc = malloc_m(m, &m->dZ1, R * 128)) ||
-        (rc = malloc_m(m, &m->P, (R / akmc_mlp_s::kChunk + 1) * 128 * 128)) ||
-        (rc = malloc_m(m, &m->lpart, R / 256 + 1)))
+        (rc = malloc_m(m, &m->Y, R * 3)) ||
+        (rc = malloc_m(m, &m->P, (size_t)akmc_mlp_grad_blocks((int)R) * NP)) ||
+        (rc = malloc_m(m, &m->lpart, AKMC_MLP_MAXBLOCKS)) || (rc = malloc_m(m, &m->ms, 96)))
         return bad(rc);
     HIPCHK(hipMemset(m->m1, 0, NP * sizeof(float)));
     HIPCHK(hipMemset(m->m2, 0, NP * sizeof(float)));
@@ -2732,20 +2732,24 @@ int akmc_mlp_get_params(akmc_mlp_t m, float *params)
 
 int akmc_mlp_forward(akmc_mlp_t m, const float *X, int M, float *Y)
 {
-    if (!m || !X || !Y || M < 0) return fail(AKMC_EINVAL, "bad arguments");
-    std::vector<float> y16;
+    return akmc_mlp_forward_scaled(m, X, nullptr, nullptr, M, Y);
+}
+
+int akmc_mlp_forward_scaled(akmc_mlp_t m, const float *X, const float *mean, const float *scale, int M, float *Y)
+{
+    if (!m || !X || !Y || M < 0 || !mean != !scale) return fail(AKMC_EINVAL, "bad arguments");
+    TRY(mlp_scaling(m, mean, scale));
     for (int r0 = 0; r0 < M; r0 += m->rows) {
         int n = std::min(m->rows, M - r0);
         HIPCHK(hipMemcpyAsync(m->X, X + (size_t)r0 * 48, (size_t)n * 48 * sizeof(float), hipMemcpyHostToDevice,
                               m->stream));
-        akmc_mlp_launch_forward(m->X, n, m->p, m->w1t, m->w2t, m->w3t, m->Z1, m->H1, m->Z2, m->H2, m->Y, m->stream);
+        if (mean) akmc_mlp_launch_standardize(m->X, n, m->ms, m->ms + 48, m->stream);
+        akmc_mlp_launch_forward(m->X, n, m->p, m->w1t, m->w2t, m->w3t, m->Y, m->stream);
         HIPCHK(hipGetLastError());
-        y16.resize((size_t)n * 16);
-        HIPCHK(hipMemcpyAsync(y16.data(), m->Y, (size_t)n * 16 * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-        HIPCHK(hipStreamSynchronize(m->stream));
-        for (int i = 0; i < n; ++i)
-            for (int c = 0; c < 3; ++c) Y[(size_t)(r0 + i) * 3 + c] = y16[(size_t)i * 16 + c];
+        HIPCHK(hipMemcpyAsync(Y + (size_t)r0 * 3, m->Y, (size_t)n * 3 * sizeof(float), hipMemcpyDeviceToHost,
+                              m->stream));
     }
+    HIPCHK(hipStreamSynchronize(m->stream));
     return AKMC_SUCCESS;
 }
 
@@ -2754,10 +2758,16 @@ int akmc_mlp_loss_grad(akmc_mlp_t m, const float *X, const float *T, int M, doub
     if (!m || !X || !T || M <= 0 || M > m->rows) return fail(AKMC_EINVAL, "M must be in [1, max_rows]");
     HIPCHK(hipMemcpyAsync(m->X, X, (size_t)M * 48 * sizeof(float), hipMemcpyHostToDevice, m->stream));
     HIPCHK(hipMemcpyAsync(m->T, T, (size_t)M * 3 * sizeof(float), hipMemcpyHostToDevice, m->stream));
-    TRY(mlp_loss_grad_dev(m, M, loss));
-    if (grad) {
-        HIPCHK(hipMemcpyAsync(grad, m->g, AKMC_MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost, m->stream));
-        HIPCHK(hipStreamSynchronize(m->stream));
+    TRY(mlp_grad(m, m->X, m->T, nullptr, M, 0, 0.0f, nullptr));
+    std::vector<double> part(akmc_mlp_grad_blocks(M));
+    if (loss)
+        HIPCHK(hipMemcpyAsync(part.data(), m->lpart, part.size() * sizeof(double), hipMemcpyDeviceToHost, m->stream));
+    if (grad) HIPCHK(hipMemcpyAsync(grad, m->g, AKMC_MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost, m->stream));
+    HIPCHK(hipStreamSynchronize(m->stream));
+    if (loss) {
+        double s = 0.0;
+        for (double v : part) s += v;
+        *loss = s / M;
     }
     return AKMC_SUCCESS;
 }
@@ -2769,12 +2779,13 @@ int akmc_mlp_time(akmc_mlp_t m, int M, int nrep, double ms[2])
     HIPCHK(hipMemsetAsync(m->T, 0, (size_t)M * 3 * sizeof(float), m->stream));
     hipEvent_t e[3];
     for (auto &v : e) HIPCHK(hipEventCreate(&v));
-    TRY(mlp_loss_grad_dev(m, M, nullptr));  // first launches outside the timing
+    TRY(mlp_grad(m, m->X, m->T, nullptr, M, 0, 0.0f, nullptr));  // first launches outside the timing
+    akmc_mlp_launch_forward(m->X, M, m->p, m->w1t, m->w2t, m->w3t, m->Y, m->stream);
     HIPCHK(hipEventRecord(e[0], m->stream));
     for (int r = 0; r < nrep; ++r)
-        akmc_mlp_launch_forward(m->X, M, m->p, m->w1t, m->w2t, m->w3t, m->Z1, m->H1, m->Z2, m->H2, m->Y, m->stream);
+        akmc_mlp_launch_forward(m->X, M, m->p, m->w1t, m->w2t, m->w3t, m->Y, m->stream);
     HIPCHK(hipEventRecord(e[1], m->stream));
-    for (int r = 0; r < nrep; ++r) TRY(mlp_loss_grad_dev(m, M, nullptr));
+    for (int r = 0; r < nrep; ++r) TRY(mlp_grad(m, m->X, m->T, nullptr, M, 0, 0.0f, nullptr));
     HIPCHK(hipEventRecord(e[2], m->stream));
     HIPCHK(hipEventSynchronize(e[2]));
     float t0 = 0.0f, t1 = 0.0f;
@@ -2789,10 +2800,18 @@ int akmc_mlp_time(akmc_mlp_t m, int M, int nrep, double ms[2])
 int akmc_mlp_train(akmc_mlp_t m, const float *X, const float *T, int M, int epochs, int batch, float lr,
                    unsigned seed, double *loss_history)
 {
-    if (!m || !X || !T || M <= 0 || epochs <= 0 || batch <= 0 || batch > m->rows)
+    return akmc_mlp_train_scaled(m, X, nullptr, nullptr, T, M, epochs, batch, lr, seed, loss_history);
+}
+
+int akmc_mlp_train_scaled(akmc_mlp_t m, const float *X, const float *mean, const float *scale, const float *T, int M,
+                          int epochs, int batch, float lr, unsigned seed, double *loss_history)
+{
+    if (!m || !X || !T || M <= 0 || epochs <= 0 || batch <= 0 || batch > m->rows || !mean != !scale)
         return fail(AKMC_EINVAL, "bad training arguments (batch must be <= max_rows)");
+    TRY(mlp_scaling(m, mean, scale));
     float *dX = nullptr, *dT = nullptr;
     int *didx = nullptr;
+    hipEvent_t copied = nullptr;  // the permutation has left host memory
     double *dacc = nullptr;  // per-epoch loss accumulator (no host sync per minibatch)
     HIPCHK(hipMalloc(&dX, (size_t)M * 48 * sizeof(float)));
     HIPCHK(hipMalloc(&dT, (size_t)M * 3 * sizeof(float)));
@@ -2804,11 +2823,25 @@ int akmc_mlp_train(akmc_mlp_t m, const float *X, const float *T, int M, int epoc
         (void)hipFree(dT);
         (void)hipFree(didx);
         (void)hipFree(dacc);
+        if (copied) (void)hipEventDestroy(copied);
     };
+    if (hipEventCreateWithFlags(&copied, hipEventDisableTiming) != hipSuccess) {
+        copied = nullptr;
+        cleanup();
+        return fail(AKMC_EHIP, "event creation failed");
+    }
     if (hipMemcpy(dX, X, (size_t)M * 48 * sizeof(float), hipMemcpyHostToDevice) != hipSuccess ||
         hipMemcpy(dT, T, (size_t)M * 3 * sizeof(float), hipMemcpyHostToDevice) != hipSuccess) {
         cleanup();
         return fail(AKMC_EHIP, "training data upload failed");
+    }
+    if (mean) {
+        akmc_mlp_launch_standardize(dX, M, m->ms, m->ms + 48, m->stream);
+        const hipError_t es = hipGetLastError();
+        if (es != hipSuccess) {
+            cleanup();
+            return fail(AKMC_EHIP, "standardisation: %s", hipGetErrorString(es));
+        }
     }
     std::vector<int> perm(M);
     unsigned long long st = 0xD1B54A32D192ED03ull ^ seed;
@@ -2819,33 +2852,22 @@ int akmc_mlp_train(akmc_mlp_t m, const float *X, const float *T, int M, int epoc
         z = (z ^ (z >> 27)) * 0x94D049BB133111EBull;
         return z ^ (z >> 31);
     };
-    int nbatch_ep = 1;
-    for (int ep = 0; ep < epochs; ++ep) {
-        // the previous epoch's copy of perm must be done before perm changes
-        if (ep > 0 && hipStreamSynchronize(m->stream) != hipSuccess) {
-            cleanup();
-            return fail(AKMC_EHIP, "training step failed");
-        }
+    auto shuffle = [&]() {
         for (int i = 0; i < M; ++i) perm[i] = i;
         for (int i = M - 1; i > 0; --i) std::swap(perm[i], perm[next() % (unsigned long long)(i + 1)]);
+    };
+    int nbatch_ep = 1;
+    shuffle();
+    for (int ep = 0; ep < epochs; ++ep) {
         if (hipMemcpyAsync(didx, perm.data(), (size_t)M * sizeof(int), hipMemcpyHostToDevice, m->stream) !=
-            hipSuccess) {
+                hipSuccess ||
+            hipEventRecord(copied, m->stream) != hipSuccess) {
             cleanup();
             return fail(AKMC_EHIP, "permutation upload failed");
         }
         int nb = 0;
         for (int b0 = 0; b0 + batch <= M || (b0 == 0 && M < batch); b0 += batch) {
-            int n = std::min(batch, M - b0);
-            akmc_mlp_launch_gather(dX, 48, didx + b0, n, m->X, m->stream);
-            akmc_mlp_launch_gather(dT, 3, didx + b0, n, m->T, m->stream);
-            int rc = mlp_loss_grad_dev(m, n, nullptr);
-            if (rc != AKMC_SUCCESS) {
-                cleanup();
-                return rc;
-            }
-            akmc_mlp_launch_loss_accum(m->lpart, (n + 255) / 256, 1.0 / n, dacc + ep, m->stream);
-            akmc_mlp_launch_adam(m->p, m->g, m->m1, m->m2, AKMC_MLP_NPARAM, lr, ++m->adam_t, m->stream);
-            rc = mlp_refresh_weights(m);
+            const int rc = mlp_grad(m, dX, dT, didx + b0, std::min(batch, M - b0), 1, lr, dacc + ep);
             if (rc != AKMC_SUCCESS) {
                 cleanup();
                 return rc;
@@ -2854,6 +2876,14 @@ int akmc_mlp_train(akmc_mlp_t m, const float *X, const float *T, int M, int epoc
             if (M < batch) break;
         }
         nbatch_ep = std::max(nb, 1);
+        // the next epoch's order while this one trains
+        if (ep + 1 < epochs) {
+            if (hipEventSynchronize(copied) != hipSuccess) {
+                cleanup();
+                return fail(AKMC_EHIP, "training step failed");
+            }
+            shuffle();
+        }
     }
     std::vector<double> acc(epochs);
     hipError_t e = hipMemcpyAsync(acc.data(), dacc, (size_t)epochs * sizeof(double), hipMemcpyDeviceToHost, m->stream);
@@ -2871,27 +2901,40 @@ int akmc_batch_descriptors(akmc_batch_t b, int nq, const int *atom, const double
     if (!b || nq <= 0 || !atom || !vac || !mover || !X) return fail(AKMC_EINVAL, "bad arguments");
     for (int q = 0; q < nq; ++q)
         if (atom[q] < 0 || atom[q] >= b->A) return fail(AKMC_EINVAL, "query %d: atom out of range", q);
-    int *qa;
-    double *qv, *qm;
-    float *qx;
-    HIPCHK(hipMalloc(&qa, nq * sizeof(int)));
-    HIPCHK(hipMalloc(&qv, 3 * (size_t)nq * sizeof(double)));
-    HIPCHK(hipMalloc(&qm, 3 * (size_t)nq * sizeof(double)));
-    HIPCHK(hipMalloc(&qx, 48 * (size_t)nq * sizeof(float)));
-    HIPCHK(hipMemcpyAsync(qa, atom, nq * sizeof(int), hipMemcpyHostToDevice, b->stream));
-    HIPCHK(hipMemcpyAsync(qv, vac, 3 * (size_t)nq * sizeof(double), hipMemcpyHostToDevice, b->stream));
-    HIPCHK(hipMemcpyAsync(qm, mover, 3 * (size_t)nq * sizeof(double), hipMemcpyHostToDevice, b->stream));
-    akmc_mlp_launch_descriptors(b->d, nq, qa, qv, qm, qx, b->stream);
+    // the distinct atoms, in the order they are first asked for
+    std::vector<int> slot_of(b->A, -1), uniq, ids(2 * (size_t)nq);
+    for (int q = 0; q < nq; ++q) {
+        int &sl = slot_of[atom[q]];
+        if (sl < 0) {
+            sl = (int)uniq.size();
+            uniq.push_back(atom[q]);
+        }
+        ids[q] = atom[q];
+        ids[nq + q] = sl;
+    }
+    const size_t n = nq, na = uniq.size();
+    // one buffer of the batch: sites, movers, rows, atom terms, indices
+    const size_t bytes = 48 * n + 192 * n + 128 * na + 8 * n + 4 * na;
+    if (bytes > b->desc_n) {
+        if (b->desc_dev) HIPCHK(hipFree(b->desc_dev));
+        b->desc_dev = nullptr;
+        b->desc_n = 0;
+        HIPCHK(hipMalloc((void **)&b->desc_dev, bytes));
+        b->desc_n = bytes;
+    }
+    double *qv = (double *)b->desc_dev, *qm = qv + 3 * n;
+    float *qx = (float *)(qm + 3 * n), *G = qx + 48 * n;
+    int *qi = (int *)(G + 32 * na), *ua = qi + 2 * n;
+    HIPCHK(hipMemcpyAsync(qv, vac, 3 * n * sizeof(double), hipMemcpyHostToDevice, b->stream));
+    HIPCHK(hipMemcpyAsync(qm, mover, 3 * n * sizeof(double), hipMemcpyHostToDevice, b->stream));
+    HIPCHK(hipMemcpyAsync(qi, ids.data(), 2 * n * sizeof(int), hipMemcpyHostToDevice, b->stream));
+    HIPCHK(hipMemcpyAsync(ua, uniq.data(), na * sizeof(int), hipMemcpyHostToDevice, b->stream));
+    akmc_mlp_launch_descriptors(b->d, (int)na, ua, nq, qi, qi + n, qv, qm, G, qx, b->stream);
     hipError_t e = hipGetLastError();
-    if (e == hipSuccess)
-        e = hipMemcpyAsync(X, qx, 48 * (size_t)nq * sizeof(float), hipMemcpyDeviceToHost, b->stream);
+    if (e == hipSuccess) e = hipMemcpyAsync(X, qx, 48 * n * sizeof(float), hipMemcpyDeviceToHost, b->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
-    (void)hipFree(qa);
-    (void)hipFree(qv);
-    (void)hipFree(qm);
-    (void)hipFree(qx);
     if (e != hipSuccess) return fail(AKMC_EHIP, "descriptors: %s", hipGetErrorString(e));
-    return AKMC_SUCCESS;
+    return check_overflow(b);
 }
 
 }  // extern "C"

@@ -35,6 +35,9 @@ def _setup(lib):
     lib.akmc_mlp_loss_grad.argtypes = [C.c_void_p, _F, _F, C.c_int, C.POINTER(C.c_double), _F]
     lib.akmc_mlp_train.argtypes = [C.c_void_p, _F, _F, C.c_int, C.c_int, C.c_int, C.c_float, C.c_uint,
                                    C.POINTER(C.c_double)]
+    lib.akmc_mlp_forward_scaled.argtypes = [C.c_void_p, _F, _F, _F, C.c_int, _F]
+    lib.akmc_mlp_train_scaled.argtypes = [C.c_void_p, _F, _F, _F, _F, C.c_int, C.c_int, C.c_int, C.c_float, C.c_uint,
+                                          C.POINTER(C.c_double)]
     lib.akmc_mlp_time.argtypes = [C.c_void_p, C.c_int, C.c_int, C.POINTER(C.c_double)]
     lib.akmc_batch_descriptors.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_int), C.POINTER(C.c_double),
                                            C.POINTER(C.c_double), _F]
@@ -123,12 +126,12 @@ class MLP:
 
     def train(self, X, T, epochs=20, batch=4096, lr=1e-3, seed=0):
         """Adam on standardised inputs; returns the per-epoch loss."""
-        Xs = _f32(self.standardize(X))
-        T = _f32(T)
+        X, T = _f32(X), _f32(T)
+        mean, scale = _f32(self.mean), _f32(self.scale)  # applied on the device
         hist = np.zeros(epochs)
-        L.check(L.load().akmc_mlp_train(self._h, _fp(Xs), _fp(T), Xs.shape[0], int(epochs),
-                                        int(min(batch, self.max_rows)), float(lr), int(seed),
-                                        hist.ctypes.data_as(C.POINTER(C.c_double))))
+        L.check(L.load().akmc_mlp_train_scaled(self._h, _fp(X), _fp(mean), _fp(scale), _fp(T), X.shape[0],
+                                               int(epochs), int(min(batch, self.max_rows)), float(lr), int(seed),
+                                               hist.ctypes.data_as(C.POINTER(C.c_double))))
         return hist
 
     def time(self, rows, nrep=20):
@@ -138,7 +141,10 @@ class MLP:
         return ms[0], ms[1]
 
     def predict(self, X):
-        return self.forward(self.standardize(X))
+        X, mean, scale = _f32(X), _f32(self.mean), _f32(self.scale)
+        Y = np.zeros((X.shape[0], 3), np.float32)
+        L.check(L.load().akmc_mlp_forward_scaled(self._h, _fp(X), _fp(mean), _fp(scale), X.shape[0], _fp(Y)))
+        return Y
 
 
 def batch_descriptors(batch: L.Batch, atoms_global, vac, mover):

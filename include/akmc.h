@@ -525,6 +525,8 @@ int akmc_mlp_set_params(akmc_mlp_t m, const float *params);
 int akmc_mlp_get_params(akmc_mlp_t m, float *params);
 /* Y[M][3] = MLP(X[M][48]) (host arrays, M <= max_rows per call chunk) */
 int akmc_mlp_forward(akmc_mlp_t m, const float *X, int M, float *Y);
+/* the same for rows standardised on the device: (X - mean[48]) * scale[48] */
+int akmc_mlp_forward_scaled(akmc_mlp_t m, const float *X, const float *mean, const float *scale, int M, float *Y);
 /* mean-squared loss against T[M][3] and its gradient (layout of params) */
 int akmc_mlp_loss_grad(akmc_mlp_t m, const float *X, const float *T, int M, double *loss, float *grad);
 /* Adam training on device-resident data: epochs passes in seeded random
@@ -535,6 +537,9 @@ int akmc_mlp_loss_grad(akmc_mlp_t m, const float *X, const float *T, int M, doub
 int akmc_mlp_time(akmc_mlp_t m, int M, int nrep, double ms[2]);
 int akmc_mlp_train(akmc_mlp_t m, const float *X, const float *T, int M, int epochs, int batch, float lr,
                    unsigned seed, double *loss_history);
+/* the same for rows standardised on the device: (X - mean[48]) * scale[48] */
+int akmc_mlp_train_scaled(akmc_mlp_t m, const float *X, const float *mean, const float *scale, const float *T, int M,
+                          int epochs, int batch, float lr, unsigned seed, double *loss_history);
 /* descriptors of nq queries (atom = index into the batch's concatenated
  * atoms; vac, mover = 3 doubles each) at the batch's resident positions,
  * whose neighbour lists must be current (after akmc_batch_forces) */
