@@ -103,6 +103,7 @@ struct FieldDev {
     int dsf_n;
     double dsf_del, dsf_rfld0, dsf_rfld1;
     SCPairDev sc[AKMC_MAXPAIR];
+    int all96;       // every species pair has a Sutton-Chen potential with n = 9, m = 6
     IonPairDev ion[AKMC_MAXPAIR];
     // tabulated EAM (kind 0 with eam = 1): species pair -> table (-1 none)
     int eam;
@@ -153,7 +154,7 @@ struct ResidentDev {
 
 struct BatchDev {
     int A, W, maxnb, ncells_total, nk_total, G1, maxnk;
-    int lpa;              // lanes per atom of the Sutton-Chen pair kernels (1, 2, 4)
+    int lpa;              // lanes per atom of the Sutton-Chen pair kernels (1, 2, 4, 8; 64: small cells)
     int nb16;             // list entries are 16-bit local indices (minimum-image
                           // many-body lists of walkers below 65536 atoms)
     int unroll;           // neighbour gathers in flight per lane (1, 2, 4, 8)
@@ -261,6 +262,8 @@ struct FieldView {
     int kind, min_image, eam, fp64;
 };
 int akmc_field_view(struct akmc_field_s *f, FieldView *v);
+// the pair kernels' variant for one cell of n atoms behind a plain force call
+void akmc_single_variant(int n, int &lpa, int &unroll);
 // records the message akmc_last_error() returns and passes code through
 extern "C" int akmc_fail(int code, const char *fmt, ...);
 

@@ -124,6 +124,12 @@ struct akmc_batch_s {
     hipStream_t stream = nullptr;
     std::vector<void *> allocs;
     std::vector<WalkerOut> hout;
+    // what a force call sends and gets back lies together on the device: x, y,
+    // z, type, rebuild and active flags, q; then forces, energy records and
+    // the overflow flag.  Small batches move each part in one transfer through
+    // pinned memory.
+    char *io = nullptr, *io_pin = nullptr;
+    size_t io_q = 0, io_in = 0, io_out = 0, io_end = 0;
     // LDS staging of the many-body pair kernels is possible when every
     // walker's gather records fit one workgroup's LDS
     bool stage_ok = false;
@@ -475,7 +481,23 @@ void build_tables(akmc_field_t f)
                 }
             }
         }
+    h.all96 = f->kind == 0 && f->eam.empty() ? 1 : 0;
+    for (int k = 0; k < ns * ns; ++k) h.all96 &= h.sc[k].on && h.sc[k].n_int == 9 && h.sc[k].m_int == 6;
 }
+
+// lanes per atom and gathers in flight of the pair kernels for one cell of n
+// atoms behind the plain force call.  Below two wavefronts per SIMD at 8
+// lanes (16,384 atoms) a wavefront per atom: 255 atoms 65 + 56 us at one lane,
+// 7 + 6 us so; above, 8 lanes: 31,980 alloy atoms 114 + 153 us at one lane
+// with the general powers, 20 + 23 us so with the table's straight products.  A batch keeps one size-independent default, so that a
+// walker gives the same bits alone and among others.
+}  // namespace
+void akmc_single_variant(int n, int &lpa, int &unroll)
+{
+    lpa = n < 16384 ? 64 : 8;
+    unroll = n < 16384 ? 1 : 2;
+}
+namespace {
 
 bool orthorhombic(const double *lat)
 {
@@ -712,8 +734,8 @@ int batch_build(akmc_field_t f, int W, const int *natoms, const double *lat, akm
     d.A = A;
     d.W = W;
     d.maxnb = maxnb;
-    d.lpa = 1;
-    d.unroll = 1;
+    d.lpa = 4;  // one default for every batch size (512 walkers: 0.72 ms an evaluation, 1.00 ms at 1 x 1)
+    d.unroll = 4;
     {
         int nmax = 0;
         for (int w = 0; w < W; ++w) nmax = std::max(nmax, natoms[w]);
@@ -736,27 +758,37 @@ int batch_build(akmc_field_t f, int W, const int *natoms, const double *lat, akm
     double *q;
     TRY(dalloc(b, &wd, W));
     TRY(dalloc(b, &wk, A));
-    TRY(dalloc(b, &tp, A));
-    TRY(dalloc(b, &q, A));
+    {
+        const size_t a = A, w = W, flags = 24 * a + 4 * a;
+        b->io_q = (flags + 8 * w + 15) / 16 * 16;
+        b->io_in = b->io_q + 8 * a;
+        b->io_out = (b->io_in + 255) / 256 * 256;
+        b->io_end = b->io_out + 24 * a + w * sizeof(WalkerOut) + sizeof(int);
+        TRY(dalloc(b, &b->io, b->io_end));
+        d.x = (double *)b->io;
+        d.y = d.x + a;
+        d.z = d.y + a;
+        tp = (int *)(d.z + a);
+        d.rebuild = tp + a;
+        d.active = d.rebuild + w;
+        q = (double *)(b->io + b->io_q);
+        d.fx = (double *)(b->io + b->io_out);
+        d.fy = d.fx + a;
+        d.fz = d.fy + a;
+        d.out = (WalkerOut *)(d.fz + a);
+        d.overflow = (int *)(d.out + w);
+    }
     d.walkers = wd;
     d.wk = wk;
     d.type = tp;
     d.q = q;
     TRY(dalloc(b, &d.p4, A));
-    TRY(dalloc(b, &d.x, A));
-    TRY(dalloc(b, &d.y, A));
-    TRY(dalloc(b, &d.z, A));
     TRY(dalloc(b, &d.xr, A));
     TRY(dalloc(b, &d.yr, A));
     TRY(dalloc(b, &d.zr, A));
-    TRY(dalloc(b, &d.fx, A));
-    TRY(dalloc(b, &d.fy, A));
-    TRY(dalloc(b, &d.fz, A));
     TRY(dalloc(b, &d.nbr, (size_t)(maxnb + AKMC_NB_PAD_ROWS) * A));
     TRY(dalloc(b, &d.nnb, A));
     TRY(dalloc(b, &d.nnear, A));
-    TRY(dalloc(b, &d.rebuild, W));
-    TRY(dalloc(b, &d.overflow, 1));
     TRY(dalloc(b, &d.cell_count, ncells));
     TRY(dalloc(b, &d.cell_start, ncells));
     TRY(dalloc(b, &d.cell_atoms, A));
@@ -769,8 +801,6 @@ int batch_build(akmc_field_t f, int W, const int *natoms, const double *lat, akm
     TRY(dalloc(b, &d.e_b64, A));
     TRY(dalloc(b, &d.e_c, A));
     TRY(dalloc(b, &d.st_atom, (size_t)6 * A));
-    TRY(dalloc(b, &d.out, W));
-    TRY(dalloc(b, &d.active, W));
     if (nk > 0) {
         int *kn;
         double *kv, *g0, *g1;
@@ -882,6 +912,7 @@ void batch_free(akmc_batch_t b)
     if (b->gat_pin) (void)hipHostFree(b->gat_pin);
     if (b->gat_dev) (void)hipFree(b->gat_dev);
     if (b->desc_dev) (void)hipFree(b->desc_dev);
+    if (b->io_pin) (void)hipHostFree(b->io_pin);
     if (b->stage_pin) (void)hipHostFree(b->stage_pin);
     if (b->stage_dev) (void)hipFree(b->stage_dev);
     if (b->st_pin) (void)hipHostFree(b->st_pin);
@@ -915,6 +946,20 @@ int check_overflow(akmc_batch_t b)
     int ov = 0;
     HIPCHK(hipMemcpyAsync(&ov, b->d.overflow, sizeof(int), hipMemcpyDeviceToHost, b->stream));
     HIPCHK(hipStreamSynchronize(b->stream));
+    return overflow_error(b, ov);
+}
+
+// forces, energy records and the overflow flag of a small batch in one
+// transfer (into hout and the pinned buffer)
+int fetch_all(akmc_batch_t b)
+{
+    char *pin = b->io_pin + b->io_out;
+    HIPCHK(hipMemcpyAsync(pin, b->io + b->io_out, b->io_end - b->io_out, hipMemcpyDeviceToHost, b->stream));
+    HIPCHK(hipStreamSynchronize(b->stream));
+    const char *out = pin + 24 * (size_t)b->A;
+    std::memcpy((void *)b->hout.data(), out, b->W * sizeof(WalkerOut));
+    int ov;
+    std::memcpy(&ov, out + b->W * sizeof(WalkerOut), sizeof ov);
     return overflow_error(b, ov);
 }
 
@@ -968,17 +1013,47 @@ int ensure_single(akmc_field_t f, int n, const double *lat)
         f->single = nullptr;
         return rc;
     }
+    akmc_single_variant(n, f->single->d.lpa, f->single->d.unroll);
     f->single_n = n;
     std::memcpy(f->single_lat, lat, sizeof f->single_lat);
     return AKMC_SUCCESS;
 }
 
-int upload(akmc_batch_t b, const double *x, const double *y, const double *z, const int *type, const double *q)
+// up to this much goes through pinned memory: a 255-atom call is seven
+// pageable copies of 5-15 us otherwise; past it a pageable copy streams as
+// fast as the host can fill a pinned buffer
+constexpr size_t kPinnedIo = (size_t)4 << 20;
+
+int ensure_io_pin(akmc_batch_t b)
+{
+    if (!b->io_pin) HIPCHK(hipHostMalloc((void **)&b->io_pin, b->io_end, hipHostMallocDefault));
+    return AKMC_SUCCESS;
+}
+
+// wait: returns with the host arrays and the pinned buffer free for reuse (a
+// caller that synchronises the stream itself need not)
+int upload(akmc_batch_t b, const double *x, const double *y, const double *z, const int *type, const double *q,
+           bool wait = true)
 {
     size_t A = b->A;
     int ns = (int)b->f->species.size();
     for (size_t i = 0; i < A; ++i)
         if (type[i] < 0 || type[i] >= ns) return fail(AKMC_EINVAL, "atom %zu: species %d out of range", i, type[i]);
+    if (b->io_end <= kPinnedIo && !b->search_alloc) {
+        TRY(ensure_io_pin(b));
+        double *px = (double *)b->io_pin;
+        std::memcpy(px, x, A * sizeof(double));
+        std::memcpy(px + A, y, A * sizeof(double));
+        std::memcpy(px + 2 * A, z, A * sizeof(double));
+        int *pt = (int *)(px + 3 * A);
+        std::memcpy(pt, type, A * sizeof(int));
+        std::fill(pt + A, pt + A + b->W, 1);                           // fresh lists
+        std::fill(pt + A + b->W, pt + A + 2 * b->W, batch_mode(b));  // every walker is evaluated
+        if (q) std::memcpy(b->io_pin + b->io_q, q, A * sizeof(double));
+        HIPCHK(hipMemcpyAsync(b->io, b->io_pin, q ? b->io_in : b->io_q, hipMemcpyHostToDevice, b->stream));
+        if (wait) HIPCHK(hipStreamSynchronize(b->stream));
+        return AKMC_SUCCESS;
+    }
     HIPCHK(hipMemcpyAsync(b->d.x, x, A * sizeof(double), hipMemcpyHostToDevice, b->stream));
     HIPCHK(hipMemcpyAsync(b->d.y, y, A * sizeof(double), hipMemcpyHostToDevice, b->stream));
     HIPCHK(hipMemcpyAsync(b->d.z, z, A * sizeof(double), hipMemcpyHostToDevice, b->stream));
@@ -1591,13 +1666,21 @@ int akmc_field_forces(akmc_field_t f, double *x, double *y, double *z, double *f
     if (f->kind == 1 && f->do_ewald && !charge) return fail(AKMC_EINVAL, "ionic field needs charges");
     TRY(ensure_single(f, n, lat));
     akmc_batch_t b = f->single;
-    TRY(upload(b, x, y, z, type, charge));
+    TRY(upload(b, x, y, z, type, charge, false));
     TRY(run_forces(b, stress != nullptr));
-    TRY(check_overflow(b));
-    HIPCHK(hipMemcpyAsync(fx, b->d.fx, n * sizeof(double), hipMemcpyDeviceToHost, b->stream));
-    HIPCHK(hipMemcpyAsync(fy, b->d.fy, n * sizeof(double), hipMemcpyDeviceToHost, b->stream));
-    HIPCHK(hipMemcpyAsync(fz, b->d.fz, n * sizeof(double), hipMemcpyDeviceToHost, b->stream));
-    TRY(fetch_out(b));
+    if (b->io_pin) {
+        TRY(fetch_all(b));
+        const double *pf = (const double *)(b->io_pin + b->io_out);
+        std::memcpy(fx, pf, n * sizeof(double));
+        std::memcpy(fy, pf + n, n * sizeof(double));
+        std::memcpy(fz, pf + 2 * (size_t)n, n * sizeof(double));
+    } else {
+        TRY(check_overflow(b));
+        HIPCHK(hipMemcpyAsync(fx, b->d.fx, n * sizeof(double), hipMemcpyDeviceToHost, b->stream));
+        HIPCHK(hipMemcpyAsync(fy, b->d.fy, n * sizeof(double), hipMemcpyDeviceToHost, b->stream));
+        HIPCHK(hipMemcpyAsync(fz, b->d.fz, n * sizeof(double), hipMemcpyDeviceToHost, b->stream));
+        TRY(fetch_out(b));
+    }
     if (e) to_energy(b->hout[0], e);
     if (stress)
         for (int c = 0; c < 6; ++c) stress[c] = b->hout[0].stress[c];
@@ -1612,7 +1695,7 @@ int akmc_field_energy(akmc_field_t f, double *x, double *y, double *z, const dou
     if (f->kind == 1 && f->do_ewald && !charge) return fail(AKMC_EINVAL, "ionic field needs charges");
     TRY(ensure_single(f, n, lat));
     akmc_batch_t b = f->single;
-    TRY(upload(b, x, y, z, type, charge));
+    TRY(upload(b, x, y, z, type, charge, false));
     // this launch's own copy of the batch descriptor carries the energy-only
     // flag: no force pass, and the energy-only short-range forms of the
     // two-body table (TwoBody.h:81-150: Morse adds C12/r^12).  Tabulated EAM
@@ -1621,8 +1704,12 @@ int akmc_field_energy(akmc_field_t f, double *x, double *y, double *z, const dou
     d.energy_only = 1;
     akmc_launch_forces_impl(d, f->host, batch_mode(b), 0, b->stream);
     HIPCHK(hipGetLastError());
-    TRY(check_overflow(b));
-    TRY(fetch_out(b));
+    if (b->io_pin) {
+        TRY(fetch_all(b));
+    } else {
+        TRY(check_overflow(b));
+        TRY(fetch_out(b));
+    }
     if (e) to_energy(b->hout[0], e);
     host_wrap(f->min_image, lat, n, x, y, z);
     // the energy path of a tabulated EAM field doubles the pair term

@@ -1029,6 +1029,22 @@ __device__ __forceinline__ void sc_density_atom(const BatchDev &b, const FieldDe
             }
 #pragma unroll
             for (int u = 0; u < U; ++u) rho += double(in[u] ? c1.rho_coef * um[u] : T(0));  // + exact zeros
+        } else if (F.all96) {
+            // a table of n = 9, m = 6 pairs: straight products, branch-free
+#pragma unroll
+            for (int u = 0; u < U; ++u) {
+                const SCCoef<T> &c = sc_coef<T>(tab[row + (int)pj[u].w]);
+                T ir2, un, um;
+                table_9_6<T>(r2[u], c.a, ir2, un, um);
+                T rh = in[u] ? c.rho_coef * um : T(0);
+                if constexpr (sizeof(T) == 4) asm("" : "+v"(rh));
+                rho += double(rh);
+                if constexpr (ZONE) {
+                    T eh = in[u] ? T(0.5) * c.eps * un : T(0);
+                    if constexpr (sizeof(T) == 4) asm("" : "+v"(eh));
+                    ep += double(eh);
+                }
+            }
         } else {
 #pragma unroll
             for (int u = 0; u < U; ++u) {
@@ -1101,7 +1117,8 @@ __global__ void __launch_bounds__(STAGED ? AKMC_STAGE_BLOCK : kBlock) k_sc_densi
 // fm = 1/2 m (eps c)^2 (1/sqrt(rho_i) + 1/sqrt(rho_j)) (a/r)^m
 // (potentials/metal/Field.cpp:587-640, ManyBody.cpp:621-757); each atom
 // also carries half of each pair's V = eps (a/r)^n
-template <typename T, bool MINIMG, bool STRESS, int LPA, int U, bool ONE, bool STAGED>
+// (WL: search micro-steps, where pass 1 has written the pair energies)
+template <typename T, bool MINIMG, bool STRESS, int LPA, int U, bool ONE, bool STAGED, bool WL>
 __device__ __forceinline__ void sc_force_atom(const BatchDev &b, const FieldDev &F, const SCPairDev *tab,
                                               const SCCoef<T> &c1, const WalkerDev &W, const double4 *stage,
                                               int i, int sub)
@@ -1192,9 +1209,37 @@ __device__ __forceinline__ void sc_force_atom(const BatchDev &b, const FieldDev 
                 fx += dft * dx[u];
                 fy += dft * dy[u];
                 fz += dft * dz[u];
-                ep += double(eh);
+                if constexpr (!WL) ep += double(eh);
             }
             continue;
+        }
+        if constexpr (!ONE && !STRESS) {
+            if (F.all96) {
+                // a table of n = 9, m = 6 pairs: straight products, branch-free
+#pragma unroll
+                for (int u = 0; u < U; ++u) {
+                    const SCCoef<T> &c = sc_coef<T>(tab[row + (int)pj[u].w]);
+                    table_9_6<T>(r2[u], c.a, ir2[u], un[u], um[u]);
+                    const T fs = c.fs_coef * un[u];
+                    T fm;
+                    if constexpr (sizeof(T) == 8)
+                        fm = (isi64 >= 0.0 && isj64[u] >= 0.0) ? c.fm_coef * T(isi64 + isj64[u]) * um[u] : T(0);
+                    else
+                        fm = (isi >= 0.0f && isj[u] >= 0.0f) ? c.fm_coef * (T(isi) + T(isj[u])) * um[u] : T(0);
+                    T ft = in[u] ? (fs - fm) * ir2[u] : T(0);
+                    T eh = in[u] ? T(0.5) * c.eps * un[u] : T(0);
+                    if constexpr (sizeof(T) == 4) {
+                        asm("" : "+v"(ft));
+                        asm("" : "+v"(eh));
+                    }
+                    const double dft = double(ft);
+                    fx += dft * dx[u];
+                    fy += dft * dy[u];
+                    fz += dft * dz[u];
+                    if constexpr (!WL) ep += double(eh);
+                }
+                continue;
+            }
         }
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -1220,7 +1265,7 @@ __device__ __forceinline__ void sc_force_atom(const BatchDev &b, const FieldDev 
             fx += dft * dx[u];
             fy += dft * dy[u];
             fz += dft * dz[u];
-            ep += double(T(0.5) * c.eps * un[u]);
+            if constexpr (!WL) ep += double(T(0.5) * c.eps * un[u]);
             if (STRESS) {
                 double h = -0.5 * dft;  // one ordered pair: -(fs-fm)/(2 r^2) r r
                 s0 += h * dx[u] * dx[u];
@@ -1235,7 +1280,7 @@ __device__ __forceinline__ void sc_force_atom(const BatchDev &b, const FieldDev 
     fx = lane_group_sum<LPA>(fx);
     fy = lane_group_sum<LPA>(fy);
     fz = lane_group_sum<LPA>(fz);
-    ep = lane_group_sum<LPA>(ep);
+    if constexpr (!WL) ep = lane_group_sum<LPA>(ep);
     if (STRESS) {
         s0 = lane_group_sum<LPA>(s0);
         s1 = lane_group_sum<LPA>(s1);
@@ -1248,7 +1293,7 @@ __device__ __forceinline__ void sc_force_atom(const BatchDev &b, const FieldDev 
     b.fx[i] = fx;
     b.fy[i] = fy;
     b.fz[i] = fz;
-    if (!b.pe1) energy_b<T>(b)[i] = ep;  // search micro-steps: pass 1 wrote it
+    if constexpr (!WL) energy_b<T>(b)[i] = ep;
     if (STRESS) {
         b.st_atom[0 * (size_t)b.A + i] = s0;
         b.st_atom[1 * (size_t)b.A + i] = s1;
@@ -1287,7 +1332,7 @@ __global__ void __launch_bounds__(STAGED ? AKMC_STAGE_BLOCK : kBlock) k_sc_force
             }
             const int la = it.y + (int)threadIdx.x / LPA;
             if (la < n)
-                sc_force_atom<T, MINIMG, STRESS, LPA, U, ONE, STAGED>(b, F, tab, c1, W, stage,
+                sc_force_atom<T, MINIMG, STRESS, LPA, U, ONE, STAGED, WL>(b, F, tab, c1, W, stage,
                                                                        wl_atom<T>(b, W, it.x, la, 2),
                                                                        (int)threadIdx.x % LPA);
         }
@@ -1295,7 +1340,7 @@ __global__ void __launch_bounds__(STAGED ? AKMC_STAGE_BLOCK : kBlock) k_sc_force
     }
     const AtomSlot sl = sc_slot<T, LPA, STAGED>(b, W, stage, 2);
     if (!sl.ok) return;
-    sc_force_atom<T, MINIMG, STRESS, LPA, U, ONE, STAGED>(b, F, tab, c1, W, stage, sl.i, sl.sub);
+    sc_force_atom<T, MINIMG, STRESS, LPA, U, ONE, STAGED, WL>(b, F, tab, c1, W, stage, sl.i, sl.sub);
 }
 
 // energy-only pass 2 of Sutton-Chen (Field::calculateEnergy,
@@ -2043,6 +2088,28 @@ static void launch_sc_density_one(const BatchDev &b, const FieldDev &hf, hipStre
     else k_sc_density<T, false, LPA, U, ONE, STAGED, false><<<L.grid, L.block, L.lds, s>>>(b);
 }
 
+// a wavefront per atom (small cells behind the plain force call)
+constexpr int kWaveLanes = 64;
+template <typename T, bool ONE>
+static void launch_sc_density_wave(const BatchDev &b, const FieldDev &hf, hipStream_t s)
+{
+    const int g = xcd_grid((b.A * kWaveLanes + kBlock - 1) / kBlock);
+    if (hf.min_image) k_sc_density<T, true, kWaveLanes, 1, ONE, false, false><<<g, kBlock, 0, s>>>(b);
+    else k_sc_density<T, false, kWaveLanes, 1, ONE, false, false><<<g, kBlock, 0, s>>>(b);
+}
+template <typename T, bool ONE>
+static void launch_sc_force_wave(const BatchDev &b, const FieldDev &hf, int want_stress, hipStream_t s)
+{
+    const int g = xcd_grid((b.A * kWaveLanes + kBlock - 1) / kBlock);
+    if (hf.min_image) {
+        if (want_stress) k_sc_force<T, true, true, kWaveLanes, 1, ONE, false, false><<<g, kBlock, 0, s>>>(b);
+        else k_sc_force<T, true, false, kWaveLanes, 1, ONE, false, false><<<g, kBlock, 0, s>>>(b);
+    } else {
+        if (want_stress) k_sc_force<T, false, true, kWaveLanes, 1, ONE, false, false><<<g, kBlock, 0, s>>>(b);
+        else k_sc_force<T, false, false, kWaveLanes, 1, ONE, false, false><<<g, kBlock, 0, s>>>(b);
+    }
+}
+
 template <typename T, int LPA, int U>
 static void launch_sc_density(const BatchDev &b, const FieldDev &hf, hipStream_t s)
 {
@@ -2156,6 +2223,9 @@ static void launch_pass1(const BatchDev &b, const FieldDev &hf, int want_stress,
     int gA = xcd_grid(blocks(b.A));
     if (hf.kind == 0 && hf.eam) {
         launch_eam_density<T>(b, hf, s);
+    } else if (hf.kind == 0 && b.lpa == kWaveLanes) {
+        if (sc_one(hf)) launch_sc_density_wave<T, true>(b, hf, s);
+        else launch_sc_density_wave<T, false>(b, hf, s);
     } else if (hf.kind == 0) {
 #define AKMC_DENS(L_, U_) launch_sc_density<T, L_, U_>(b, hf, s)
         AKMC_SC_VARIANT(AKMC_DENS);
@@ -2185,6 +2255,11 @@ static BatchDev pass2_view(const BatchDev &b)
 template <typename T>
 static void launch_sc_force_variant(const BatchDev &b, const FieldDev &hf, int want_stress, hipStream_t s)
 {
+    if (b.lpa == kWaveLanes) {
+        if (sc_one(hf)) launch_sc_force_wave<T, true>(b, hf, want_stress, s);
+        else launch_sc_force_wave<T, false>(b, hf, want_stress, s);
+        return;
+    }
 #define AKMC_FORCE(L_, U_) launch_sc_force<T, L_, U_>(b, hf, want_stress, s)
     AKMC_SC_VARIANT(AKMC_FORCE);
 #undef AKMC_FORCE

@@ -175,8 +175,7 @@ extern "C" int akmc_field_forces_noalloc(akmc_field_t f, const double *x, const 
     d.maxnb = kMaxNb;
     d.ncells_total = ncells;
     d.G1 = 1;
-    d.lpa = 1;  // the default variant of a fresh batch, as akmc_field_forces runs
-    d.unroll = 1;
+    akmc_single_variant(n, d.lpa, d.unroll);  // as akmc_field_forces runs
     d.staged = 0;
     d.nb16 = (v.min_image && n <= 65535) ? 1 : 0;
     d.field = v.dev;

@@ -121,6 +121,37 @@ __device__ inline void pow_6(const T (&u2)[U], T (&u6)[U])
     for (int u = 0; u < U; ++u) u6[u] = u2[u] * (u2[u] * u2[u]);
 }
 
+// sqrt(x) to within half a unit in the last place or so: the hardware
+// estimate and one Newton step (the general kernels' table pairs take the
+// correctly rounded square root at twice the instructions)
+__device__ inline float root_refined(float x)
+{
+    const float y = __builtin_amdgcn_rsqf(x), r = x * y;
+    return __builtin_fmaf(__builtin_fmaf(-r, r, x), 0.5f * y, r);
+}
+
+// 1/r^2, (a/r)^9 and (a/r)^6 of a table pair: the products of pow_half's
+// repeated squaring, without its loops (a pair table whose exponents are 9
+// and 6 throughout)
+template <typename T>
+__device__ inline void table_9_6(double r2, T a, T &ir2, T &un, T &um)
+{
+    T u2, rt;
+    if constexpr (sizeof(T) == 8) {
+        const double ir = rsqrt_fp64(r2);
+        ir2 = ir * ir;
+        u2 = a * a * ir2;
+        rt = a * ir;
+    } else {
+        ir2 = recip<T>(T(r2));
+        u2 = a * a * ir2;
+        rt = root_refined(u2);
+    }
+    const T u4 = u2 * u2;
+    un = u4 * u4 * rt;
+    um = u2 * u4;
+}
+
 template <typename T>
 __device__ inline T pow_half(T u2, int k, T e)
 {

@@ -115,15 +115,6 @@ __device__ __forceinline__ double row_sum(double v)
 __device__ inline int slot_stride(int nz) { return (nz + 15) & ~15; }
 __device__ inline bool lists_fit(int entries, int S) { return entries <= 4 * (kLzLds - 4 * S); }
 
-// sqrt(x) to within half a unit in the last place or so: the hardware
-// estimate and one Newton step (the general kernels' table pairs take the
-// correctly rounded square root at twice the instructions)
-__device__ inline float root_refined(float x)
-{
-    const float y = __builtin_amdgcn_rsqf(x), r = x * y;
-    return __builtin_fmaf(__builtin_fmaf(-r, r, x), 0.5f * y, r);
-}
-
 // powers of U pairs: un = (a/r)^n, um = (a/r)^m, ir2 = 1/r^2.  KIND 1: one
 // species pair, n = 9, m = 6; 2: a pair table with n = 9, m = 6 throughout;
 // 0: any exponents (un = um = 0 for species pairs without a potential)
@@ -136,19 +127,8 @@ __device__ inline void pair_terms(const double (&r2)[U], const bool (&in)[U], co
         sc_powers_in<T, U>(r2, c1.a, ir2, u2, rt);
         pow_9_6<T, U>(u2, rt, un, um);
     } else if constexpr (KIND == 2) {
-        T u2[U], rt[U];
 #pragma unroll
-        for (int u = 0; u < U; ++u) {
-            const double r1[1] = {r2[u]};
-            T i1[1], v1[1], t1[1];
-            sc_powers_in<T, 1>(r1, sc_coef<T>(*p[u]).a, i1, v1, t1);
-            ir2[u] = i1[0];
-            u2[u] = v1[0];
-            rt[u] = sizeof(T) == 8 ? t1[0] : T(root_refined(float(v1[0])));
-            const T u4 = u2[u] * u2[u];
-            un[u] = u4 * u4 * rt[u];
-            um[u] = u2[u] * u4;
-        }
+        for (int u = 0; u < U; ++u) table_9_6<T>(r2[u], sc_coef<T>(*p[u]).a, ir2[u], un[u], um[u]);
     } else {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
