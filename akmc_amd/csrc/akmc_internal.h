@@ -333,6 +333,7 @@ struct WalkerState {
     // status, force calls and iterations of its relax
     double eb2, eb2_64, b2_maxd2;
     int b2_new, b2_status, b2_calls, b2_iters;
+    int fire_done;  // k_relax_fire advanced the walker on this micro-step
     int too_big;  // the walker does not fit the resident kernel's capacities
 };
 
@@ -360,7 +361,10 @@ struct SearchDev {
     double basin2_delta, basin_r2, max_r2;
     int basin2_on;
     int final64;                      // relaxes end with one FP64 energy evaluation
+    int fire_on;                      // k_relax_fire runs (the logic kernel leaves its walkers alone)
 };
+// atoms of a walker that k_relax_fire takes at most
+#define AKMC_FIRE_ATOMS 4096
 
 // after pass 1 of the chain: what frozen neighbours contribute to the
 // density and pair energy of every atom of the resident walkers it serves
@@ -380,12 +384,14 @@ void akmc_launch_leave_resident(const BatchDev &b, hipStream_t st);
 // 0 general pair table, 1 one species pair with n = 9, m = 6, 2 every
 // species pair present with n = 9, m = 6
 int akmc_sc_kind(const FieldDev &hf);
+// FIRE iterations of the walkers relaxing with every atom free
+void akmc_launch_relax_fire(const BatchDev &b, const SearchDev &s, hipStream_t st);
 void akmc_launch_search_logic(const BatchDev &b, const SearchDev &s, hipStream_t st);
 // the same state machines in 1024-thread workgroups (large walkers)
 void akmc_launch_search_logic_wide(const BatchDev &b, const SearchDev &s, hipStream_t st);
 // one walker start packed for akmc_launch_load_walkers: doubles at dbl
-// (mode [3][n], then positions [3][n] when has_x), ints at ints (frozen [n],
-// then the free-atom list [nact])
+// (mode of the free atoms [3][nact], then positions [3][n] when has_x), the
+// free-atom list [nact] at ints
 struct LoadItem {
     int walker, has_x, nact, pad;
     long long dbl, ints;

@@ -1076,6 +1076,25 @@ int upload(akmc_batch_t b, const double *x, const double *y, const double *z, co
 }
 
 
+// f(first atom, atoms) for each run of neighbouring selected walkers (all
+// when null): their slices lie together, so a run is one transfer (one per
+// walker took 30 ms for 512)
+template <typename F>
+int for_runs(akmc_batch_t b, const int *walkers, F f)
+{
+    for (int w = 0; w < b->W;) {
+        if (walkers && !walkers[w]) {
+            ++w;
+            continue;
+        }
+        const int off = b->hw[w].off;
+        int end = off;
+        for (; w < b->W && (!walkers || walkers[w]); ++w) end = b->hw[w].off + b->hw[w].n;
+        TRY(f((size_t)off, (size_t)(end - off)));
+    }
+    return AKMC_SUCCESS;
+}
+
 // rebuild the free-atom lists of the selected walkers (all when null) from
 // the host copy of the frozen mask and upload them
 int upload_active(akmc_batch_t b, const int *walkers)
@@ -1087,10 +1106,12 @@ int upload_active(akmc_batch_t b, const int *walkers)
         for (int i = 0; i < n; ++i)
             if (!b->hfrozen[off + i]) b->hact[off + m++] = off + i;
         b->hnact[w] = m;
-        if (m > 0)
-            HIPCHK(hipMemcpyAsync((void *)(b->s.act + off), b->hact.data() + off, m * sizeof(int),
-                                  hipMemcpyHostToDevice, b->stream));
     }
+    TRY(for_runs(b, walkers, [&](size_t off, size_t n) {
+        HIPCHK(hipMemcpyAsync((void *)(b->s.act + off), b->hact.data() + off, n * sizeof(int), hipMemcpyHostToDevice,
+                              b->stream));
+        return (int)AKMC_SUCCESS;
+    }));
     HIPCHK(hipMemcpyAsync((void *)b->s.nact, b->hnact.data(), b->W * sizeof(int), hipMemcpyHostToDevice, b->stream));
     HIPCHK(hipStreamSynchronize(b->stream));
     return AKMC_SUCCESS;
@@ -1326,6 +1347,10 @@ void enqueue_chain(akmc_batch_t b, const BatchDev &d, int res, int j)
 // 40 us); a search waits for it once, at the start of its FP64 verification.
 constexpr int kResidentSteps = 9;
 
+// some running walker relaxes by plain FIRE with every atom free and fits the
+// relax kernel (part of SearchDev, so that a captured graph is for one answer)
+bool relax_fire(akmc_batch_t b) { return b->s.fire_on != 0; }
+
 // the kernels of a chunk of micro-steps, res as resident_mode
 void enqueue_steps(akmc_batch_t b, int steps, int res)
 {
@@ -1333,6 +1358,7 @@ void enqueue_steps(akmc_batch_t b, int steps, int res)
     // walkers that need the chain take it on every step; with zones off the
     // chain evaluates every atom on every step, and a search still waits as
     // it does with zones on
+    const bool fire = relax_fire(b);
     const int runs = res == 2 && !b->ktimer ? (steps + kResidentSteps - 1) / kResidentSteps : steps;
     for (int j = 0, done = 0; j < runs; ++j) {
         const int k = (steps - done) / (runs - j), launches = b->zone_on ? 1 : k;
@@ -1342,6 +1368,7 @@ void enqueue_steps(akmc_batch_t b, int steps, int res)
                 akmc_launch_search_resident(b->W, b->f->host, b->res_args, k / launches, 1, l == 0, b->stream);
             // walkers of tens of thousands of atoms: 1024-thread state machines
             if (res < 2) {
+                if (fire) akmc_launch_relax_fire(d, b->s, b->stream);
                 if (b->logic_wide) akmc_launch_search_logic_wide(d, b->s, b->stream);
                 else akmc_launch_search_logic(d, b->s, b->stream);
             }
@@ -1472,12 +1499,20 @@ int load_walkers(akmc_batch_t b, const int *walkers, const double *x0, const dou
         if (walkers && !walkers[w]) continue;
         const int off = b->hw[w].off, n = b->hw[w].n;
         if (frozen) std::copy(frozen + off, frozen + off + n, b->hfrozen.begin() + off);
+        // the free-atom list (global ids)
+        const int *fr = b->hfrozen.data() + off;
+        int *act = b->hact.data() + off, m = 0;
+        for (int i = 0; i < n; ++i)
+            if (!fr[i]) act[m++] = off + i;
+        b->hnact[w] = m;
         LoadItem it{};
         it.walker = w;
+        it.has_x = x0 ? 1 : 0;
+        it.nact = m;
         it.dbl = (long long)dwords;
         it.ints = (long long)iwords;
-        dwords += (x0 ? 6 : 3) * (size_t)n;
-        iwords += 2 * (size_t)n;
+        dwords += 3 * (size_t)m + (x0 ? 3 * (size_t)n : 0);
+        iwords += m;
         items.push_back(it);
     }
     if (items.empty()) return AKMC_SUCCESS;
@@ -1487,35 +1522,24 @@ int load_walkers(akmc_batch_t b, const int *walkers, const double *x0, const dou
     char *base = (char *)b->stage_pin;
     double *D = (double *)(base + ibytes);
     int *I = (int *)(base + ibytes + dbytes);
-    for (LoadItem &it : items) {
-        const int w = it.walker, off = b->hw[w].off, n = b->hw[w].n;
-        const int *fr = b->hfrozen.data() + off;
+    for (const LoadItem &it : items) {
+        const int w = it.walker, off = b->hw[w].off, n = b->hw[w].n, m = it.nact;
+        const int *act = b->hact.data() + off;
         double *nw = D + it.dbl;
         double nn = 0.0;
         for (int c = 0; c < 3; ++c)
-            for (int i = 0; i < n; ++i) {
-                double v = fr[i] ? 0.0 : mode[c * A + off + i];
-                nw[(size_t)c * n + i] = v;
+            for (int k = 0; k < m; ++k) {
+                const double v = mode[c * A + act[k]];
+                nw[(size_t)c * m + k] = v;
                 nn += v * v;
             }
         if (nn <= 0.0) return fail(AKMC_EINVAL, "walker %d: zero start mode", w);
         nn = 1.0 / std::sqrt(nn);
-        for (size_t k = 0; k < 3 * (size_t)n; ++k) nw[k] *= nn;
-        it.has_x = x0 ? 1 : 0;
+        for (size_t k = 0; k < 3 * (size_t)m; ++k) nw[k] *= nn;
         if (x0)
-            for (int c = 0; c < 3; ++c) std::memcpy(nw + (size_t)(3 + c) * n, x0 + c * A + off, n * sizeof(double));
-        // frozen mask and free-atom list (global ids)
-        int *iw = I + it.ints;
-        int m = 0;
-        for (int i = 0; i < n; ++i) {
-            iw[i] = fr[i];
-            if (!fr[i]) {
-                iw[n + m++] = off + i;
-                b->hact[off + m - 1] = off + i;
-            }
-        }
-        it.nact = m;
-        b->hnact[w] = m;
+            for (int c = 0; c < 3; ++c)
+                std::memcpy(nw + 3 * (size_t)m + (size_t)c * n, x0 + c * A + off, n * sizeof(double));
+        std::memcpy(I + it.ints, act, m * sizeof(int));
     }
     std::memcpy(base, items.data(), ibytes);
     HIPCHK(hipMemcpyAsync(b->stage_dev, b->stage_pin, ibytes + dbytes + nbytes, hipMemcpyHostToDevice, b->stream));
@@ -1955,14 +1979,11 @@ int akmc_batch_start_relax(akmc_batch_t b, const int *walkers, const akmc_relax_
     r.N_maxUphill = p->N_maxUphill;
     r.initialDelay = p->initialDelay ? 1 : 0;
     // velocities start at zero
-    if (!walkers) {
-        HIPCHK(hipMemset(b->s.V, 0, 3 * (size_t)b->A * sizeof(double)));
-    } else {
-        for (int w = 0; w < b->W; ++w)
-            if (walkers[w])
-                for (int c = 0; c < 3; ++c)
-                    HIPCHK(hipMemset(b->s.V + (size_t)c * b->A + b->hw[w].off, 0, b->hw[w].n * sizeof(double)));
-    }
+    TRY(for_runs(b, walkers, [&](size_t off, size_t n) {
+        for (int c = 0; c < 3; ++c)
+            HIPCHK(hipMemsetAsync(b->s.V + (size_t)c * b->A + off, 0, n * sizeof(double), b->stream));
+        return (int)AKMC_SUCCESS;
+    }));
     return start_walkers(b, walkers, WK_RELAX, p->initTimeStep, p->alphaStart);
 }
 
@@ -2042,6 +2063,11 @@ int launch_chunk(akmc_batch_t b, int steps, int running)
     // HIP events recorded inside a replayed graph cannot be timed, so the
     // kernel timer launches the micro-steps one by one
     const int res = resident_mode(b);
+    b->s.fire_on = 0;
+    if (b->s.rp.method == AKMC_RELAX_FIRE && !b->s.rp.verlet)
+        for (int w = 0; w < b->W && !b->s.fire_on; ++w)
+            b->s.fire_on = b->hws[w].kind == WK_RELAX && b->hws[w].state != ST_DONE && b->hnact[w] == b->hw[w].n &&
+                           b->hw[w].n <= AKMC_FIRE_ATOMS;
     TRY(sync_res_args(b));
     if (b->use_graphs && !b->ktimer) {
         const BatchDev bd = step_dev(b);
@@ -2603,9 +2629,7 @@ int akmc_batch_start_relax_at(akmc_batch_t b, const int *walkers, const double *
     if (!b || !p) return fail(AKMC_EINVAL, "bad arguments");
     TRY(search_alloc(b));
     const size_t A = b->A;
-    for (int w = 0; w < b->W; ++w) {
-        if (walkers && !walkers[w]) continue;
-        const int off = b->hw[w].off, n = b->hw[w].n;
+    TRY(for_runs(b, walkers, [&](size_t off, size_t n) {
         if (frozen) {
             std::copy(frozen + off, frozen + off + n, b->hfrozen.begin() + off);
             HIPCHK(hipMemcpyAsync((void *)(b->s.frozen + off), frozen + off, n * sizeof(int), hipMemcpyHostToDevice,
@@ -2615,7 +2639,8 @@ int akmc_batch_start_relax_at(akmc_batch_t b, const int *walkers, const double *
             for (int c = 0; c < 3; ++c)
                 HIPCHK(hipMemcpyAsync(b->s.X + c * A + off, x0 + c * A + off, n * sizeof(double),
                                       hipMemcpyHostToDevice, b->stream));
-    }
+        return (int)AKMC_SUCCESS;
+    }));
     HIPCHK(hipStreamSynchronize(b->stream));
     if (frozen) TRY(upload_active(b, walkers));
     return akmc_batch_start_relax(b, walkers, p);
