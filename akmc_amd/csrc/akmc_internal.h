@@ -32,6 +32,9 @@
 #define AKMC_RES_SLOTS 2048
 #define AKMC_RES_ATOMS 16383
 #define AKMC_RES_CAND 4096
+// atoms of a walker that one workgroup bins into cells; larger ones are
+// binned in segments of 1024 atoms
+#define AKMC_BIN_ATOMS 8192
 // cells per axis are capped so a walker's grid fits one workgroup's LDS
 #define AKMC_MAX_CELLS_AXIS 16
 #define AKMC_MAX_WALKER_CELLS (AKMC_MAX_CELLS_AXIS * AKMC_MAX_CELLS_AXIS * AKMC_MAX_CELLS_AXIS)
@@ -179,6 +182,10 @@ struct BatchDev {
     int *overflow;        // sticky capacity flag
     int *cell_count, *cell_start, *cell_atoms;
     const int *cell_wk;   // cell -> walker
+    int nbin_seg, nbin_walker;  // segments and count of the walkers past AKMC_BIN_ATOMS
+    const int2 *bin_seg;        // segment -> (walker, first local atom)
+    const int4 *bin_walker;     // (walker, first segment, segments, 0)
+    int *bin_cnt, *bin_cell;    // [segments][MAX_WALKER_CELLS] counts, then first slots; [A] cells
     int *cell_work;       // cells whose lists are rebuilt this step (queued by k_cell_bin)
     int *cell_work_n;
     double *rho;          // SC density

@@ -855,6 +855,30 @@ int batch_build(akmc_field_t f, int W, const int *natoms, const double *lat, akm
             d.nchunk_tab[li] = (int)ch.size();
         }
     }
+    if (f->min_image) {
+        std::vector<int2> seg;
+        std::vector<int4> lw;
+        for (int w = 0; w < W; ++w) {
+            if (natoms[w] <= AKMC_BIN_ATOMS) continue;
+            const int s0 = (int)seg.size();
+            for (int a0 = 0; a0 < natoms[w]; a0 += 1024) seg.push_back(make_int2(w, a0));
+            lw.push_back(make_int4(w, s0, (int)seg.size() - s0, 0));
+        }
+        if (!seg.empty()) {
+            int2 *ds;
+            int4 *dw;
+            TRY(dalloc(b, &ds, seg.size()));
+            TRY(dalloc(b, &dw, lw.size()));
+            TRY(dalloc(b, &d.bin_cnt, seg.size() * AKMC_MAX_WALKER_CELLS));
+            TRY(dalloc(b, &d.bin_cell, A));
+            HIPCHK(hipMemcpy(ds, seg.data(), seg.size() * sizeof(int2), hipMemcpyHostToDevice));
+            HIPCHK(hipMemcpy(dw, lw.data(), lw.size() * sizeof(int4), hipMemcpyHostToDevice));
+            d.bin_seg = ds;
+            d.bin_walker = dw;
+            d.nbin_seg = (int)seg.size();
+            d.nbin_walker = (int)lw.size();
+        }
+    }
     {
         std::vector<int> hcw(ncells);
         for (int w = 0; w < W; ++w) {

@@ -175,7 +175,7 @@ __device__ inline int atom_cell_of(const BatchDev &b, const WalkerDev &W, int i)
 // cells of walkers up to kBinAtoms atoms stay in LDS between the counting
 // and the placement
 constexpr int kBinBlock = 1024;
-constexpr int kBinAtoms = 8192;
+constexpr int kBinAtoms = AKMC_BIN_ATOMS;
 
 // home atoms per list-build work item (k_nbr_build_cells)
 constexpr int kNbSlotsQ = 16;
@@ -207,6 +207,42 @@ __device__ inline int bin_scan(int v, int *wsum, int &total)
     return x + before;
 }
 
+// places kBinBlock consecutive atoms (thread t: atom first + t, its cell c,
+// -1 none) into their cells' next slots fill, in index order: each wavefront
+// finds, by ballots, the lanes of its 64 atoms that hold the same cell (rank
+// below, group size, highest lane); then one wavefront walks the groups of 64
+// in order: an atom's slot is the cell's fill plus its rank, and the highest
+// lane of each group advances the fill
+__device__ inline void bin_place(int c, int first, int *cell_atoms, int *fill, int *chunk, int *rank_, int *gsize)
+{
+    const int tid = threadIdx.x;
+    unsigned long long todo = __ballot(c >= 0);
+    unsigned long long same = 0;
+    while (todo) {
+        const int leader = __ffsll((long long)todo) - 1;
+        const int cl = __shfl(c, leader);
+        const unsigned long long grp = __ballot(c == cl);
+        if (c == cl) same = grp;
+        todo &= ~grp;
+    }
+    const int wl = tid & 63;
+    chunk[tid] = c;
+    rank_[tid] = __popcll(same & ((1ull << wl) - 1ull));
+    gsize[tid] = (c >= 0 && (same >> wl) == 1ull) ? __popcll(same) : 0;  // set on the group's highest lane
+    __syncthreads();
+    if (tid < 64) {
+        for (int wv = 0; wv < kBinBlock / 64; ++wv) {
+            const int k = wv * 64 + tid;
+            const int ck = chunk[k];
+            if (ck >= 0) {
+                cell_atoms[fill[ck] + rank_[k]] = first + k;
+                if (gsize[k]) fill[ck] += gsize[k];
+            }
+        }
+    }
+    __syncthreads();
+}
+
 __global__ void __launch_bounds__(kBinBlock) k_cell_bin(BatchDev b)
 {
     __shared__ int fill[AKMC_MAX_WALKER_CELLS];
@@ -216,6 +252,7 @@ __global__ void __launch_bounds__(kBinBlock) k_cell_bin(BatchDev b)
     const int w = blockIdx.x;
     if (!b.rebuild[w]) return;
     const WalkerDev W = b.walkers[w];
+    if (b.nbin_seg && W.n > kBinAtoms) return;  // k_bin_count, k_bin_scan, k_bin_place
     const int nc = W.nc[0] * W.nc[1] * W.nc[2];
     const int tid = threadIdx.x;
     for (int c = tid; c < nc; c += kBinBlock) fill[c] = 0;
@@ -253,39 +290,11 @@ __global__ void __launch_bounds__(kBinBlock) k_cell_bin(BatchDev b)
         carry += tot;
     }
     __syncthreads();
-    // stable placement in index order, kBinBlock atoms at a time: each
-    // wavefront finds, by ballots, the lanes of its 64 atoms that hold the
-    // same cell (rank below, group size, highest lane); then one wavefront
-    // walks the groups of 64 in order: an atom's slot is the cell's fill
-    // plus its rank, and the highest lane of each group advances the fill
+    // stable placement in index order, kBinBlock atoms at a time
     for (int base = 0; base < W.n; base += kBinBlock) {
         const int l = base + tid;
         const int c = l < W.n ? (keep ? acell[l] : atom_cell_of(b, W, W.off + l)) : -1;
-        unsigned long long todo = __ballot(c >= 0);
-        unsigned long long same = 0;
-        while (todo) {
-            const int leader = __ffsll((long long)todo) - 1;
-            const int cl = __shfl(c, leader);
-            const unsigned long long grp = __ballot(c == cl);
-            if (c == cl) same = grp;
-            todo &= ~grp;
-        }
-        const int wl = tid & 63;
-        chunk[tid] = c;
-        rank_[tid] = __popcll(same & ((1ull << wl) - 1ull));
-        gsize[tid] = (c >= 0 && (same >> wl) == 1ull) ? __popcll(same) : 0;  // set on the group's highest lane
-        __syncthreads();
-        if (tid < 64) {
-            for (int wv = 0; wv < kBinBlock / 64; ++wv) {
-                const int k = wv * 64 + tid;
-                const int ck = chunk[k];
-                if (ck >= 0) {
-                    b.cell_atoms[fill[ck] + rank_[k]] = W.off + base + k;
-                    if (gsize[k]) fill[ck] += gsize[k];
-                }
-            }
-        }
-        __syncthreads();
+        bin_place(c, W.off + base, b.cell_atoms, fill, chunk, rank_, gsize);
     }
     // queue this walker's list-build items: home chunks of kNbSlots atoms per
     // cell (chunk indices above 255 are served by the item of chunk % 256),
@@ -317,6 +326,109 @@ __global__ void __launch_bounds__(kBinBlock) k_cell_bin(BatchDev b)
         }
         carry += tot;
     }
+}
+
+// k_cell_bin for walkers past kBinAtoms, whose one workgroup would place
+// 1024 atoms at a time (134 us for 31,980 atoms): a workgroup per segment of
+// kBinBlock atoms counts its cells, one per walker turns the counts into each
+// segment's first slot per cell, and a workgroup per segment places its atoms
+// in index order (26 us together).
+__global__ void __launch_bounds__(kBinBlock) k_bin_count(BatchDev b)
+{
+    __shared__ int hist[AKMC_MAX_WALKER_CELLS];
+    const int2 sg = b.bin_seg[blockIdx.x];
+    const int w = sg.x, tid = threadIdx.x;
+    if (!b.rebuild[w]) return;
+    const WalkerDev W = b.walkers[w];
+    const int nc = W.nc[0] * W.nc[1] * W.nc[2];
+    for (int c = tid; c < nc; c += kBinBlock) hist[c] = 0;
+    __syncthreads();
+    const int l = sg.y + tid;
+    if (l < W.n) {
+        const int i = W.off + l;
+        const double x = b.x[i], y = b.y[i], z = b.z[i];
+        b.xr[i] = x;
+        b.yr[i] = y;
+        b.zr[i] = z;
+        if (b.zflag && (b.zflag[w] & (AKMC_ZONE_RESET | AKMC_ZONE_RES)) == AKMC_ZONE_RESET) b.zmark[i] = 0;
+        const int cell = (cell_coord(x, W.invL[0], W.nc[0]) * W.nc[1] + cell_coord(y, W.invL[1], W.nc[1])) * W.nc[2] +
+                         cell_coord(z, W.invL[2], W.nc[2]);
+        b.bin_cell[i] = cell;
+        atomicAdd(&hist[cell], 1);
+    }
+    __syncthreads();
+    int *out = b.bin_cnt + (size_t)blockIdx.x * AKMC_MAX_WALKER_CELLS;
+    for (int c = tid; c < nc; c += kBinBlock) out[c] = hist[c];
+}
+
+__global__ void __launch_bounds__(kBinBlock) k_bin_scan(BatchDev b)
+{
+    __shared__ int wsum[kBinBlock / 64];
+    __shared__ int qbase;
+    const int4 lw = b.bin_walker[blockIdx.x];  // walker, first segment, segments
+    const int w = lw.x, tid = threadIdx.x;
+    if (!b.rebuild[w]) return;
+    const WalkerDev W = b.walkers[w];
+    const int nc = W.nc[0] * W.nc[1] * W.nc[2];
+    int *cnt = b.bin_cnt + (size_t)lw.y * AKMC_MAX_WALKER_CELLS;
+    auto items_of = [](int n) {
+        const int k = (n + kNbSlotsQ - 1) / kNbSlotsQ;
+        return k < 256 ? k : 256;
+    };
+    int carry = W.off, mine = 0;
+    for (int base = 0; base < nc; base += kBinBlock) {
+        const int c = base + tid;
+        int v = 0;
+        if (c < nc)
+            for (int s = 0; s < lw.z; ++s) v += cnt[(size_t)s * AKMC_MAX_WALKER_CELLS + c];
+        int tot;
+        const int incl = bin_scan(v, wsum, tot);
+        if (c < nc) {
+            int at = carry + incl - v;
+            b.cell_count[W.cell_off + c] = v;
+            b.cell_start[W.cell_off + c] = at;
+            for (int s = 0; s < lw.z; ++s) {
+                const size_t o = (size_t)s * AKMC_MAX_WALKER_CELLS + c;
+                const int k = cnt[o];
+                cnt[o] = at;
+                at += k;
+            }
+            mine += items_of(v);
+        }
+        carry += tot;
+    }
+    // the walker's list-build items, as k_cell_bin queues them
+    int items;
+    (void)bin_scan(mine, wsum, items);
+    if (tid == 0) qbase = atomicAdd(b.cell_work_n, items);
+    __syncthreads();
+    carry = 0;
+    for (int base = 0; base < nc; base += kBinBlock) {
+        const int c = base + tid;
+        const int v = c < nc ? items_of(b.cell_count[W.cell_off + c]) : 0;
+        int tot;
+        const int incl = bin_scan(v, wsum, tot);
+        if (c < nc) {
+            const int at = qbase + carry + incl - v;
+            for (int ch = 0; ch < v; ++ch) b.cell_work[at + ch] = ((W.cell_off + c) << 8) | ch;
+        }
+        carry += tot;
+    }
+}
+
+__global__ void __launch_bounds__(kBinBlock) k_bin_place(BatchDev b)
+{
+    __shared__ int fill[AKMC_MAX_WALKER_CELLS];
+    __shared__ int chunk[kBinBlock], rank_[kBinBlock], gsize[kBinBlock];
+    const int2 sg = b.bin_seg[blockIdx.x];
+    const int w = sg.x, tid = threadIdx.x;
+    if (!b.rebuild[w]) return;
+    const WalkerDev W = b.walkers[w];
+    const int nc = W.nc[0] * W.nc[1] * W.nc[2];
+    const int *first = b.bin_cnt + (size_t)blockIdx.x * AKMC_MAX_WALKER_CELLS;
+    for (int c = tid; c < nc; c += kBinBlock) fill[c] = first[c];
+    const int l = sg.y + tid;
+    bin_place(l < W.n ? b.bin_cell[W.off + l] : -1, W.off + sg.y, b.cell_atoms, fill, chunk, rank_, gsize);
 }
 
 // The entry after atom i's list (row n <= maxnb; the buffer holds
@@ -648,45 +760,125 @@ __device__ inline void image_hits(const BatchDev &b, const WalkerDev &W, int i, 
     }
 }
 
+// the same over one shell of images per axis, as bit masks of the 27 images
+// in (sa, sb, sc) order: near (inside the near shell) and rest; an image past
+// the entry's range is reported and not counted
+__device__ inline void image_masks(const BatchDev &b, const WalkerDev &W, int i, int jl, double xi, double yi, double zi,
+                                   double rl2, double rn2, uint32_t &near, uint32_t &rest, int (&m)[3])
+{
+    const int j = W.off + jl;
+    const double bx = xi - b.x[j], by = yi - b.y[j], bz = zi - b.z[j];
+    m[0] = (int)rint(bx * W.invL[0]);
+    m[1] = (int)rint(by * W.invL[1]);
+    m[2] = (int)rint(bz * W.invL[2]);
+    near = rest = 0u;
+#pragma unroll
+    for (int k = 0; k < 27; ++k) {
+        const int sa = m[0] + k / 9 - 1, sb = m[1] + k / 3 % 3 - 1, sc = m[2] + k % 3 - 1;
+        const double dx = bx - sa * W.L[0], dy = by - sb * W.L[1], dz = bz - sc * W.L[2];
+        const double r2 = dx * dx + dy * dy + dz * dz;
+        if (r2 <= rl2 && !(j == i && sa == 0 && sb == 0 && sc == 0)) {
+            if (sa < -7 || sa > 7 || sb < -7 || sb > 7 || sc < -7 || sc > 7) {
+                *b.overflow = 1;
+            } else if (r2 <= rn2) {
+                near |= 1u << k;
+            } else {
+                rest |= 1u << k;
+            }
+        }
+    }
+    if (!(rn2 > 0.0)) near = 0u;
+}
+
 // Explicit-image list of a rebuilding walker (no-image fields, rc > L/2):
-// one wavefront per atom.  Candidates are taken 64 at a time, one per
-// lane; each lane counts its hits, a wavefront prefix sum gives every lane
-// its first slot, and the lanes write their entries there.  The list holds
-// the near-shell entries first, then the rest, each in (j, image)
-// ascending order -- the order of a serial scan, so the list does not
-// depend on scheduling.
+// one workgroup per atom, each wavefront a quarter of the candidates, 64 at a
+// time, one per lane.  A first sweep counts the wavefronts' near-shell and
+// other hits, the second writes them from the offsets that follow: the
+// near-shell entries first, then the rest, each in (j, image) ascending
+// order, the order of a serial scan, so the list does not depend on
+// scheduling.  Bound by the FP64 distances to 27 images: the 510-ion cell
+// takes 14 us (116 us with one wavefront per atom, whose near and other
+// entries were separate passes, each evaluating every image twice).
 __global__ void __launch_bounds__(kBlock) k_nbr_build_images(BatchDev b)
 {
-    constexpr int kAtomsPerBlock = kBlock / 64;
-    const int nblk = (b.A + kAtomsPerBlock - 1) / kAtomsPerBlock;
-    const int i = blockIdx.x * kAtomsPerBlock + int(threadIdx.x) / 64, lane = int(threadIdx.x) % 64;
-    if (blockIdx.x >= nblk || i >= b.A) return;  // whole wavefronts leave together
+    constexpr int kWaves = kBlock / 64;
+    __shared__ int tot[2][kWaves];
+    const int i = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int w = walker_of(b, i);
     if (!b.rebuild[w]) return;
     const WalkerDev W = b.walkers[w];
     const double rl2 = b.field->rlist2, rn2 = b.field->rnear2;
     const double xi = b.x[i], yi = b.y[i], zi = b.z[i];
-    int cnt = 0, nnear = 0;
-    for (int pass = (rn2 > 0.0 ? 0 : 1); pass < 2; ++pass) {
-        for (int jb = 0; jb < W.n; jb += 64) {
-            const int jl = jb + lane;
-            int c = 0;
-            if (jl < W.n) image_hits(b, W, i, jl, xi, yi, zi, rl2, rn2, pass, [&](uint32_t) { ++c; });
-            int incl = c;
-            for (int o = 1; o < 64; o <<= 1) {
-                const int t = __shfl_up(incl, o);
-                if (lane >= o) incl += t;
+    const bool one = W.shells[0] == 1 && W.shells[1] == 1 && W.shells[2] == 1;
+    const int nchunk = (W.n + 63) / 64;
+    const int c0 = wave * nchunk / kWaves, c1 = (wave + 1) * nchunk / kWaves;
+    int at[2] = {0, 0};
+#pragma unroll 1  // one copy of the distances: both sweeps see the same hits
+    for (int sweep = 0; sweep < 2; ++sweep) {
+        int sum[2] = {0, 0};
+        for (int ch = c0; ch < c1; ++ch) {
+            const int jl = 64 * ch + lane;
+            uint32_t hit[2] = {0u, 0u};
+            int m[3] = {0, 0, 0}, cnt[2] = {0, 0};
+            if (jl < W.n) {
+                if (one) {
+                    image_masks(b, W, i, jl, xi, yi, zi, rl2, rn2, hit[0], hit[1], m);
+                    cnt[0] = __popc(hit[0]);
+                    cnt[1] = __popc(hit[1]);
+                } else {
+                    for (int p = 0; p < 2; ++p) {
+                        if (p == 0 && !(rn2 > 0.0)) continue;
+                        image_hits(b, W, i, jl, xi, yi, zi, rl2, rn2, p, [&](uint32_t) { ++cnt[p]; });
+                    }
+                }
             }
-            int slot = cnt + incl - c;
-            if (c > 0) image_hits(b, W, i, jl, xi, yi, zi, rl2, rn2, pass, [&](uint32_t e) { put_nbr(b, i, slot++, e); });
-            cnt += __shfl(incl, 63);
+            if (sweep == 0) {
+                sum[0] += cnt[0];
+                sum[1] += cnt[1];
+                continue;
+            }
+            for (int p = 0; p < 2; ++p) {
+                int incl = cnt[p];
+                for (int o = 1; o < 64; o <<= 1) {
+                    const int t = __shfl_up(incl, o);
+                    if (lane >= o) incl += t;
+                }
+                int slot = at[p] + incl - cnt[p];
+                at[p] += __shfl(incl, 63);
+                if (cnt[p] == 0) continue;
+                if (one) {
+                    for (uint32_t h = hit[p]; h; h &= h - 1u) {
+                        const int k = __ffs((int)h) - 1;
+                        const int sa = m[0] + k / 9 - 1, sb = m[1] + k / 3 % 3 - 1, sc = m[2] + k % 3 - 1;
+                        put_nbr(b, i, slot++, uint32_t(jl) | (uint32_t(sa + 7) << 20) | (uint32_t(sb + 7) << 24) |
+                                                  (uint32_t(sc + 7) << 28));
+                    }
+                } else {
+                    image_hits(b, W, i, jl, xi, yi, zi, rl2, rn2, p, [&](uint32_t e) { put_nbr(b, i, slot++, e); });
+                }
+            }
         }
-        if (pass == 0) nnear = cnt;
+        if (sweep == 0) {
+            for (int p = 0; p < 2; ++p) {
+                for (int o = 32; o > 0; o >>= 1) sum[p] += __shfl_xor(sum[p], o);
+                if (lane == 0) tot[p][wave] = sum[p];
+            }
+            __syncthreads();
+            int near = 0;
+            for (int v = 0; v < kWaves; ++v) {
+                near += tot[0][v];
+                if (v < wave) {
+                    at[0] += tot[0][v];
+                    at[1] += tot[1][v];
+                }
+            }
+            at[1] += near;
+        }
     }
-    if (lane != 0) return;
-    const int n = cnt < b.maxnb ? cnt : b.maxnb;
+    if (threadIdx.x != kBlock - 1) return;  // the last wavefront's offsets are the ends
+    const int n = at[1] < b.maxnb ? at[1] : b.maxnb, nn = at[0];
     b.nnb[i] = n;
-    b.nnear[i] = nnear < b.maxnb ? nnear : b.maxnb;
+    b.nnear[i] = nn < b.maxnb ? nn : b.maxnb;
     put_sentinel(b, i, n, W.off);
 }
 
@@ -2038,10 +2230,15 @@ static void launch_lists(const BatchDev &b, const FieldDev &hf, hipStream_t s)
     else k_pack_check<<<gA, kBlock, 0, s>>>(b);
     if (hf.min_image) {
         k_cell_bin<<<b.W, kBinBlock, 0, s>>>(b);  // records the reference positions too
+        if (b.nbin_seg) {
+            k_bin_count<<<b.nbin_seg, kBinBlock, 0, s>>>(b);
+            k_bin_scan<<<b.nbin_walker, kBinBlock, 0, s>>>(b);
+            k_bin_place<<<b.nbin_seg, kBinBlock, 0, s>>>(b);
+        }
         k_nbr_build_cells<<<kNbGrid, kBlock, 0, s>>>(b);
     } else {
         k_ref_positions<<<gA, kBlock, 0, s>>>(b);
-        k_nbr_build_images<<<(b.A + kBlock / 64 - 1) / (kBlock / 64), kBlock, 0, s>>>(b);
+        k_nbr_build_images<<<b.A, kBlock, 0, s>>>(b);
     }
     // the zones of search micro-steps, with the rebuild bookkeeping
     if (b.zflag) k_zone_build<<<b.W, kBlock, 0, s>>>(b, b.rebuild_count);
