@@ -156,7 +156,7 @@ struct ResidentDev {
 };
 
 struct BatchDev {
-    int A, W, maxnb, ncells_total, nk_total, G1, maxnk;
+    int A, W, maxnb, ncells_total, nk_total, G1, maxnk, maxn;  // maxn: atoms of the largest walker
     int lpa;              // lanes per atom of the Sutton-Chen pair kernels (1, 2, 4, 8; 64: small cells)
     int nb16;             // list entries are 16-bit local indices (minimum-image
                           // many-body lists of walkers below 65536 atoms)

@@ -489,8 +489,9 @@ void build_tables(akmc_field_t f)
 // atoms behind the plain force call.  Below two wavefronts per SIMD at 8
 // lanes (16,384 atoms) a wavefront per atom: 255 atoms 65 + 56 us at one lane,
 // 7 + 6 us so; above, 8 lanes: 31,980 alloy atoms 114 + 153 us at one lane
-// with the general powers, 20 + 23 us so with the table's straight products.  A batch keeps one size-independent default, so that a
-// walker gives the same bits alone and among others.
+// with the general powers, 20 + 23 us so with the table's straight products.
+// A batch keeps one size-independent default, so that a walker gives the same
+// bits alone and among others.
 }  // namespace
 void akmc_single_variant(int n, int &lpa, int &unroll)
 {
@@ -734,7 +735,7 @@ int batch_build(akmc_field_t f, int W, const int *natoms, const double *lat, akm
     d.A = A;
     d.W = W;
     d.maxnb = maxnb;
-    d.lpa = 4;  // one default for every batch size (512 walkers: 0.72 ms an evaluation, 1.00 ms at 1 x 1)
+    d.lpa = 4;  // one default for every batch size (512 walkers, unstaged: 1.13 ms an evaluation, 1.80 at 1 x 1)
     d.unroll = 4;
     {
         int nmax = 0;
@@ -750,6 +751,7 @@ int batch_build(akmc_field_t f, int W, const int *natoms, const double *lat, akm
     d.nk_total = nk;
     d.G1 = G1;
     d.maxnk = maxnk;
+    d.maxn = *std::max_element(natoms, natoms + W);
     HIPCHK(hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking));
     HIPCHK(hipEventCreate(&b->ev0));
     HIPCHK(hipEventCreate(&b->ev1));

@@ -1988,39 +1988,45 @@ __device__ inline double2 phase_of(const double2 *t, int G1, int nx, int ny, int
 }
 
 // C_k = sum_i q_i cos(k.r_i), S_k = sum_i q_i sin(k.r_i) (Ewald.cpp:596-611).
-// One 1024-thread workgroup per (tile of 64 k vectors, walker): lane l of
-// every wavefront owns k = 64 tile + l, wavefront v sums the atoms
-// v, v + 16, ... of the walker, and the 16 wavefront partials are added in
-// wavefront order through LDS (FP64 throughout; a fixed order, so the sums
-// do not depend on the batch).  The per-k products g0 C and g0 S of the
-// force pass are written with them.
-constexpr int kSkWaves = AKMC_STAGE_BLOCK / 64;
+// One 512-thread workgroup per (tile of 32 k vectors, walker): lane l of
+// every wavefront owns k = 32 tile + l % 32, half-wavefront h sums the atoms
+// h, h + 16, ... of the walker; the two halves meet by a shuffle and the 8
+// wavefronts' sums are added in wavefront order through LDS (FP64 throughout;
+// a fixed order, so the sums do not depend on the batch).  Bound by the table
+// gathers and their latency: 16 walkers of 510 ions, 1147 k, 26 us and one
+// 18; 33 and 19 with 1024 threads on 64 k, 29 and 13 with 1024 on 32 (the
+// batch decides: searches are where the path is used).
+constexpr int kSkBlock = 512, kSkWaves = kSkBlock / 64, kSkTile = 32;
 
-__global__ void __launch_bounds__(AKMC_STAGE_BLOCK) k_ewald_sk(BatchDev b)
+__global__ void __launch_bounds__(kSkBlock) k_ewald_sk(BatchDev b)
 {
-    __shared__ double part[2][kSkWaves][64];
+    __shared__ double part[2][kSkWaves][kSkTile];
     const int w = blockIdx.y;
     if (skipped(b, w)) return;
     const WalkerDev W = b.walkers[w];
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    const int k = blockIdx.x * 64 + lane;
-    if (blockIdx.x * 64 >= W.nk) return;
+    const int lane = threadIdx.x % kSkTile, half = threadIdx.x / kSkTile, wave = threadIdx.x >> 6;
+    const int k = blockIdx.x * kSkTile + lane;
+    if (blockIdx.x * kSkTile >= W.nk) return;
     const bool has = k < W.nk;
     const int kk = W.k_off + (has ? k : 0);
     const int nx = b.kn[kk], ny = b.kn[b.nk_total + kk], nz = b.kn[2 * b.nk_total + kk];
     double C = 0.0, S = 0.0;
-    if (has) {
-        for (int i = W.off + wave; i < W.off + W.n; i += kSkWaves) {
-            const double2 p = phase_of(b.ptab + (size_t)i * 3 * b.G1, b.G1, nx, ny, nz);
-            const double q = b.q[i];
-            C += q * p.x;
-            S += q * p.y;
-        }
+#pragma unroll 4
+    for (int l = half; l < W.n; l += 2 * kSkWaves) {
+        const size_t i = W.off + l;
+        const double2 p = phase_of(b.ptab + i * 3 * b.G1, b.G1, nx, ny, nz);
+        const double q = b.q[i];
+        C += q * p.x;
+        S += q * p.y;
     }
-    part[0][wave][lane] = C;
-    part[1][wave][lane] = S;
+    C += __shfl_xor(C, kSkTile);
+    S += __shfl_xor(S, kSkTile);
+    if ((threadIdx.x & 63) < kSkTile) {
+        part[0][wave][lane] = C;
+        part[1][wave][lane] = S;
+    }
     __syncthreads();
-    if (wave == 0 && has) {
+    if (half == 0 && has) {
         double Ct = part[0][0][lane], St = part[1][0][lane];
         for (int v = 1; v < kSkWaves; ++v) {
             Ct += part[0][v][lane];
@@ -2032,43 +2038,89 @@ __global__ void __launch_bounds__(AKMC_STAGE_BLOCK) k_ewald_sk(BatchDev b)
 }
 
 // F_i += -g0 (-q sin C + q cos S) k;  E_i = 1/2 sum_k g0 q (cos C + sin S)
-// (Ewald.cpp:636-646).  One wavefront per atom, its lanes over the walker's
-// k vectors (k = lane, lane + 64, ...: every load of k data is one coalesced
-// 64-wide read), lane sums by shuffles.
+// (Ewald.cpp:636-646).  One workgroup per kEwAtoms atoms of a walker, its
+// threads over the walker's k vectors (each load of k data is one coalesced
+// read, used for all the atoms); the atoms' tables are staged in LDS where
+// they fit (STAGED: G1 <= kEwG).  The 16 lane sums meet in one transposing
+// butterfly (each exchange halves the values a lane holds), then the
+// wavefronts' in order.  Bound by FP64 issue and the table gathers: 16
+// walkers of 510 ions, 1147 k, take 19 us and one 11; 46 and 12 with a
+// wavefront per atom, which reads the k data four times as often and the
+// tables from global memory.
+constexpr int kEwAtoms = 4, kEwG = 64;
+
+// one stage of the butterfly: of 2 H values each lane keeps H, the upper ones
+// where its bit o is set, and adds its partner's
+template <int H>
+__device__ inline void halve(double (&v)[4 * kEwAtoms], int lane, int o)
+{
+    const bool up = lane & o;
+#pragma unroll
+    for (int c = 0; c < H; ++c) {
+        const double give = up ? v[c] : v[c + H], keep = up ? v[c + H] : v[c];
+        v[c] = keep + __shfl_xor(give, o);
+    }
+}
+
+template <bool STAGED>
 __global__ void __launch_bounds__(kBlock) k_ewald_force(BatchDev b)
 {
-    const int nblk = (b.A + kIonAtomsPerBlock - 1) / kIonAtomsPerBlock;
-    const int per = (nblk + kXCD - 1) / kXCD;
-    const int blk = (blockIdx.x % kXCD) * per + blockIdx.x / kXCD;
-    const int i = blk * kIonAtomsPerBlock + int(threadIdx.x) / kIonLanes, sub = int(threadIdx.x) % kIonLanes;
-    if (blk >= nblk || i >= b.A) return;
-    if (skipped(b, walker_of(b, i))) return;
-    const WalkerDev W = b.walkers[walker_of(b, i)];
-    const double2 *t = b.ptab + (size_t)i * 3 * b.G1;
-    const double q = b.q[i];
+    __shared__ double2 tab[STAGED ? kEwAtoms * 3 * kEwG : 1];
+    __shared__ double part[kBlock / 64][4 * kEwAtoms];
+    const int w = blockIdx.y, l0 = blockIdx.x * kEwAtoms;
+    if (skipped(b, w)) return;
+    const WalkerDev W = b.walkers[w];
+    if (l0 >= W.n) return;
+    const int na = W.n - l0 < kEwAtoms ? W.n - l0 : kEwAtoms, i0 = W.off + l0, G3 = 3 * b.G1;
+    const double2 *src = b.ptab + (size_t)i0 * G3;
+    if (STAGED) {
+        for (int t = threadIdx.x; t < na * G3; t += kBlock) tab[t] = src[t];
+        __syncthreads();
+    }
+    const double2 *t[kEwAtoms];
+    double q[kEwAtoms], v[4 * kEwAtoms];
+    for (int a = 0; a < kEwAtoms; ++a) {  // past the walker's last atom: its first with no charge
+        t[a] = (STAGED ? tab : src) + (a < na ? a * G3 : 0);
+        q[a] = a < na ? b.q[i0 + a] : 0.0;
+    }
+#pragma unroll
+    for (int c = 0; c < 4 * kEwAtoms; ++c) v[c] = 0.0;
     const int nk = b.nk_total;
-    double fx = 0.0, fy = 0.0, fz = 0.0, e = 0.0;
-    for (int k = sub; k < W.nk; k += kIonLanes) {
+    for (int k = threadIdx.x; k < W.nk; k += kBlock) {
         const int kk = W.k_off + k;
-        const double2 p = phase_of(t, b.G1, b.kn[kk], b.kn[nk + kk], b.kn[2 * nk + kk]);
+        const int nx = b.kn[kk], ny = b.kn[nk + kk], nz = b.kn[2 * nk + kk];
         const double g0 = b.g0[kk];
         const double gC = g0 * b.Ck[kk], gS = g0 * b.Sk[kk];
-        const double cs = q * p.x, sn = q * p.y;
-        const double pf = -(-sn * gC + cs * gS);
-        fx += pf * b.kv[kk];
-        fy += pf * b.kv[nk + kk];
-        fz += pf * b.kv[2 * nk + kk];
-        e += cs * gC + sn * gS;
+        const double kx = b.kv[kk], ky = b.kv[nk + kk], kz = b.kv[2 * nk + kk];
+#pragma unroll
+        for (int a = 0; a < kEwAtoms; ++a) {
+            const double2 p = phase_of(t[a], b.G1, nx, ny, nz);
+            const double cs = q[a] * p.x, sn = q[a] * p.y;
+            const double pf = -(-sn * gC + cs * gS);
+            v[4 * a] += pf * kx;
+            v[4 * a + 1] += pf * ky;
+            v[4 * a + 2] += pf * kz;
+            v[4 * a + 3] += cs * gC + sn * gS;
+        }
     }
-    fx = lane_group_sum<kIonLanes>(fx);
-    fy = lane_group_sum<kIonLanes>(fy);
-    fz = lane_group_sum<kIonLanes>(fz);
-    e = lane_group_sum<kIonLanes>(e);
-    if (sub != 0) return;
-    b.fx[i] += fx;
-    b.fy[i] += fy;
-    b.fz[i] += fz;
-    b.e_c[i] = 0.5 * e;
+    const int lane = threadIdx.x & 63;
+    halve<8>(v, lane, 32);
+    halve<4>(v, lane, 16);
+    halve<2>(v, lane, 8);
+    halve<1>(v, lane, 4);
+    const int mine = lane >> 2;  // the sum this lane ends up with
+    v[0] += __shfl_xor(v[0], 2);
+    v[0] += __shfl_xor(v[0], 1);
+    if ((lane & 3) == 0) part[threadIdx.x >> 6][mine] = v[0];
+    __syncthreads();
+    const int c = threadIdx.x, i = i0 + c / 4;
+    if (c >= 4 * na) return;
+    double sum = part[0][c];
+    for (int u = 1; u < kBlock / 64; ++u) sum += part[u][c];
+    if (c % 4 == 0) b.fx[i] += sum;
+    else if (c % 4 == 1) b.fy[i] += sum;
+    else if (c % 4 == 2) b.fz[i] += sum;
+    else b.e_c[i] = 0.5 * sum;
 }
 
 // ----------------------------------------------------- walker reductions
@@ -2475,8 +2527,8 @@ static void launch_pass2(const BatchDev &b, const FieldDev &hf, int want_stress,
         // the reciprocal energy needs the structure factors only
         if (hf.do_ewald == 1) {
             k_ewald_tables<<<gA, kBlock, 0, s>>>(b);
-            dim3 g((b.maxnk + 63) / 64, b.W);
-            k_ewald_sk<<<g, AKMC_STAGE_BLOCK, 0, s>>>(b);
+            dim3 g((b.maxnk + kSkTile - 1) / kSkTile, b.W);
+            k_ewald_sk<<<g, kSkBlock, 0, s>>>(b);
         }
         return;
     }
@@ -2486,9 +2538,11 @@ static void launch_pass2(const BatchDev &b, const FieldDev &hf, int want_stress,
         launch_sc_force_variant<T>(b.lpa2 ? pass2_view(b) : b, hf, want_stress, s);
     } else if (hf.do_ewald == 1) {
         k_ewald_tables<<<gA, kBlock, 0, s>>>(b);
-        dim3 g((b.maxnk + 63) / 64, b.W);
-        k_ewald_sk<<<g, AKMC_STAGE_BLOCK, 0, s>>>(b);
-        k_ewald_force<<<xcd_grid((b.A + kIonAtomsPerBlock - 1) / kIonAtomsPerBlock), kBlock, 0, s>>>(b);
+        dim3 g((b.maxnk + kSkTile - 1) / kSkTile, b.W);
+        k_ewald_sk<<<g, kSkBlock, 0, s>>>(b);
+        const dim3 ga((b.maxn + kEwAtoms - 1) / kEwAtoms, b.W);
+        if (b.G1 <= kEwG) k_ewald_force<true><<<ga, kBlock, 0, s>>>(b);
+        else k_ewald_force<false><<<ga, kBlock, 0, s>>>(b);
     }
 }
 

@@ -15,7 +15,7 @@
 // plus that of the atoms outside it, which changes only with the zone.
 //
 // What bounds it: one walker's chain of dependent phases (gathers, pair
-// terms, sums, the state machine's reductions; one walker alone runs at 60%
+// terms, sums, the state machine's reductions; one walker alone runs at 76%
 // of the rate of two on a CU), so a workgroup has eight wavefronts, two fit
 // a CU, the functions are out of line for 128 registers each, lists and
 // records are in LDS, and sums go by DPP moves.  512 walkers of 500-4000
