@@ -24,8 +24,8 @@ densities and energies within the list radius of a free atom), bit for bit
 the results of full evaluations.
 Also reported: the plain unbatched GPU dimer (one walker, host-driven
 micro-steps) on the same cells, force evaluations per second, the roofline
-of the dominant kernel of the search micro-steps (the zoned Sutton-Chen
-pass 1) timed with HIP events on the batch's stream, with the full
+of the search micro-steps' resident kernel, one evaluation of every search
+walker timed with HIP events on the batch's stream, with the full
 evaluation's pass 2 beside it, the learned-proposal A/B test, the KMC step
 (64 systems x 8 walkers taking kmcSteps steps of 5 valid events each), the
 tabulated-EAM field's force evaluation on the same walkers, the ionic
@@ -51,20 +51,18 @@ sys.path.insert(0, ROOT)
 METRIC = "FP64-verified saddles/sec at ≤0.01 eV barrier error; force evals/sec vs CPU"
 FP32_VECTOR_PEAK_TFLOPS = 157.3
 FP64_VECTOR_PEAK_TFLOPS = 78.6
-# algorithmic FLOP per ordered in-cutoff pair of the zoned pass 1 of the
-# search micro-steps: the density's 20 (1/r^2, (a/r)^2, (a/r)^6, the
-# coefficient, the sum, with the FP64 displacement and cutoff test) plus 5
-# for the pair energy (a/r)^9 = (a/r)^8 sqrt((a/r)^2), 1/2 eps (a/r)^9, its sum
-ZONE_PASS1_FLOP = 25
+# algorithmic FLOP per ordered in-cutoff pair of a free atom in a search
+# evaluation: the density's 20 (1/r^2, (a/r)^2, (a/r)^6, the coefficient, the
+# sum, with the FP64 displacement and cutoff test), 5 for the pair energy
+# ((a/r)^9 = (a/r)^8 sqrt((a/r)^2), 1/2 eps (a/r)^9, its sum) and the force
+# pass's 40; pairs of two frozen atoms keep their sums
+SEARCH_PAIR_FLOP = 65
 HBM_PEAK_GBS = 8000.0
 # HBM bytes per ordered pair of one all-walker k_sc_force launch, from
 # rocprofv3 --pmc FETCH_SIZE / WRITE_SIZE on `bench.py --forces-only 5`,
 # calibrated on a 1 GiB device copy (FETCH_SIZE reads half the copied bytes,
 # WRITE_SIZE all of them); the summary is under profiles/
 TRAFFIC_BYTES_PER_PAIR = 3.35
-# the same for the zoned pass 1 of the search micro-steps (k_sc_density with
-# pair energies), from the counter runs of `bench.py --zone-passes 10`
-ZONE_TRAFFIC_BYTES_PER_PAIR = 9.72
 
 
 def ordered_pairs(cells, positions, rc):
@@ -95,32 +93,21 @@ def atom_pairs(cells, positions, rc):
 
 def zone_work(camp, cells, rc):
     """The algorithmic work of one evaluation of the search walkers as the
-    micro-steps run it: ordered in-cutoff pairs of pass 1 (each walker's
-    zone, or all its atoms when it evaluates in full) and of pass 2 (its
-    free atoms, or all), over the walkers in FP32 mode, at the current
-    probes; zone atoms and free atoms per walker."""
-    member, size, flags, active = camp.batch.zone()
+    micro-steps run it: ordered in-cutoff pairs of the free atoms over the
+    walkers in FP32 mode, at the current probes, and the free atoms."""
+    _, _, _, active = camp.batch.zone()
     probes, _ = camp.batch.download()
     cnt = atom_pairs(cells, probes, rc)
-    p1 = p2 = n_zone = n_free = n_w = 0
+    pairs = n_free = n_w = 0
     for w, c in enumerate(cells):
         if active[w] != 1:
             continue
         o, k = camp.off[w], cnt[w]
         n_w += 1
-        if (flags[w] & 1) and not (flags[w] & 2):
-            zm = member[o:o + c.n] != 0
-            fr = camp._frozen[o:o + c.n] == 0
-            p1 += int(k[zm].sum())
-            p2 += int(k[fr].sum())
-            n_zone += int(zm.sum())
-            n_free += int(fr.sum())
-        else:
-            p1 += int(k.sum())
-            p2 += int(k.sum())
-            n_zone += c.n
-            n_free += c.n
-    return dict(pairs_pass1=p1, pairs_pass2=p2, zone_atoms=n_zone, free_atoms=n_free, walkers=n_w)
+        fr = camp._frozen[o:o + c.n] == 0
+        pairs += int(k[fr].sum())
+        n_free += int(fr.sum())
+    return dict(pairs_free=pairs, free_atoms=n_free, walkers=n_w)
 
 
 def plain_dimer_rate(L, W, text, cells, basins, proposal_fn, params, n_search, basin32, basin64, eager=False):
@@ -257,7 +244,7 @@ def forces_only(L, W, args):
 
 
 def zone_passes(L, S, W, args):
-    """The zoned pass kernels of the search micro-steps alone, for hardware
+    """The evaluation of the search micro-steps alone, for hardware
     counter runs: the batched campaign (3 pooled basins per walker, kernels
     launched one by one) after a 250-micro-step warm window and the per-pass
     variant tuning, then args.zone_passes evaluations of the running searches
@@ -733,7 +720,7 @@ def main():
     evals = camp.batch.eval_counts() - counts0
     camp.batch.kernel_timer(False)
     timed_ms = k_ms / max(k_launches, 1)
-    print(f"[bench] k_sc_force in the roofline window: {k_launches} launches, {timed_ms:.4f} ms per launch "
+    print(f"[bench] pass 2 in the roofline window: {k_launches} launches, {timed_ms:.4f} ms per launch "
           f"({int(evals.sum())} walker evaluations)", file=sys.stderr, flush=True)
     # ---- the pass kernels as the search micro-steps run them (active zones),
     # timed with HIP events on the batch's stream at the searches' current
@@ -742,10 +729,10 @@ def main():
     camp.batch.time_search_phases(1)
     zw = zone_work(camp, cells, rc)
     zph = camp.batch.time_search_phases(20)
-    z_tf1 = ZONE_PASS1_FLOP * zw["pairs_pass1"] / (zph[1] * 1e-3) / 1e12
-    z_tf2 = 40.0 * zw["pairs_pass2"] / (zph[2] * 1e-3) / 1e12
-    print(f"[bench] zoned search evaluation: {zw}; ms lists {zph[0]:.4f} pass 1 {zph[1]:.4f} ({z_tf1:.2f} TFLOP/s) "
-          f"pass 2 {zph[2]:.4f} ({z_tf2:.2f} TFLOP/s) reduce {zph[3]:.4f}", file=sys.stderr, flush=True)
+    z_ms = float(zph[1] + zph[2])
+    z_tf = SEARCH_PAIR_FLOP * zw["pairs_free"] / (z_ms * 1e-3) / 1e12
+    print(f"[bench] search evaluation: {zw}; ms lists {zph[0]:.4f} evaluation {z_ms:.4f} ({z_tf:.2f} TFLOP/s) "
+          f"reduce {zph[3]:.4f}", file=sys.stderr, flush=True)
     value = tot.distinct / t_timed
     verified_rate = tot.verified / t_timed
     moves_timed = camp.basin_moves
@@ -833,24 +820,18 @@ def main():
                      "no matrix form and uses no MFMA); peak is MI355X's published FP32 vector figure (packed "
                      "FP32). This build compiles without packed FP32 instructions, so its reachable FP32 "
                      "vector ceiling is half that: frac_vs_unpacked_ceiling",
-                     "kernel": "k_sc_density, zoned (Sutton-Chen pass 1 of the search micro-steps: density and "
-                               "pair energy of each walker's active zone, autotuned variant)",
-                     "achieved": round(z_tf1, 3), "peak": FP32_VECTOR_PEAK_TFLOPS, "unit": "TFLOP/s",
-                     "frac": round(z_tf1 / FP32_VECTOR_PEAK_TFLOPS, 4),
+                     "kernel": "k_search_resident (one evaluation of every search walker: densities, pair "
+                               "energies and forces of the pairs of its free atoms)",
+                     "achieved": round(z_tf, 3), "peak": FP32_VECTOR_PEAK_TFLOPS, "unit": "TFLOP/s",
+                     "frac": round(z_tf / FP32_VECTOR_PEAK_TFLOPS, 4),
                      "unpacked_ceiling": FP32_VECTOR_PEAK_TFLOPS / 2,
-                     "frac_vs_unpacked_ceiling": round(z_tf1 / (FP32_VECTOR_PEAK_TFLOPS / 2), 4),
-                     "traffic": round(ZONE_TRAFFIC_BYTES_PER_PAIR * zw["pairs_pass1"]),
-                     "traffic_note": "HBM bytes of one zoned pass-1 launch: 9.72 B per ordered pair (FETCH_SIZE x "
-                                     "2.0 + WRITE_SIZE x 1.0, scales from a 1 GiB copy) from the counter runs of "
-                                     "bench.py --zone-passes 10, times this launch's pairs",
+                     "frac_vs_unpacked_ceiling": round(z_tf / (FP32_VECTOR_PEAK_TFLOPS / 2), 4),
                      "measured_over": "20 evaluations of the search walkers at their probes after the timed "
-                                      "windows, as the micro-steps launch them (HIP events on the batch's stream)",
-                     "ms_per_launch": round(float(zph[1]), 4),
-                     "flops_per_launch": round(ZONE_PASS1_FLOP * zw["pairs_pass1"]),
-                     "flop_per_pair": ZONE_PASS1_FLOP,
+                                      "windows (HIP events on the batch's stream)",
+                     "ms_per_launch": round(z_ms, 4),
+                     "flops_per_launch": round(SEARCH_PAIR_FLOP * zw["pairs_free"]),
+                     "flop_per_pair": SEARCH_PAIR_FLOP,
                      "zones": zw,
-                     "pass2_zoned": {"kernel": "k_sc_force (free atoms)", "ms_per_launch": round(float(zph[2]), 4),
-                                     "flops_per_launch": 40 * zw["pairs_pass2"], "tflops": round(z_tf2, 3)},
                      "window_k_sc_force_ms_per_launch": round(timed_ms, 4),
                      "full_evaluation": {"kernel": "k_sc_force over every atom of every walker at the basins",
                                          "ms_per_launch": round(force_ms, 4), "flops_per_launch": 40 * Ptot,
