@@ -330,11 +330,14 @@ int akmc_batch_set_search_zone(akmc_batch_t b, int enable);
 /* Workgroup size of the walker state machines: 256 threads, or 1024 (the
  * default for batches whose largest walker has at least 16 384 atoms).  No
  * counterpart in the reference; the two differ only in the order of their
- * block sums. */
+ * block sums.  Search walkers whose free region fits one workgroup are
+ * advanced by the resident kernel, which has its own block. */
 int akmc_batch_set_logic_block(akmc_batch_t b, int threads);
 /* akmc_batch_time_phases for the search walkers at their current probes, as
  * the search micro-steps launch the kernels (active zones included), without
- * advancing any search (no counterpart in the reference: measurement). */
+ * advancing any search (no counterpart in the reference: measurement).  The
+ * resident kernel's whole evaluation counts in ms[1]; ms[2] is the second
+ * pass of the walkers outside it. */
 int akmc_batch_time_search_phases(akmc_batch_t b, int nrep, double ms[4]);
 /* The active zones (no counterpart in the reference: inspection): member[A]
  * 1 for the atoms in their walker's zone, size[W] zone sizes, flags[W] the
