@@ -426,19 +426,20 @@ void akmc_launch_harvest_pack(const BatchDev &b, const SearchDev &s, int *harves
 void akmc_mlp_launch_weights(const float *p, uint16_t *w1t, uint16_t *w2t, uint16_t *w3t, uint16_t *w2r,
                              uint16_t *w3r, hipStream_t s);
 #define AKMC_MLP_PARAMS 23171
-#define AKMC_MLP_MAXBLOCKS 256  // workgroups of the gradient kernel at most
 // rows of X standardised in place: (X - mean) * scale
 void akmc_mlp_launch_standardize(float *X, long long rows, const float *mean, const float *scale, hipStream_t s);
 // Y [M][3] of the rows X [M][48]
 void akmc_mlp_launch_forward(const float *X, int M, const float *p, const uint16_t *w1t, const uint16_t *w2t,
                              const uint16_t *w3t, float *Y, hipStream_t s);
-// gradient sums of rows idx[0 .. M) (null: rows 0 .. M) per workgroup into P
-// [blocks][AKMC_MLP_PARAMS], squared errors into part [blocks]
-int akmc_mlp_grad_blocks(int M);
+// gradient sums of rows idx[0 .. M) (null: rows 0 .. M): weights per chunk of
+// rows into P [chunks][AKMC_MLP_PARAMS], biases into g, squared errors into
+// part [chunks]; rows: akmc_mlp_rows_bytes(M) bytes between its two kernels
+int akmc_mlp_grad_chunks(int M);
+size_t akmc_mlp_rows_bytes(int rows);
 void akmc_mlp_launch_grad(const float *X, const float *T, const int *idx, int M, const float *p, const uint16_t *w1t,
-                          const uint16_t *w2t, const uint16_t *w3t, const uint16_t *w2r, const uint16_t *w3r, float *P,
-                          double *part, hipStream_t s);
-// the gradient g from P; step: Adam step t and the BF16 weights too; the mean
+                          const uint16_t *w2t, const uint16_t *w3t, const uint16_t *w2r, const uint16_t *w3r,
+                          void *rows, float *P, double *part, float *g, hipStream_t s);
+// the weights' gradient into g from P; step: Adam step t and the BF16 weights too; the mean
 // loss of the M rows is added to acc (device, may be null)
 void akmc_mlp_launch_update(const float *P, int M, float *g, float *p, float *m1, float *m2, uint16_t *w1t,
                             uint16_t *w2t, uint16_t *w3t, uint16_t *w2r, uint16_t *w3r, int step, float lr, int t,

@@ -2746,6 +2746,7 @@ struct akmc_mlp_s {
     float *p = nullptr, *g = nullptr, *m1 = nullptr, *m2 = nullptr;
     uint16_t *w1t = nullptr, *w2t = nullptr, *w3t = nullptr, *w2r = nullptr, *w3r = nullptr;
     float *X = nullptr, *T = nullptr, *Y = nullptr, *P = nullptr, *ms = nullptr;  // ms: mean and scale of the inputs
+    char *rbuf = nullptr;  // the gradient's per-row operands
     double *lpart = nullptr;
     int adam_t = 0;
 };
@@ -2788,7 +2789,8 @@ int mlp_scaling(akmc_mlp_t m, const float *mean, const float *scale)
 // Adam step); acc: where the rows' mean loss is added, or null
 int mlp_grad(akmc_mlp_t m, const float *X, const float *T, const int *idx, int M, int step, float lr, double *acc)
 {
-    akmc_mlp_launch_grad(X, T, idx, M, m->p, m->w1t, m->w2t, m->w3t, m->w2r, m->w3r, m->P, m->lpart, m->stream);
+    akmc_mlp_launch_grad(X, T, idx, M, m->p, m->w1t, m->w2t, m->w3t, m->w2r, m->w3r, m->rbuf, m->P,
+                         m->lpart, m->g, m->stream);
     if (step) ++m->adam_t;
     akmc_mlp_launch_update(m->P, M, m->g, m->p, m->m1, m->m2, m->w1t, m->w2t, m->w3t, m->w2r, m->w3r, step, lr,
                            std::max(m->adam_t, 1), m->lpart, acc, m->stream);
@@ -2819,8 +2821,9 @@ int akmc_mlp_create(int max_rows, unsigned seed, akmc_mlp_t *out)
         (rc = malloc_m(m, &m->w2r, 128 * 128)) || (rc = malloc_m(m, &m->w3r, 128 * 16)) ||
         (rc = malloc_m(m, &m->X, R * 48)) || (rc = malloc_m(m, &m->T, R * 3)) ||
         (rc = malloc_m(m, &m->Y, R * 3)) ||
-        (rc = malloc_m(m, &m->P, (size_t)akmc_mlp_grad_blocks((int)R) * NP)) ||
-        (rc = malloc_m(m, &m->lpart, AKMC_MLP_MAXBLOCKS)) || (rc = malloc_m(m, &m->ms, 96)))
+        (rc = malloc_m(m, &m->rbuf, akmc_mlp_rows_bytes((int)R))) ||
+        (rc = malloc_m(m, &m->P, (size_t)akmc_mlp_grad_chunks((int)R) * NP)) ||
+        (rc = malloc_m(m, &m->lpart, akmc_mlp_grad_chunks((int)R))) || (rc = malloc_m(m, &m->ms, 96)))
         return bad(rc);
     HIPCHK(hipMemset(m->m1, 0, NP * sizeof(float)));
     HIPCHK(hipMemset(m->m2, 0, NP * sizeof(float)));
@@ -2897,7 +2900,7 @@ int akmc_mlp_loss_grad(akmc_mlp_t m, const float *X, const float *T, int M, doub
     HIPCHK(hipMemcpyAsync(m->X, X, (size_t)M * 48 * sizeof(float), hipMemcpyHostToDevice, m->stream));
     HIPCHK(hipMemcpyAsync(m->T, T, (size_t)M * 3 * sizeof(float), hipMemcpyHostToDevice, m->stream));
     TRY(mlp_grad(m, m->X, m->T, nullptr, M, 0, 0.0f, nullptr));
-    std::vector<double> part(akmc_mlp_grad_blocks(M));
+    std::vector<double> part(akmc_mlp_grad_chunks(M));
     if (loss)
         HIPCHK(hipMemcpyAsync(part.data(), m->lpart, part.size() * sizeof(double), hipMemcpyDeviceToHost, m->stream));
     if (grad) HIPCHK(hipMemcpyAsync(grad, m->g, AKMC_MLP_NPARAM * sizeof(float), hipMemcpyDeviceToHost, m->stream));

@@ -33,34 +33,11 @@ constexpr int kW1 = 0, kB1 = kIn * kHid, kW2 = kB1 + kHid, kB2 = kW2 + kHid * kH
               kB3 = kW3 + kHid * kOut, kParam = kB3 + kOut;
 static_assert(kParam == AKMC_MLP_PARAMS, "parameter count");
 
-// Forward and backward of a tile of 64 rows stay in one workgroup: wavefront
-// v takes rows 16 v .. 16 v + 15 through every layer (its pre-activations
-// stay in registers for the backward pass), activations pass from layer to
-// layer through LDS as the BF16 operands of the next product, row-major for
-// the layers and transposed for the weight gradients.  Before, each layer
-// was a launch that wrote its FP32 activations to memory: 17 launches per
-// minibatch, most of them launch latency at 4096 rows.
-constexpr int kTile = 64;
-constexpr int kTP = kTile + 4;  // pitch of the transposed operands (BF16), rows of 8-byte multiples
-constexpr int kRP = kHid + 4;   // pitch of the row-major ones
-
-struct MlpLds {
-    uint16_t xt[kIn][kTP], h1t[kHid][kTP], h2t[kHid][kTP], z1t[kHid][kTP], z2t[kHid][kTP], yt[16][kTP];
-    uint16_t hr[kTile][kRP];   // H1, then dZ2, row-major
-    uint16_t h2r[kTile][kRP];
-    uint16_t yr[kTile][20];    // dY
-    float bsum[4][2 * kHid + 16];  // per wavefront: column sums of dZ1, dZ2, dY
-    double loss[4];
-};
+constexpr int kTile = 64;      // rows of a forward workgroup, 16 per wavefront
+constexpr int kRP = kHid + 4;  // pitch of row-major BF16 operands in LDS
 
 __device__ inline f32x4 mfma(bf16x4 a, bf16x4 b, f32x4 c) { return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0); }
 __device__ inline bf16x4 bf4(const uint16_t *p) { return *reinterpret_cast<const bf16x4 *>(p); }
-__device__ inline float dsilu(float z)
-{
-    const float s = sigm(z);
-    return s * (1.0f + z * (1.0f - s));
-}
-
 // the operand of 16 rows of X (48 inputs) per lane: X[row][16 s + lk ..+3]
 __device__ inline void load_rows(const float *X, long long row, bool ok, int lk, bf16x4 (&a)[3])
 {
@@ -85,10 +62,10 @@ __device__ inline bf16x4 wfrag(const uint16_t *w, int nt, int s, int ks)
 }
 
 // one hidden layer of the wavefront's 16 rows: Z = A W + b into registers,
-// silu(Z) as BF16 row-major (hr) and, when TR, transposed (ht)
-template <int KS, bool TR>
+// silu(Z) as BF16 row-major (hr) and per column tile to put(tile, 4 rows)
+template <int KS, typename PUT>
 __device__ inline void hidden_layer(const bf16x4 (&a)[KS], const uint16_t *wt, const float *bias, int r0, int li, int lk,
-                                    f32x4 (&Z)[8], uint16_t (*hr)[kRP], uint16_t (*ht)[kTP])
+                                    f32x4 (&Z)[8], uint16_t (*hr)[kRP], PUT put)
 {
 #pragma unroll
     for (int nt = 0; nt < 8; ++nt) {
@@ -105,7 +82,7 @@ __device__ inline void hidden_layer(const bf16x4 (&a)[KS], const uint16_t *wt, c
             h[e] = (short)to_bf16(z * sigm(z));
             hr[r0 + lk + e][col] = (uint16_t)h[e];
         }
-        if constexpr (TR) *reinterpret_cast<bf16x4 *>(&ht[col][r0 + lk]) = h;
+        put(nt, h);
         // a few column tiles' weights in flight, not all eight: registers
         if (nt % 2 == 1) __builtin_amdgcn_sched_barrier(0);
     }
@@ -123,11 +100,11 @@ __global__ void __launch_bounds__(kB) k_mlp_forward(const float *__restrict__ X,
     bf16x4 a1[3], a[8];
     f32x4 Z[8];
     load_rows(X, m0 + r0 + li, m0 + r0 + li < M, lk, a1);
-    hidden_layer<3, false>(a1, w1t, p + kB1, r0, li, lk, Z, h1, nullptr);
+    hidden_layer<3>(a1, w1t, p + kB1, r0, li, lk, Z, h1, [](int, bf16x4) {});
     __syncthreads();
 #pragma unroll
     for (int s = 0; s < 8; ++s) a[s] = bf4(&h1[r0 + li][16 * s + lk]);
-    hidden_layer<8, false>(a, w2t, p + kB2, r0, li, lk, Z, h2, nullptr);
+    hidden_layer<8>(a, w2t, p + kB2, r0, li, lk, Z, h2, [](int, bf16x4) {});
     __syncthreads();
     f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
 #pragma unroll
@@ -142,173 +119,204 @@ __global__ void __launch_bounds__(kB) k_mlp_forward(const float *__restrict__ X,
 }
 
 // Gradient of the mean-squared loss over rows idx[0 .. M) of (X, T) (idx
-// null: rows 0 .. M): the tiles of a workgroup add up in registers, its sums
-// go to P[blockIdx.x][kParam] and its squared error to part[blockIdx.x]
-__global__ void __launch_bounds__(kB, 1) k_mlp_grad(const float *__restrict__ X, const float *__restrict__ T,
+// null: rows 0 .. M), in an order of summation that depends on M alone:
+// weight gradients over kChunk rows at a time by one matrix-instruction chain
+// each, the chunks in order; bias gradients as the sums over the rows equal
+// modulo kChunk, in order, and a tree over these.
+//
+// k_mlp_rows: one wavefront per 16 rows, forward and backward.  What the
+// weight gradients contract over the rows goes to memory in the order the
+// matrix instruction reads it (MlpRows: a 16-row x 16-column tile is 64 lanes
+// x 4 rows, 512 contiguous bytes in BF16).  k_mlp_wgrad: per chunk 96
+// wavefronts, one per 16 x 16 tile of dW1, dW2, dW3, and a workgroup per 16
+// bias columns.  Bound by latency at 4096 rows.
+constexpr int kChunk = 256;  // rows of a weight-gradient partial sum
+
+struct MlpRows {
+    uint16_t *x, *h1, *h2;  // [row tile][column tile][64][4] BF16: inputs, activations
+    float *z1, *z2;         // the same in FP32: d loss / d pre-activation
+    float *r;               // [row tile][64][4]: Y - T, 3 of 16 columns
+};
+
+__global__ void __launch_bounds__(64) k_mlp_rows(const float *__restrict__ X, const float *__restrict__ T,
                                                  const int *__restrict__ idx, int M, const float *__restrict__ p,
                                                  const uint16_t *__restrict__ w1t, const uint16_t *__restrict__ w2t,
                                                  const uint16_t *__restrict__ w3t, const uint16_t *__restrict__ w2r,
-                                                 const uint16_t *__restrict__ w3r, float *__restrict__ P,
-                                                 double *__restrict__ part)
+                                                 const uint16_t *__restrict__ w3r, MlpRows o)
 {
-    __shared__ MlpLds L;
-    const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
-    int r0 = 16 * wave, li = lane & 15, lk = (lane >> 4) * 4;
-    f32x4 g1[6], g2[16], g3[2];  // this wavefront's tiles of dW1, dW2, dW3
-    const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
-    for (auto &v : g1) v = zero;
-    for (auto &v : g2) v = zero;
-    for (auto &v : g3) v = zero;
-    float s1[8] = {}, s2[8] = {}, s3 = 0.0f;  // column sums of dZ1, dZ2, dY
-    double sq = 0.0;
-    const int ntiles = (M + kTile - 1) / kTile;
-    for (int tile = blockIdx.x; tile < ntiles; tile += gridDim.x) {
-        const int m0 = tile * kTile;
-        __syncthreads();  // the previous tile's operands are read
-        // (the LDS addresses below are not worth a register each across tiles)
-        asm volatile("" : "+v"(r0), "+v"(li), "+v"(lk));
-        f32x4 Z1[8], Z2[8];
-        {
-            bf16x4 a[3];
-            const int m = m0 + r0 + li;
-            const bool ok = m < M;
-            load_rows(X, ok ? (idx ? idx[m] : m) : 0, ok, lk, a);
+    __shared__ uint16_t hr[16][kRP], h2r[16][kRP];  // H1, then dZ2; H2
+    __shared__ uint16_t xt[kIn][20], yr[16][20];    // X transposed; dY
+    const int lane = threadIdx.x, li = lane & 15, lk = (lane >> 4) * 4;
+    const size_t tile = blockIdx.x;
+    const int m0 = 16 * blockIdx.x;
+    f32x4 Z1[8], Z2[8];
+    // rows past M have no part in the sums: zeros
+    auto put = [&](uint16_t *dst, int nt, bf16x4 v) {
 #pragma unroll
-            for (int s = 0; s < 3; ++s)
+        for (int e = 0; e < 4; ++e)
+            if (m0 + lk + e >= M) v[e] = 0;
+        *reinterpret_cast<bf16x4 *>(dst + ((tile * 8 + nt) * 64 + lane) * 4) = v;
+    };
+    {
+        bf16x4 a[3];
+        const bool ok = m0 + li < M;
+        load_rows(X, ok ? (idx ? idx[m0 + li] : m0 + li) : 0, ok, lk, a);
 #pragma unroll
-                for (int e = 0; e < 4; ++e) L.xt[16 * s + lk + e][r0 + li] = (uint16_t)a[s][e];
-            hidden_layer<3, true>(a, w1t, p + kB1, r0, li, lk, Z1, L.hr, L.h1t);
-        }
-        __syncthreads();
-        {
-            bf16x4 a[8];
+        for (int s = 0; s < 3; ++s)
 #pragma unroll
-            for (int s = 0; s < 8; ++s) a[s] = bf4(&L.hr[r0 + li][16 * s + lk]);
-            hidden_layer<8, true>(a, w2t, p + kB2, r0, li, lk, Z2, L.h2r, L.h2t);
-        }
-        __syncthreads();
-        {
-            // output layer, error and dY = 2 (Y - T) / M; rows past M have none
-            f32x4 acc = zero;
-#pragma unroll
-            for (int s = 0; s < 8; ++s) acc = mfma(bf4(&L.h2r[r0 + li][16 * s + lk]), wfrag(w3t, 0, s, 8), acc);
-            const float bb = li < kOut ? p[kB3 + li] : 0.0f;
-            bf16x4 d;
-#pragma unroll
-            for (int e = 0; e < 4; ++e) {
-                const int m = m0 + r0 + lk + e;
-                float r = 0.0f;
-                if (m < M && li < kOut) r = acc[e] + bb - T[(long long)(idx ? idx[m] : m) * kOut + li];
-                sq += (double)r * r;
-                const float dy = 2.0f * r / (float)M;
-                s3 += dy;
-                d[e] = (short)to_bf16(dy);
-                L.yr[r0 + lk + e][li] = (uint16_t)d[e];
-            }
-            *reinterpret_cast<bf16x4 *>(&L.yt[li][r0 + lk]) = d;
-        }
-        __syncthreads();
-        {
-            const bf16x4 a = bf4(&L.yr[r0 + li][lk]);
-#pragma unroll
-            for (int nt = 0; nt < 8; ++nt) {
-                const int col = 16 * nt + li;
-                const f32x4 acc = mfma(a, wfrag(w3r, nt, 0, 1), zero);
-                bf16x4 d;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float v = acc[e] * dsilu(Z2[nt][e]);
-                    s2[nt] += v;
-                    d[e] = (short)to_bf16(v);
-                    L.hr[r0 + lk + e][col] = (uint16_t)d[e];
-                }
-                *reinterpret_cast<bf16x4 *>(&L.z2t[col][r0 + lk]) = d;
-            }
-        }
-        __syncthreads();
-        {
-            bf16x4 a[8];
-#pragma unroll
-            for (int s = 0; s < 8; ++s) a[s] = bf4(&L.hr[r0 + li][16 * s + lk]);
-#pragma unroll
-            for (int nt = 0; nt < 8; ++nt) {
-                const int col = 16 * nt + li;
-                f32x4 acc = zero;
-#pragma unroll
-                for (int s = 0; s < 8; ++s) acc = mfma(a[s], wfrag(w2r, nt, s, 8), acc);
-                bf16x4 d;
-#pragma unroll
-                for (int e = 0; e < 4; ++e) {
-                    const float v = acc[e] * dsilu(Z1[nt][e]);
-                    s1[nt] += v;
-                    d[e] = (short)to_bf16(v);
-                }
-                *reinterpret_cast<bf16x4 *>(&L.z1t[col][r0 + lk]) = d;
-                if (nt % 2 == 1) __builtin_amdgcn_sched_barrier(0);
-            }
-        }
-        __syncthreads();
-        // weight gradients over the tile's 64 rows: wavefront v takes row
-        // tiles 2 v, 2 v + 1 of dW2 and dW3 and the tiles 6 v .. 6 v + 5 of dW1
-#pragma unroll 1
-        for (int s = 0; s < 4; ++s) {
-            const int m = 16 * s + lk;
-#pragma unroll
-            for (int i = 0; i < 2; ++i) {
-                const bf16x4 a = bf4(&L.h1t[16 * (2 * wave + i) + li][m]);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) g2[8 * i + j] = mfma(a, bf4(&L.z2t[16 * j + li][m]), g2[8 * i + j]);
-                g3[i] = mfma(bf4(&L.h2t[16 * (2 * wave + i) + li][m]), bf4(&L.yt[li][m]), g3[i]);
-            }
-#pragma unroll
-            for (int t = 0; t < 6; ++t) {
-                const int i = (6 * wave + t) / 8, j = (6 * wave + t) % 8;
-                g1[t] = mfma(bf4(&L.xt[16 * i + li][m]), bf4(&L.z1t[16 * j + li][m]), g1[t]);
-            }
-        }
+            for (int e = 0; e < 4; ++e) xt[16 * s + lk + e][li] = (uint16_t)a[s][e];
+        hidden_layer<3>(a, w1t, p + kB1, 0, li, lk, Z1, hr, [&](int nt, bf16x4 h) { put(o.h1, nt, h); });
     }
-    float *out = P + (size_t)blockIdx.x * kParam;
+    __syncthreads();
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
+    for (int s = 0; s < 3; ++s)
+        *reinterpret_cast<bf16x4 *>(o.x + ((tile * 3 + s) * 64 + lane) * 4) = bf4(&xt[16 * s + li][lk]);
+    {
+        bf16x4 a[8];
 #pragma unroll
-        for (int i = 0; i < 2; ++i) {
-            const int k = 16 * (2 * wave + i) + lk + e;
-#pragma unroll
-            for (int j = 0; j < 8; ++j) out[kW2 + k * kHid + 16 * j + li] = g2[8 * i + j][e];
-            if (li < kOut) out[kW3 + k * kOut + li] = g3[i][e];
-        }
-#pragma unroll
-        for (int t = 0; t < 6; ++t) {
-            const int i = (6 * wave + t) / 8, j = (6 * wave + t) % 8;
-            out[kW1 + (16 * i + lk + e) * kHid + 16 * j + li] = g1[t][e];
-        }
+        for (int s = 0; s < 8; ++s) a[s] = bf4(&hr[li][16 * s + lk]);
+        hidden_layer<8>(a, w2t, p + kB2, 0, li, lk, Z2, h2r, [&](int nt, bf16x4 h) { put(o.h2, nt, h); });
     }
-    // column sums: the four row groups of a wavefront, then the wavefronts in order
+    __syncthreads();
+    {
+        // output layer, error r = Y - T and dY = 2 r / M
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f}, r = acc;
 #pragma unroll
-    for (int nt = 0; nt < 8; ++nt) {
-        s1[nt] += __shfl_xor(s1[nt], 16);
-        s1[nt] += __shfl_xor(s1[nt], 32);
-        s2[nt] += __shfl_xor(s2[nt], 16);
-        s2[nt] += __shfl_xor(s2[nt], 32);
+        for (int s = 0; s < 8; ++s) acc = mfma(bf4(&h2r[li][16 * s + lk]), wfrag(w3t, 0, s, 8), acc);
+        const float bb = li < kOut ? p[kB3 + li] : 0.0f;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int m = m0 + lk + e;
+            if (m < M && li < kOut) r[e] = acc[e] + bb - T[(long long)(idx ? idx[m] : m) * kOut + li];
+            yr[lk + e][li] = to_bf16(2.0f * r[e] / (float)M);
+        }
+        *reinterpret_cast<f32x4 *>(o.r + (tile * 64 + lane) * 4) = r;
     }
-    s3 += __shfl_xor(s3, 16);
-    s3 += __shfl_xor(s3, 32);
-    for (int o = 1; o < 64; o <<= 1) sq += __shfl_xor(sq, o);
-    if (lane < 16) {
+    __syncthreads();
+    {
+        const bf16x4 a = bf4(&yr[li][lk]);
 #pragma unroll
         for (int nt = 0; nt < 8; ++nt) {
-            L.bsum[wave][16 * nt + li] = s1[nt];
-            L.bsum[wave][kHid + 16 * nt + li] = s2[nt];
+            f32x4 v = mfma(a, wfrag(w3r, nt, 0, 1), f32x4{0.0f, 0.0f, 0.0f, 0.0f});
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float z = Z2[nt][e], s = sigm(z);
+                v[e] = m0 + lk + e < M ? v[e] * s * (1.0f + z * (1.0f - s)) : 0.0f;
+                hr[lk + e][16 * nt + li] = to_bf16(v[e]);
+            }
+            *reinterpret_cast<f32x4 *>(o.z2 + ((tile * 8 + nt) * 64 + lane) * 4) = v;
         }
-        L.bsum[wave][2 * kHid + li] = s3;
     }
-    if (lane == 0) L.loss[wave] = sq;
     __syncthreads();
-    for (int c = threadIdx.x; c < 2 * kHid + kOut; c += kB) {
-        const float v = ((L.bsum[0][c] + L.bsum[1][c]) + L.bsum[2][c]) + L.bsum[3][c];
-        out[c < kHid ? kB1 + c : c < 2 * kHid ? kB2 + c - kHid : kB3 + c - 2 * kHid] = v;
+    {
+        bf16x4 a[8];
+#pragma unroll
+        for (int s = 0; s < 8; ++s) a[s] = bf4(&hr[li][16 * s + lk]);
+#pragma unroll
+        for (int nt = 0; nt < 8; ++nt) {
+            f32x4 v = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll
+            for (int s = 0; s < 8; ++s) v = mfma(a[s], wfrag(w2r, nt, s, 8), v);
+#pragma unroll
+            for (int e = 0; e < 4; ++e) {
+                const float z = Z1[nt][e], s = sigm(z);
+                v[e] = m0 + lk + e < M ? v[e] * s * (1.0f + z * (1.0f - s)) : 0.0f;
+            }
+            *reinterpret_cast<f32x4 *>(o.z1 + ((tile * 8 + nt) * 64 + lane) * 4) = v;
+            if (nt % 2 == 1) __builtin_amdgcn_sched_barrier(0);
+        }
     }
-    if (threadIdx.x == 0) part[blockIdx.x] = ((L.loss[0] + L.loss[1]) + L.loss[2]) + L.loss[3];
+}
+
+__device__ inline bf16x4 bf16_of(f32x4 v)
+{
+    return bf16x4{(short)to_bf16(v[0]), (short)to_bf16(v[1]), (short)to_bf16(v[2]), (short)to_bf16(v[3])};
+}
+
+// Per chunk seven workgroups of 16 wavefronts: six with a 16 x 16 tile of the
+// weight gradients per wavefront (P [chunk][kParam]) and one for the squared
+// error (part [chunk]); after them one per 16 bias columns (into g)
+constexpr int kWgBlock = 1024, kWgPer = 7;
+constexpr int kWgBias = 17;  // dZ1, dZ2 (8 column tiles each), dY
+__global__ void __launch_bounds__(kWgBlock) k_mlp_wgrad(MlpRows in, int M, int nchunk, float *__restrict__ P,
+                                                        double *__restrict__ part, float *__restrict__ g)
+{
+    constexpr int kTiles = kChunk / 16;  // row tiles of a chunk
+    __shared__ double sh[kChunk * 17 / 2];
+    const int tid = threadIdx.x, lane = tid & 63, wave = tid >> 6, li = lane & 15, lk = (lane >> 4) * 4;
+    const int ntile = (M + 15) / 16;
+    auto frag4 = [&](const float *src, size_t t) { return *reinterpret_cast<const f32x4 *>(src + (t * 64 + lane) * 4); };
+    auto dy = [&](f32x4 r) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) r[e] = 2.0f * r[e] / (float)M;
+        return r;
+    };
+    if ((int)blockIdx.x < kWgPer * nchunk) {
+        const int chunk = blockIdx.x / kWgPer, part_of = blockIdx.x % kWgPer;
+        const int t0 = chunk * kTiles, t1 = min(t0 + kTiles, ntile);
+        if (part_of == kWgPer - 1) {
+            if (tid < kChunk) {
+                double l = 0.0;
+                const int m = chunk * kChunk + tid;
+                if (m < M)
+                    for (int c = 0; c < kOut; ++c) {
+                        const float r = in.r[((size_t)(m / 16) * 64 + (m % 16) / 4 * 16 + c) * 4 + m % 4];
+                        l += (double)r * r;
+                    }
+                sh[tid] = l;
+            }
+            __syncthreads();
+            for (int o = kChunk / 2; o > 0; o >>= 1) {
+                if (tid < o) sh[tid] += sh[tid + o];
+                __syncthreads();
+            }
+            if (tid == 0) part[chunk] = sh[0];
+            return;
+        }
+        // tiles 0 .. 63: dW2, 64 .. 87: dW1, 88 .. 95: dW3
+        const int t = part_of * (kWgBlock / 64) + wave;
+        const int kind = t < 64 ? 0 : t < 88 ? 1 : 2, u = kind == 0 ? t : kind == 1 ? t - 64 : t - 88;
+        const int i = kind == 2 ? u : u / 8, j = kind == 2 ? 0 : u % 8, an = kind == 1 ? 3 : 8;
+        const uint16_t *A = kind == 0 ? in.h1 : kind == 1 ? in.x : in.h2;
+        f32x4 acc = {0.0f, 0.0f, 0.0f, 0.0f};
+        for (int r0 = t0; r0 < t1; r0 += 4) {  // four row tiles' operands in flight
+            bf16x4 a[4];
+            f32x4 v[4];
+#pragma unroll
+            for (int q = 0; q < 4; ++q) {
+                const size_t rt = min(r0 + q, t1 - 1);
+                a[q] = bf4(A + ((rt * an + i) * 64 + lane) * 4);
+                v[q] = kind == 0 ? frag4(in.z2, rt * 8 + j) : kind == 1 ? frag4(in.z1, rt * 8 + j) : dy(frag4(in.r, rt));
+            }
+#pragma unroll
+            for (int q = 0; q < 4; ++q)
+                if (r0 + q < t1) acc = mfma(a[q], bf16_of(v[q]), acc);
+        }
+        float *out = P + (size_t)chunk * kParam;
+#pragma unroll
+        for (int e = 0; e < 4; ++e) {
+            const int k = 16 * i + lk + e;
+            if (kind == 0) out[kW2 + k * kHid + 16 * j + li] = acc[e];
+            else if (kind == 1) out[kW1 + k * kHid + 16 * j + li] = acc[e];
+            else if (li < kOut) out[kW3 + k * kOut + li] = acc[e];
+        }
+        return;
+    }
+    // column sums: wavefront v holds the rows 16 v .. 16 v + 15 modulo kChunk
+    const int bt = blockIdx.x - kWgPer * nchunk, j = bt % 8;
+    float (*tree)[17] = reinterpret_cast<float (*)[17]>(sh);
+    f32x4 s = {0.0f, 0.0f, 0.0f, 0.0f};
+#pragma unroll 4
+    for (int rt = wave; rt < ntile; rt += kTiles)
+        s += bt < 8 ? frag4(in.z1, (size_t)rt * 8 + j) : bt < 16 ? frag4(in.z2, (size_t)rt * 8 + j) : dy(frag4(in.r, rt));
+#pragma unroll
+    for (int e = 0; e < 4; ++e) tree[16 * wave + lk + e][li] = s[e];
+    __syncthreads();
+    for (int o = kChunk / 2; o > 0; o >>= 1) {
+        for (int q = tid; q < o * 16; q += kWgBlock) tree[q / 16][q % 16] += tree[q / 16 + o][q % 16];
+        __syncthreads();
+    }
+    if (tid < (bt < 16 ? 16 : kOut)) g[(bt < 8 ? kB1 + 16 * j : bt < 16 ? kB2 + 16 * j : kB3) + tid] = tree[0][tid];
 }
 
 // BF16 copies of parameter i in fragment order: the forward operands
@@ -346,26 +354,28 @@ __global__ void k_weights_bf16(const float *__restrict__ p, MlpBf16 w)
     if (i < kParam) store_bf16(w, i, p[i]);
 }
 
-// the gradient: the workgroups' sums in order, four interleaved runs of them
-// per parameter added in a fixed order; with step the Adam step and the
-// BF16 copies of the parameter; the loss of the rows, scaled, is added to acc
-constexpr int kUpd = 64;  // parameters per workgroup
-__global__ void __launch_bounds__(4 * kUpd) k_mlp_update(const float *__restrict__ P, int nb, float *__restrict__ g,
-                                                         float *__restrict__ p, float *__restrict__ m1,
-                                                         float *__restrict__ m2, MlpBf16 w, int step, float lr, float b1, float b2,
-                                                         float eps, float c1, float c2, const double *__restrict__ part,
-                                                         double scale, double *__restrict__ acc)
+// the weights' gradient: the chunks' sums in order (the biases' is in g
+// already); with step the Adam step and the BF16 copies of the parameter; the
+// loss of the rows, scaled, is added to acc
+constexpr int kUpd = 128;  // parameters per workgroup
+__global__ void __launch_bounds__(kUpd) k_mlp_update(const float *__restrict__ P, int nchunk, float *__restrict__ g,
+                                                     float *__restrict__ p, float *__restrict__ m1,
+                                                     float *__restrict__ m2, MlpBf16 w, int step, float lr, float b1,
+                                                     float b2, float eps, float c1, float c2,
+                                                     const double *__restrict__ part, double scale,
+                                                     double *__restrict__ acc)
 {
-    __shared__ float sh[4][kUpd];
-    const int c = threadIdx.x % kUpd, run = threadIdx.x / kUpd, i = blockIdx.x * kUpd + c;
-    float s = 0.0f;
-    if (i < kParam)
-        for (int k = run; k < nb; k += 4) s += P[(size_t)k * kParam + i];
-    sh[run][c] = s;
-    __syncthreads();
-    if (run == 0 && i < kParam) {
-        const float gi = (sh[0][c] + sh[1][c]) + (sh[2][c] + sh[3][c]);
-        g[i] = gi;
+    const int i = blockIdx.x * kUpd + threadIdx.x;
+    if (i < kParam) {
+        const bool bias = (i >= kB1 && i < kW2) || (i >= kB2 && i < kW3) || i >= kB3;
+        float gi = 0.0f;
+        if (bias) {
+            gi = g[i];
+        } else {
+#pragma unroll 8
+            for (int c = 0; c < nchunk; ++c) gi += P[(size_t)c * kParam + i];
+            g[i] = gi;
+        }
         if (step) {
             const float a = b1 * m1[i] + (1.0f - b1) * gi;
             const float b = b2 * m2[i] + (1.0f - b2) * gi * gi;
@@ -376,9 +386,9 @@ __global__ void __launch_bounds__(4 * kUpd) k_mlp_update(const float *__restrict
             store_bf16(w, i, v);
         }
     }
-    if (acc && blockIdx.x == 0 && threadIdx.x == 4 * kUpd - 1) {
+    if (acc && blockIdx.x == 0 && threadIdx.x == kUpd - 1) {
         double t = 0.0;
-        for (int k = 0; k < nb; ++k) t += part[k];
+        for (int c = 0; c < nchunk; ++c) t += part[c];
         *acc += t * scale;
     }
 }
@@ -578,17 +588,29 @@ void akmc_mlp_launch_forward(const float *X, int M, const float *p, const uint16
     k_mlp_forward<<<(M + kTile - 1) / kTile, kB, 0, s>>>(X, M, p, w1t, w2t, w3t, Y);
 }
 
-int akmc_mlp_grad_blocks(int M)
+int akmc_mlp_grad_chunks(int M) { return (M + kChunk - 1) / kChunk; }
+
+size_t akmc_mlp_rows_bytes(int rows)
 {
-    const int tiles = (M + kTile - 1) / kTile;
-    return tiles < AKMC_MLP_MAXBLOCKS ? tiles : AKMC_MLP_MAXBLOCKS;
+    const size_t tiles = (rows + 15) / 16;
+    return tiles * 64 * 4 * ((3 + 8 + 8) * sizeof(uint16_t) + (8 + 8 + 1) * sizeof(float));
 }
 
 void akmc_mlp_launch_grad(const float *X, const float *T, const int *idx, int M, const float *p, const uint16_t *w1t,
-                          const uint16_t *w2t, const uint16_t *w3t, const uint16_t *w2r, const uint16_t *w3r, float *P,
-                          double *part, hipStream_t s)
+                          const uint16_t *w2t, const uint16_t *w3t, const uint16_t *w2r, const uint16_t *w3r,
+                          void *rows, float *P, double *part, float *g, hipStream_t s)
 {
-    k_mlp_grad<<<akmc_mlp_grad_blocks(M), kB, 0, s>>>(X, T, idx, M, p, w1t, w2t, w3t, w2r, w3r, P, part);
+    const int tiles = (M + 15) / 16, nchunk = akmc_mlp_grad_chunks(M);
+    const size_t t = (size_t)tiles * 64 * 4;
+    MlpRows o;
+    o.z1 = (float *)rows;
+    o.z2 = o.z1 + 8 * t;
+    o.r = o.z2 + 8 * t;
+    o.h1 = (uint16_t *)(o.r + t);
+    o.h2 = o.h1 + 8 * t;
+    o.x = o.h2 + 8 * t;
+    k_mlp_rows<<<tiles, 64, 0, s>>>(X, T, idx, M, p, w1t, w2t, w3t, w2r, w3r, o);
+    k_mlp_wgrad<<<kWgPer * nchunk + kWgBias, kWgBlock, 0, s>>>(o, M, nchunk, P, part, g);
 }
 
 void akmc_mlp_launch_update(const float *P, int M, float *g, float *p, float *m1, float *m2, uint16_t *w1t,
@@ -597,9 +619,9 @@ void akmc_mlp_launch_update(const float *P, int M, float *g, float *p, float *m1
 {
     const float b1 = 0.9f, b2 = 0.999f;
     const float c1 = 1.0f - powf(b1, (float)t), c2 = 1.0f - powf(b2, (float)t);
-    k_mlp_update<<<(kParam + kUpd - 1) / kUpd, 4 * kUpd, 0, s>>>(P, akmc_mlp_grad_blocks(M), g, p, m1, m2,
-                                                                 MlpBf16{w1t, w2t, w3t, w2r, w3r}, step, lr, b1, b2,
-                                                                 1.0e-8f, c1, c2, part, 1.0 / M, acc);
+    k_mlp_update<<<(kParam + kUpd - 1) / kUpd, kUpd, 0, s>>>(P, akmc_mlp_grad_chunks(M), g, p, m1, m2,
+                                                             MlpBf16{w1t, w2t, w3t, w2r, w3r}, step, lr, b1, b2,
+                                                             1.0e-8f, c1, c2, part, 1.0 / M, acc);
 }
 
 void akmc_mlp_launch_descriptors(const BatchDev &b, int na, const int *atoms, int nq, const int *qatom,
