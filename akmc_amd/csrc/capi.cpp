@@ -1090,8 +1090,12 @@ int upload(akmc_batch_t b, const double *x, const double *y, const double *z, co
     std::vector<int> ones(b->W, 1), mode(b->W, batch_mode(b));
     HIPCHK(hipMemcpyAsync(b->d.rebuild, ones.data(), b->W * sizeof(int), hipMemcpyHostToDevice, b->stream));
     HIPCHK(hipMemcpyAsync(b->d.active, mode.data(), b->W * sizeof(int), hipMemcpyHostToDevice, b->stream));
-    // a running search's zone does not survive new positions
-    if (b->zflag) HIPCHK(hipMemsetAsync(b->zflag, 0, b->W * sizeof(int), b->stream));
+    // a running search's zone does not survive new positions; neither do the
+    // resident kernel's lists, so its walkers go on through the chain
+    if (b->zflag) {
+        HIPCHK(hipMemsetAsync(b->zflag, 0, b->W * sizeof(int), b->stream));
+        std::fill(b->hzflag.begin(), b->hzflag.end(), 0);
+    }
     if (b->search_alloc) {
         HIPCHK(hipMemcpyAsync(b->s.X, x, A * sizeof(double), hipMemcpyHostToDevice, b->stream));
         HIPCHK(hipMemcpyAsync(b->s.X + A, y, A * sizeof(double), hipMemcpyHostToDevice, b->stream));

@@ -1,0 +1,55 @@
+"""Calls that change a running search's inputs between chunks of micro-steps:
+the search goes on with the new inputs, whichever kernels advance it.
+
+The end of a FIRE relax is compared with a force call of the whole cell at
+its positions: FP64, the same terms in another order, 1e-11.
+"""
+import numpy as np
+import pytest
+
+from akmc_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+CU = W.SC_CU
+ONE = [("Cu", "Cu", CU["eps"], CU["a"], CU["n"], CU["m"], CU["c"])]
+
+
+def _field():
+    from akmc_amd import lib as L
+    f = L.Field(L.sc_potentials_text(ONE, 2 * CU["a"]))
+    f.set_precision(64)
+    return L, f
+
+
+def _frozen(c, nfree):
+    frozen = np.ones(c.n, np.int32)
+    frozen[np.argsort(W.site_distances(c, c.vacancies[0]), kind="stable")[:nfree]] = 0
+    return frozen
+
+
+def _check(f, c, pos, force, energy, free):
+    ref = f.calculate_forces(pos.copy(), c.types, c.lat, stress=False)
+    assert np.abs(force - ref["force"])[:, free].max() < 1e-11
+    assert abs(energy - ref["energy"]["total"]) < 1e-11 * abs(ref["energy"]["total"])
+
+
+def test_new_positions_under_a_running_search():
+    L, f = _field()
+    cells = [W.sc_cell(4, 4, 5, n_vac=1, jitter=0.02, seed=s) for s in (1, 2)]
+    frozen = [_frozen(c, 60) for c in cells]
+    b = L.Batch(f, cells)
+    b.set_frozen(frozen)
+    b.start_relax(L.relax_defaults(maxIter=40, maxTimeStep=0.003, initTimeStep=0.002))
+    b.run(10, sync_every=5)
+    calls = [s["force_calls"] for s in b.status()]
+    assert all(k == calls[0] for k in calls) and 0 < calls[0] <= 10
+    moved = [W.sc_cell(4, 4, 5, n_vac=1, jitter=0.03, seed=s) for s in (3, 4)]
+    moved = [W.Cell(m.pos, c.types, c.lat) for m, c in zip(moved, cells)]
+    b.upload(moved)
+    b.run(200, sync_every=13)
+    st, pos, frc = b.status(), b.positions(), b.download()[1]
+    for w, c in enumerate(moved):
+        assert st[w]["done"] == 1 and st[w]["force_calls"] > calls[w]
+        fixed = frozen[w] == 1
+        assert np.array_equal(pos[w][:, fixed], c.pos[:, fixed])
+        _check(f, c, pos[w], frc[w], st[w]["energy"], ~fixed)
