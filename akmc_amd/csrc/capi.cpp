@@ -1979,7 +1979,19 @@ int akmc_batch_set_frozen(akmc_batch_t b, const int *frozen)
 {
     if (!b || !frozen) return fail(AKMC_EINVAL, "bad arguments");
     TRY(search_alloc(b));
-    HIPCHK(hipMemcpy((void *)b->s.frozen, frozen, b->A * sizeof(int), hipMemcpyHostToDevice));
+    HIPCHK(hipMemcpyAsync((void *)b->s.frozen, frozen, b->A * sizeof(int), hipMemcpyHostToDevice, b->stream));
+    // a search under way whose free atoms change starts over with its zone,
+    // and on the chain: the resident kernel's lists and fixed parts are those
+    // of its old free atoms, and its buffers hold AKMC_RES_FREE of them
+    const int fresh = AKMC_ZONE_ON | AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64 | AKMC_ZONE_RESET, one = 1;
+    for (int w = 0; w < b->W; ++w) {
+        const int off = b->hw[w].off, n = b->hw[w].n;
+        if (!(b->hzflag[w] & AKMC_ZONE_ON) || std::equal(frozen + off, frozen + off + n, b->hfrozen.begin() + off))
+            continue;
+        b->hzflag[w] = fresh;
+        HIPCHK(hipMemcpyAsync(b->zflag + w, &fresh, sizeof(int), hipMemcpyHostToDevice, b->stream));
+        HIPCHK(hipMemcpyAsync(b->d.rebuild + w, &one, sizeof(int), hipMemcpyHostToDevice, b->stream));
+    }
     std::copy(frozen, frozen + b->A, b->hfrozen.begin());
     return upload_active(b, nullptr);
 }

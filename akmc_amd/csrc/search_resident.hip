@@ -654,6 +654,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *ar
     if (L.ws.kind == WK_IDLE || L.ws.state == ST_DONE) return;
     const WalkerDev W = load_uniform(b.walkers + wid);
     const int nf = s.nact[wid];
+    if (nf < 1 || nf > kFree) return;  // (the host admits no such walker)
     const double h2 = b.field->half_skin2;
     int nz = b.r.n[wid], evals32 = 0, eok = b.r.eok[wid];
     if (nz >= 0) {

@@ -53,3 +53,30 @@ def test_new_positions_under_a_running_search():
         fixed = frozen[w] == 1
         assert np.array_equal(pos[w][:, fixed], c.pos[:, fixed])
         _check(f, c, pos[w], frc[w], st[w]["energy"], ~fixed)
+
+
+@pytest.mark.parametrize("nfree", [20, 64, 300])
+def test_new_frozen_mask_under_a_running_search(nfree):
+    """Fewer free atoms, a few more, and more than a resident walker takes,
+    for one of two walkers; the other keeps its mask."""
+    L, f = _field()
+    cells = [W.sc_cell(4, 4, 6, n_vac=1, jitter=0.02, seed=s) for s in (1, 2)]
+    frozen = [_frozen(c, 60) for c in cells]
+    b = L.Batch(f, cells)
+    b.set_frozen(frozen)
+    b.start_relax(L.relax_defaults(maxIter=40, maxTimeStep=0.003, initTimeStep=0.002))
+    b.run(10, sync_every=5)
+    part = b.positions()
+    assert (b.zone()[2] & 16).all()
+    frozen[0] = _frozen(cells[0], nfree)
+    b.set_frozen(frozen)
+    b.run(300, sync_every=13)
+    flags = b.zone()[2]
+    assert not flags[0] & 16 and flags[1] & 16
+    st, pos, frc = b.status(), b.positions(), b.download()[1]
+    for w, c in enumerate(cells):
+        assert st[w]["done"] == 1
+        fixed = frozen[w] == 1
+        assert np.array_equal(pos[w][:, fixed], part[w][:, fixed])
+        assert np.abs(pos[w] - part[w])[:, ~fixed].max() > 1e-4
+        _check(f, c, pos[w], frc[w], st[w]["energy"], ~fixed)
