@@ -8,6 +8,7 @@
 #include <cstdio>
 #include <cstring>
 #include <fstream>
+#include <memory>
 #include <sstream>
 #include <string>
 #include <vector>
@@ -1524,17 +1525,17 @@ int load_walkers(akmc_batch_t b, const int *walkers, const double *x0, const dou
     const size_t A = b->A;
     TRY(wait_staging(b->stage_ev, b->stage_pending));
     std::vector<LoadItem> items;
-    size_t dwords = 0, iwords = 0;
+    size_t dwords = 0, iwords = 0, total = 0;
+    for (int w = 0; w < b->W; ++w)
+        if (!walkers || walkers[w]) total += b->hw[w].n;
+    std::unique_ptr<int[]> acts(new int[total]);  // the free-atom lists (global ids), walker after walker
     for (int w = 0; w < b->W; ++w) {
         if (walkers && !walkers[w]) continue;
         const int off = b->hw[w].off, n = b->hw[w].n;
-        if (frozen) std::copy(frozen + off, frozen + off + n, b->hfrozen.begin() + off);
-        // the free-atom list (global ids)
-        const int *fr = b->hfrozen.data() + off;
-        int *act = b->hact.data() + off, m = 0;
+        const int *fr = frozen ? frozen + off : b->hfrozen.data() + off;
+        int *act = acts.get() + iwords, m = 0;
         for (int i = 0; i < n; ++i)
             if (!fr[i]) act[m++] = off + i;
-        b->hnact[w] = m;
         LoadItem it{};
         it.walker = w;
         it.has_x = x0 ? 1 : 0;
@@ -1554,7 +1555,7 @@ int load_walkers(akmc_batch_t b, const int *walkers, const double *x0, const dou
     int *I = (int *)(base + ibytes + dbytes);
     for (const LoadItem &it : items) {
         const int w = it.walker, off = b->hw[w].off, n = b->hw[w].n, m = it.nact;
-        const int *act = b->hact.data() + off;
+        const int *act = acts.get() + it.ints;
         double *nw = D + it.dbl;
         double nn = 0.0;
         for (int c = 0; c < 3; ++c)
@@ -1570,6 +1571,14 @@ int load_walkers(akmc_batch_t b, const int *walkers, const double *x0, const dou
             for (int c = 0; c < 3; ++c)
                 std::memcpy(nw + 3 * (size_t)m + (size_t)c * n, x0 + c * A + off, n * sizeof(double));
         std::memcpy(I + it.ints, act, m * sizeof(int));
+    }
+    // every walker's data are good: the host's masks and lists become those
+    // the device gets
+    for (const LoadItem &it : items) {
+        const int off = b->hw[it.walker].off, n = b->hw[it.walker].n;
+        if (frozen) std::copy(frozen + off, frozen + off + n, b->hfrozen.begin() + off);
+        std::copy(acts.get() + it.ints, acts.get() + it.ints + it.nact, b->hact.begin() + off);
+        b->hnact[it.walker] = it.nact;
     }
     std::memcpy(base, items.data(), ibytes);
     HIPCHK(hipMemcpyAsync(b->stage_dev, b->stage_pin, ibytes + dbytes + nbytes, hipMemcpyHostToDevice, b->stream));
@@ -1996,12 +2005,18 @@ int akmc_batch_set_frozen(akmc_batch_t b, const int *frozen)
     return upload_active(b, nullptr);
 }
 
+static int check_relax_method(const akmc_relax_params *p)
+{
+    if (p->method != AKMC_RELAX_FIRE && p->method != AKMC_RELAX_FIRE2 && p->method != AKMC_RELAX_NONE)
+        return fail(AKMC_EINVAL, "relax method %d is not one of AKMC_RELAX_FIRE, _FIRE2, _NONE", p->method);
+    return AKMC_SUCCESS;
+}
+
 int akmc_batch_start_relax(akmc_batch_t b, const int *walkers, const akmc_relax_params *p)
 {
     if (!b || !p) return fail(AKMC_EINVAL, "bad arguments");
     TRY(search_alloc(b));
-    if (p->method != AKMC_RELAX_FIRE && p->method != AKMC_RELAX_FIRE2 && p->method != AKMC_RELAX_NONE)
-        return fail(AKMC_EINVAL, "relax method %d is not one of AKMC_RELAX_FIRE, _FIRE2, _NONE", p->method);
+    TRY(check_relax_method(p));
     RelaxParamsDev &r = b->s.rp;
     r.normTol = p->normTol;
     r.forceTol = p->forceTol;
@@ -2669,6 +2684,7 @@ int akmc_batch_start_relax_at(akmc_batch_t b, const int *walkers, const double *
                               const akmc_relax_params *p)
 {
     if (!b || !p) return fail(AKMC_EINVAL, "bad arguments");
+    TRY(check_relax_method(p));  // before the masks of running walkers change
     TRY(search_alloc(b));
     const size_t A = b->A;
     TRY(for_runs(b, walkers, [&](size_t off, size_t n) {

@@ -80,3 +80,28 @@ def test_new_frozen_mask_under_a_running_search(nfree):
         assert np.array_equal(pos[w][:, fixed], part[w][:, fixed])
         assert np.abs(pos[w] - part[w])[:, ~fixed].max() > 1e-4
         _check(f, c, pos[w], frc[w], st[w]["energy"], ~fixed)
+
+
+def test_refused_start_leaves_masks_alone():
+    """A start refused for one walker's zero mode, with masks that would let
+    the walkers run resident, changes no walker's mask: the relax after it
+    moves the atoms that were free before."""
+    L, f = _field()
+    cells = [W.sc_cell(5, 5, 5, n_vac=1, jitter=0.02, seed=s) for s in (1, 2)]
+    frozen = [_frozen(c, 300) for c in cells]
+    b = L.Batch(f, cells)
+    b.set_frozen(frozen)
+    modes = [np.ones((3, cells[0].n)), np.zeros((3, cells[1].n))]
+    with pytest.raises(L.AkmcError, match="zero start mode"):
+        b.start_dimer(modes, frozen_per_walker=[_frozen(c, 60) for c in cells])
+    with pytest.raises(L.AkmcError, match="relax method"):
+        b.start_relax_at(None, frozen=np.concatenate([_frozen(c, 60) for c in cells]),
+                         params=L.relax_defaults(method=7))
+    b.start_relax(L.relax_defaults(maxIter=20, maxTimeStep=0.003, initTimeStep=0.002))
+    b.run(300, sync_every=13)
+    st, pos, frc = b.status(), b.positions(), b.download()[1]
+    for w, c in enumerate(cells):
+        assert st[w]["done"] == 1
+        moved = np.abs(pos[w] - c.pos).max(0) > 0
+        assert np.array_equal(moved, frozen[w] == 0)
+        _check(f, c, pos[w], frc[w], st[w]["energy"], frozen[w] == 0)
