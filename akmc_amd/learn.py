@@ -124,12 +124,26 @@ class MLP:
     def standardize(self, X):
         return (np.asarray(X, np.float32) - self.mean) * self.scale
 
+    def _inputs(self, X):
+        """(X, mean, scale) as the library takes them: rows of 48 with 48
+        means and scales, applied on the device; anything else goes through
+        standardize(), which broadcasts or raises ValueError, and must come
+        out as rows of 48 (no scaling is left then)."""
+        X, mean, scale = _f32(X), _f32(self.mean), _f32(self.scale)
+        if X.ndim != 2 or X.shape[1] != 48 or mean.shape != (48,) or scale.shape != (48,):
+            X = _f32(self.standardize(X))
+            if X.ndim != 2 or X.shape[1] != 48:
+                raise ValueError(f"inputs must be rows of 48 features, got shape {X.shape}")
+            return X, None, None
+        return X, _fp(mean), _fp(scale)
+
     def train(self, X, T, epochs=20, batch=4096, lr=1e-3, seed=0):
         """Adam on standardised inputs; returns the per-epoch loss."""
-        X, T = _f32(X), _f32(T)
-        mean, scale = _f32(self.mean), _f32(self.scale)  # applied on the device
+        (X, mean, scale), T = self._inputs(X), _f32(T)
+        if T.size != 3 * X.shape[0]:
+            raise ValueError(f"{X.shape[0]} rows need as many targets of 3, got shape {T.shape}")
         hist = np.zeros(epochs)
-        L.check(L.load().akmc_mlp_train_scaled(self._h, _fp(X), _fp(mean), _fp(scale), _fp(T), X.shape[0],
+        L.check(L.load().akmc_mlp_train_scaled(self._h, _fp(X), mean, scale, _fp(T), X.shape[0],
                                                int(epochs), int(min(batch, self.max_rows)), float(lr), int(seed),
                                                hist.ctypes.data_as(C.POINTER(C.c_double))))
         return hist
@@ -141,9 +155,9 @@ class MLP:
         return ms[0], ms[1]
 
     def predict(self, X):
-        X, mean, scale = _f32(X), _f32(self.mean), _f32(self.scale)
+        X, mean, scale = self._inputs(X)
         Y = np.zeros((X.shape[0], 3), np.float32)
-        L.check(L.load().akmc_mlp_forward_scaled(self._h, _fp(X), _fp(mean), _fp(scale), X.shape[0], _fp(Y)))
+        L.check(L.load().akmc_mlp_forward_scaled(self._h, _fp(X), mean, scale, X.shape[0], _fp(Y)))
         return Y
 
 
