@@ -36,7 +36,7 @@
 namespace {
 
 constexpr int kFree = AKMC_RES_FREE, kSlots = AKMC_RES_SLOTS, kCand = AKMC_RES_CAND;
-constexpr int kBitWords = 6784;  // hit words of a list build: free atoms x candidate wavefronts
+constexpr int kBitWords = 6784;  // hit words of a list build's strip: free atoms x candidate wavefronts
 constexpr int kFreeLanes = 16;   // lanes per free atom's list
 constexpr int kFreeIlp = 5;      // list entries in flight per lane: two batches for a bulk list of 155
 constexpr int kFzLanes = 4;      // lanes (mask words) per frozen slot
@@ -255,7 +255,10 @@ __device__ __attribute__((noinline)) bool res_build(const ResArgs *args, int nf)
     }
     const int ncw = (nc + 63) / 64;
     __syncthreads();
-    if (nc > kCand || nf * ncw > kBitWords) return false;
+    if (nc > kCand) return false;
+    // the hit words of this many free atoms fit at a time (106 with every
+    // candidate's worth; a 6 A region's 75 atoms always)
+    const int strip = min(nf, (kBitWords / ncw) & ~(kFzLanes - 1));
     // every candidate against every free atom: its mask (frozen candidates)
     // and, by ballot, the free atoms' hit words over the candidates.  FP32
     // distances with a margin above their rounding (coordinates of up to L/2,
@@ -273,29 +276,42 @@ __device__ __attribute__((noinline)) bool res_build(const ResArgs *args, int nf)
     const float L0 = float(W.L[0]), L1 = float(W.L[1]), L2 = float(W.L[2]);
     const float i0 = float(W.invL[0]), i1 = float(W.invL[1]), i2 = float(W.invL[2]);
     const float margin = 1.0e-6f * float(sqrt(rl2)) * fmaxf(fmaxf(L0, L1), fmaxf(L2, 16.0f));
+    // atom j of the walker in the box's frame, and whether free atom f is
+    // within its radius
+    auto place = [&](int j, float &x, float &y, float &z, float &lim) {
+        const int i = W.off + j;
+        double xd = b.x[i] - bc[0], yd = b.y[i] - bc[1], zd = b.z[i] - bc[2];
+        min_image(xd, yd, zd, W);
+        x = float(xd);
+        y = float(yd);
+        z = float(zd);
+        const bool fr = s.frozen[i] != 0;
+        lim = float(fr ? rz2 : rl2) + margin;
+        return fr;
+    };
+    auto within = [&](int j, float x, float y, float z, float lim, int f) {
+        float dx = x - gx[f], dy = y - gy[f], dz = z - gz[f];
+        dx -= L0 * rintf(dx * i0);
+        dy -= L1 * rintf(dy * i1);
+        dz -= L2 * rintf(dz * i2);
+        return dx * dx + dy * dy + dz * dz <= lim && L.fid[f] != j;
+    };
     int nz = 0, nfree = 0;
     for (int c0 = 0; c0 < nc; c0 += kBlock) {
         const int c = c0 + tid;
         const bool has = c < nc;
-        const int j = has ? cand[c] : 0, i = W.off + j;
-        double xd = b.x[i] - bc[0], yd = b.y[i] - bc[1], zd = b.z[i] - bc[2];
-        min_image(xd, yd, zd, W);
-        const float x = float(xd), y = float(yd), z = float(zd);
-        const bool fr = s.frozen[i] != 0;
-        const float lim = float(fr ? rz2 : rl2) + margin;
+        const int j = has ? cand[c] : 0;
+        float x, y, z, lim;
+        const bool fr = place(j, x, y, z, lim);
         unsigned long long m[kFzLanes] = {};
         const int word = (c0 >> 6) + wave;
         for (int f0 = 0; f0 < nf; f0 += kFzLanes) {
 #pragma unroll
             for (int q = 0; q < kFzLanes; ++q) {
                 const int f = f0 + q < nf ? f0 + q : 0;
-                float dx = x - gx[f], dy = y - gy[f], dz = z - gz[f];
-                dx -= L0 * rintf(dx * i0);
-                dy -= L1 * rintf(dy * i1);
-                dz -= L2 * rintf(dz * i2);
-                const bool hit = has && f0 + q < nf && dx * dx + dy * dy + dz * dz <= lim && L.fid[f] != j;
+                const bool hit = has && f0 + q < nf && within(j, x, y, z, lim, f);
                 const unsigned long long bal = __ballot(hit);
-                if (lane == 0 && word < ncw && f0 + q < nf) bits[f * ncw + word] = bal;
+                if (lane == 0 && word < ncw && f0 + q < strip) bits[f * ncw + word] = bal;
                 m[q] |= (unsigned long long)hit << (f0 >> 2);
             }
         }
@@ -312,7 +328,7 @@ __device__ __attribute__((noinline)) bool res_build(const ResArgs *args, int nf)
                 L.fslot[fi] = uint16_t(sl);
                 R.fslot[w * kFree + fi] = uint16_t(sl);
             }
-            b.zmark[i] = 1;
+            b.zmark[W.off + j] = 1;
         }
         nz += tot;
         nfree += totf;
@@ -320,17 +336,35 @@ __device__ __attribute__((noinline)) bool res_build(const ResArgs *args, int nf)
     }
     if (nz > kSlots) return false;
     // the free atoms' lists from their hit words, one (atom, word) per thread
-    for (int t = tid; t < nf * ncw; t += kBlock) {
-        const int f = t / ncw, wd = t - f * ncw;
-        const unsigned long long *bw = bits + f * ncw;
-        int at = 0;
-        for (int v = 0; v < wd; ++v) at += __popcll(bw[v]);
-        uint16_t *fl = R.flist + ((size_t)w * kFree + f) * R.fcap;
-        for (unsigned long long m = bw[wd]; m; m &= m - 1ull, ++at)
-            if (at < R.fcap) fl[at] = cand[64 * wd + __ffsll((long long)m) - 1];
-        if (wd == ncw - 1) {
-            R.fcnt[w * kFree + f] = at < R.fcap ? at : R.fcap;
-            if (at > R.fcap) atomicOr(b.overflow, AKMC_OV_LIST);
+    for (int s0 = 0; s0 < nf; s0 += strip) {
+        const int ns = min(strip, nf - s0);
+        if (s0 > 0) {  // the words of the next strip; its members' slots are in cand
+            __syncthreads();
+            for (int c0 = 0; c0 < nc; c0 += kBlock) {
+                const int c = c0 + tid, word = (c0 >> 6) + wave;
+                const bool has = c < nc && cand[c] != 0xFFFF;
+                const int j = has ? R.slot[(size_t)w * kSlots + cand[c]] : 0;
+                float x, y, z, lim;
+                (void)place(j, x, y, z, lim);
+                for (int f = 0; f < ns; ++f) {
+                    const unsigned long long bal = __ballot(has && within(j, x, y, z, lim, s0 + f));
+                    if (lane == 0 && word < ncw) bits[f * ncw + word] = bal;
+                }
+            }
+            __syncthreads();
+        }
+        for (int t = tid; t < ns * ncw; t += kBlock) {
+            const int k = t / ncw, wd = t - k * ncw, f = s0 + k;
+            const unsigned long long *bw = bits + k * ncw;
+            int at = 0;
+            for (int v = 0; v < wd; ++v) at += __popcll(bw[v]);
+            uint16_t *fl = R.flist + ((size_t)w * kFree + f) * R.fcap;
+            for (unsigned long long m = bw[wd]; m; m &= m - 1ull, ++at)
+                if (at < R.fcap) fl[at] = cand[64 * wd + __ffsll((long long)m) - 1];
+            if (wd == ncw - 1) {
+                R.fcnt[w * kFree + f] = at < R.fcap ? at : R.fcap;
+                if (at > R.fcap) atomicOr(b.overflow, AKMC_OV_LIST);
+            }
         }
     }
     // the order frozen slots are served in: classes of the number of free
