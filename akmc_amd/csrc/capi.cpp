@@ -1351,18 +1351,18 @@ BatchDev step_dev(akmc_batch_t b)
     return d;
 }
 
-// the kernels of one force evaluation of the chain, with the fixed parts of
-// the resident walkers it serves; j >= 0: the kernel timer's events of a
-// chunk's step j
-void enqueue_chain(akmc_batch_t b, const BatchDev &d, int res, int j)
+// the kernels of one force evaluation of the chain; base: with the fixed
+// parts of resident walkers; sums: with the walker sums; j: the chunk's step,
+// for the kernel timer's events
+void enqueue_chain(akmc_batch_t b, const BatchDev &d, bool base, bool sums, int j)
 {
     // FP64 pair terms run when a walker may ask for them: verification or
     // the closing FP64 energy of a relax
     const int prec = batch_mode(b) | ((b->s.verify_nl > 0 || b->s.final64) ? 2 : 0);
     const FieldDev &hf = b->f->host;
     for (int ph = 0; ph < 2; ++ph) akmc_launch_phase(d, hf, prec, 0, ph, b->stream);
-    if (res) akmc_launch_res_base(d, hf, b->stream);
-    if (j >= 0 && b->ktimer && (prec & 1) && hf.kind == 0) {
+    if (base) akmc_launch_res_base(d, hf, b->stream);
+    if (b->ktimer && (prec & 1) && hf.kind == 0) {
         (void)hipEventRecord(b->kev[0][j], b->stream);
         akmc_launch_phase(d, hf, 1, 0, 2, b->stream);
         (void)hipEventRecord(b->kev[1][j], b->stream);
@@ -1370,41 +1370,34 @@ void enqueue_chain(akmc_batch_t b, const BatchDev &d, int res, int j)
     } else {
         akmc_launch_phase(d, hf, prec, 0, 2, b->stream);
     }
-    if (res < 2) akmc_launch_phase(d, hf, prec, 0, 3, b->stream);
+    if (sums) akmc_launch_phase(d, hf, prec, 0, 3, b->stream);
 }
-
-// Micro-steps between two runs of the chain when every running walker is
-// resident.  The chain is ten kernels that then have nothing to do (about
-// 40 us); a search waits for it once, at the start of its FP64 verification.
-constexpr int kResidentSteps = 9;
 
 // some running walker relaxes by plain FIRE with every atom free and fits the
 // relax kernel (part of SearchDev, so that a captured graph is for one answer)
 bool relax_fire(akmc_batch_t b) { return b->s.fire_on != 0; }
 
-// the kernels of a chunk of micro-steps, res as resident_mode
+// The kernels of a chunk of micro-steps, res as resident_mode.  A resident
+// walker needs the chain once, on its first micro-step, and a walker starts
+// between chunks: one chain evaluation serves those of a chunk, one resident
+// launch takes all its micro-steps, and the chain goes on for the other
+// walkers alone.  With zones off the chain evaluates every atom on every
+// step; the kernel timer times a chain launch of every step.
 void enqueue_steps(akmc_batch_t b, int steps, int res)
 {
     const BatchDev d = step_dev(b);
-    // walkers that need the chain take it on every step; with zones off the
-    // chain evaluates every atom on every step, and a search still waits as
-    // it does with zones on
-    const bool fire = relax_fire(b);
-    const int runs = res == 2 && !b->ktimer ? (steps + kResidentSteps - 1) / kResidentSteps : steps;
-    for (int j = 0, done = 0; j < runs; ++j) {
-        const int k = (steps - done) / (runs - j), launches = b->zone_on ? 1 : k;
-        for (int l = 0; l < launches; ++l) {
-            enqueue_chain(b, d, res, done + l);
-            if (res)
-                akmc_launch_search_resident(b->W, b->f->host, b->res_args, k / launches, 1, l == 0, b->stream);
-            // walkers of tens of thousands of atoms: 1024-thread state machines
-            if (res < 2) {
-                if (fire) akmc_launch_relax_fire(d, b->s, b->stream);
-                if (b->logic_wide) akmc_launch_search_logic_wide(d, b->s, b->stream);
-                else akmc_launch_search_logic(d, b->s, b->stream);
-            }
+    const bool fire = relax_fire(b), every = !b->zone_on || b->ktimer;
+    for (int j = 0; j < steps; ++j) {
+        if (res == 2 && j > 0 && !every) break;
+        enqueue_chain(b, d, res && j == 0, res < 2, j);
+        // walkers of tens of thousands of atoms: 1024-thread state machines
+        if (res < 2) {
+            if (fire) akmc_launch_relax_fire(d, b->s, b->stream);
+            if (b->logic_wide) akmc_launch_search_logic_wide(d, b->s, b->stream);
+            else akmc_launch_search_logic(d, b->s, b->stream);
         }
-        done += k;
+        if (res && (j == 0 || every))
+            akmc_launch_search_resident(b->W, b->f->host, b->res_args, every ? 1 : steps, 1, j == 0, b->stream);
     }
 }
 

@@ -6,8 +6,8 @@
 // its free atoms.  A frozen atom's density and pair energy are a part from
 // frozen neighbours, fixed for the whole search, and a part from the free
 // atoms in reach.  The chain (list build, all-atom passes) evaluates a
-// walker once per precision at its start and k_res_base keeps the fixed
-// parts; from then on an evaluation visits
+// walker once, on its first micro-step, and k_res_base keeps the fixed parts
+// of both precisions; from then on an evaluation visits
 //   - the free atoms' own neighbours (densities, then forces), and
 //   - per frozen atom of the zone, the free atoms in reach (a bit mask),
 // about 35,000 pairs for the 75 free atoms of a 6 A region against 160,000
@@ -669,10 +669,9 @@ __device__ __attribute__((noinline)) void res_step(const ResArgs *args, int nf)
     if (threadIdx.x == 0) L.ws = w;
 }
 
-// Micro-steps of resident walkers, one workgroup each.  A walker whose full
-// evaluation in its precision is pending has had it from the chain that ran
-// before a service launch; one that comes to need it later (a search
-// entering FP64 verification) waits for the next service launch.
+// Micro-steps of resident walkers, one workgroup each.  service: the chain
+// has just run, and with it k_res_base for the walkers on their first
+// micro-step; from then on a walker needs nothing from outside.
 template <int KIND>
 __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *args, int nsteps, int logic, int service)
 {
@@ -704,11 +703,10 @@ __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *ar
         const int mode = step == 0 ? b.active[wid]
                                    : (L.ws.kind == WK_VERIFY || L.ws.state == ST_R_E64) ? 2 : s.default_mode;
         const int prec = mode == 2 ? 1 : 0;
-        const int full = prec ? AKMC_ZONE_FULL64 : AKMC_ZONE_FULL32;
-        if (flags & full) {
+        if (flags & (AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64)) {
             if (step > 0 || !service) break;
-            flags &= ~full;
-            eok &= ~(1 << prec);
+            flags &= ~(AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64);
+            eok = 0;
         }
         bool moved = nz < 0;
         for (int f = tid; f < nf; f += kBlock) {
@@ -835,19 +833,20 @@ __device__ inline void res_base_atoms(const BatchDev &b, const WalkerDev &W, con
 }
 
 // The parts of every atom's density and pair energy that come from frozen
-// neighbours, for the resident walkers the chain evaluates on this step
-// (once per search and precision; kBaseSplit workgroups per walker)
+// neighbours, in both precisions, for the resident walkers on their first
+// micro-step (kBaseSplit workgroups per walker).  A search goes over to FP64
+// at its verification; with these parts at hand it does so without waiting
+// for an evaluation of the chain.
 template <int KIND>
 __global__ void __launch_bounds__(kBaseBlock) k_res_base(BatchDev b)
 {
     __shared__ SCPairDev tab[KIND == 1 ? 1 : kResSpec * kResSpec];
     const int w = blockIdx.x, mode = b.active[w], f = b.zflag[w];
-    if (mode == 0 || !(f & AKMC_ZONE_RES)) return;
-    if (!b.zone_off && !(f & (mode == 2 ? AKMC_ZONE_FULL64 : AKMC_ZONE_FULL32))) return;
+    if (mode == 0 || !(f & AKMC_ZONE_RES) || !(f & (AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64))) return;
     if constexpr (KIND != 1) stage_sc_table(*b.field, tab);
     const WalkerDev W = b.walkers[w];
-    if (mode == 2) res_base_atoms<double, KIND>(b, W, tab);
-    else res_base_atoms<float, KIND>(b, W, tab);
+    res_base_atoms<float, KIND>(b, W, tab);
+    res_base_atoms<double, KIND>(b, W, tab);
 }
 
 __global__ void k_leave_resident(BatchDev b)
