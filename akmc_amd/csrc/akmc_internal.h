@@ -26,6 +26,8 @@
 // its FULL bits then ask the chain of list and pair kernels for one
 // evaluation of all its atoms in that precision
 #define AKMC_ZONE_RES 16
+// a search walker's flags at its start on the chain
+#define AKMC_ZONE_FRESH (AKMC_ZONE_ON | AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64 | AKMC_ZONE_RESET)
 // capacities of a resident walker: free atoms, zone atoms, atoms of the
 // cell, candidates of its list build
 #define AKMC_RES_FREE 256
@@ -341,7 +343,7 @@ struct WalkerState {
     double eb2, eb2_64, b2_maxd2;
     int b2_new, b2_status, b2_calls, b2_iters;
     int fire_done;  // k_relax_fire advanced the walker on this micro-step
-    int too_big;  // the walker does not fit the resident kernel's capacities
+    int left;  // its lists do not fit the resident kernel: the chain advances it
 };
 
 struct SearchDev {
@@ -386,8 +388,9 @@ struct ResArgs {
 };
 void akmc_launch_search_resident(int nwalkers, const FieldDev &hf, const ResArgs *args, int nsteps, int logic,
                                  int service, hipStream_t st);
-// every resident walker goes over to the chain (fresh zone, full evaluations)
-void akmc_launch_leave_resident(const BatchDev &b, hipStream_t st);
+// the first list build of freshly started resident walkers; one that does not
+// fit goes over to the chain
+void akmc_launch_res_admit(int nwalkers, const FieldDev &hf, const ResArgs *args, hipStream_t st);
 // 0 general pair table, 1 one species pair with n = 9, m = 6, 2 every
 // species pair present with n = 9, m = 6
 int akmc_sc_kind(const FieldDev &hf);

@@ -165,14 +165,13 @@ struct akmc_batch_s {
     bool logic_wide = false;
     int *zflag = nullptr, *zmark = nullptr, *zlist = nullptr, *nz = nullptr;
     std::vector<int> hzflag;
-    // resident searches (search_resident.hip): their lists, off for good once
-    // a walker has not fit them, and whether the captured graph is for a batch
-    // whose running walkers are all resident
+    // resident searches (search_resident.hip): their buffers (res_none: no
+    // memory for them, so every walker takes the chain)
     ResidentDev r{};
-    bool res_off = false;
+    bool res_none = false;
+    int *zf_pin = nullptr;            // zflag after the last starts (pinned)
     ResArgs *res_args = nullptr;      // device copy of the descriptors its kernel
     ResArgs res_host{};               // reads, and what it holds
-    int nmax = 0;
     int graph_res = 0;
     // kernel variants of the search micro-steps' Sutton-Chen passes:
     // (lanes, unroll, staged) of pass 1, of pass 2, then of the FP64 passes
@@ -742,7 +741,6 @@ int batch_build(akmc_field_t f, int W, const int *natoms, const double *lat, akm
         int nmax = 0;
         for (int w = 0; w < W; ++w) nmax = std::max(nmax, natoms[w]);
         d.nb16 = (f->kind == 0 && f->min_image && nmax <= 65535) ? 1 : 0;
-        b->nmax = nmax;
         // above this size a 256-thread workgroup loops 64 times over a
         // walker's atoms per vector operation of its state machine
         constexpr int kWideLogicAtoms = 16384;
@@ -936,6 +934,7 @@ void batch_free(akmc_batch_t b)
             if (e) (void)hipEventDestroy(e);
     if (b->hws_pin) (void)hipHostFree(b->hws_pin);
     if (b->ov_pin) (void)hipHostFree(b->ov_pin);
+    if (b->zf_pin) (void)hipHostFree(b->zf_pin);
     if (b->gat_pin) (void)hipHostFree(b->gat_pin);
     if (b->gat_dev) (void)hipFree(b->gat_dev);
     if (b->desc_dev) (void)hipFree(b->desc_dev);
@@ -1093,16 +1092,15 @@ int upload(akmc_batch_t b, const double *x, const double *y, const double *z, co
     HIPCHK(hipMemcpyAsync(b->d.active, mode.data(), b->W * sizeof(int), hipMemcpyHostToDevice, b->stream));
     // a running search's zone does not survive new positions; neither do the
     // resident kernel's lists, so its walkers go on through the chain
-    if (b->zflag) {
-        HIPCHK(hipMemsetAsync(b->zflag, 0, b->W * sizeof(int), b->stream));
-        std::fill(b->hzflag.begin(), b->hzflag.end(), 0);
-    }
+    if (b->zflag) HIPCHK(hipMemsetAsync(b->zflag, 0, b->W * sizeof(int), b->stream));
     if (b->search_alloc) {
         HIPCHK(hipMemcpyAsync(b->s.X, x, A * sizeof(double), hipMemcpyHostToDevice, b->stream));
         HIPCHK(hipMemcpyAsync(b->s.X + A, y, A * sizeof(double), hipMemcpyHostToDevice, b->stream));
         HIPCHK(hipMemcpyAsync(b->s.X + 2 * A, z, A * sizeof(double), hipMemcpyHostToDevice, b->stream));
     }
     HIPCHK(hipStreamSynchronize(b->stream));
+    if (b->zflag)
+        for (int w = 0; w < b->W; ++w) b->hzflag[w] = b->zf_pin[w] = 0;
     return AKMC_SUCCESS;
 }
 
@@ -1205,6 +1203,8 @@ int search_alloc(akmc_batch_t b)
     TRY(upload_active(b, nullptr));
     HIPCHK(hipHostMalloc((void **)&b->hws_pin, b->W * sizeof(WalkerState), hipHostMallocDefault));
     HIPCHK(hipHostMalloc((void **)&b->ov_pin, sizeof(int), hipHostMallocDefault));
+    HIPCHK(hipHostMalloc((void **)&b->zf_pin, b->W * sizeof(int), hipHostMallocDefault));
+    std::fill(b->zf_pin, b->zf_pin + b->W, 0);
     HIPCHK(hipHostMalloc((void **)&b->st_pin, b->W * sizeof(StartItem), hipHostMallocDefault));
     TRY(dalloc(b, &b->st_dev, b->W));
     HIPCHK(hipEventCreateWithFlags(&b->stage_ev, hipEventDisableTiming));
@@ -1229,49 +1229,50 @@ bool zone_usable(akmc_batch_t b)
     return b->zflag && h.kind == 0 && !h.eam && h.min_image;
 }
 
-// bytes of a resident walker's lists
-size_t resident_bytes(akmc_batch_t b)
-{
-    return AKMC_RES_SLOTS * 36 + AKMC_RES_FREE * (30 + 2 * (size_t)b->d.maxnb) + 64;
-}
-
-// searches may run in the resident kernel: zones apply, and the walkers,
-// the field's pair table and the lists' memory are within its capacities
-bool resident_usable(akmc_batch_t b)
-{
-    constexpr size_t kMaxBytes = (size_t)8 << 30;
-    return zone_usable(b) && !b->res_off && b->f->host.nspec <= 4 && b->nmax <= AKMC_RES_ATOMS &&
-           resident_bytes(b) * b->W <= kMaxBytes;
-}
-
-// a search of m free atoms of the walker w runs there
+// a search of walker w runs in the resident kernel, as far as the host can
+// tell: a rule on the walker and its field alone, so that its results do not
+// depend on the batch it is in (the device then tries its first list build,
+// k_res_admit)
 bool resident_walker(akmc_batch_t b, int w)
 {
-    const int m = b->hnact[w];
-    return m > 0 && m < b->hw[w].n && m <= AKMC_RES_FREE && resident_usable(b);
+    const int m = b->hnact[w], n = b->hw[w].n;
+    return zone_usable(b) && !b->res_none && b->f->host.nspec <= 4 && m > 0 && m < n && m <= AKMC_RES_FREE &&
+           n <= AKMC_RES_ATOMS;
 }
 
+// the buffers of the resident walkers; where there is no memory for them
+// (some 200 KB a walker) every walker of the batch takes the chain
 int ensure_resident(akmc_batch_t b)
 {
-    if (b->r.on) return AKMC_SUCCESS;
-    const size_t W = b->W, A = b->A;
+    if (b->r.on || b->res_none) return AKMC_SUCCESS;
+    const size_t W = b->W, A = b->A, had = b->allocs.size();
     ResidentDev r{};
     r.fcap = b->d.maxnb;
-    TRY(dalloc(b, &r.n, W));
-    TRY(dalloc(b, &r.slot, W * AKMC_RES_SLOTS));
-    TRY(dalloc(b, &r.mask, W * AKMC_RES_SLOTS * 4));
-    TRY(dalloc(b, &r.task, W * AKMC_RES_SLOTS));
-    TRY(dalloc(b, &r.fslot, W * AKMC_RES_FREE));
-    TRY(dalloc(b, &r.flist, W * AKMC_RES_FREE * r.fcap));
-    TRY(dalloc(b, &r.fcnt, W * AKMC_RES_FREE));
-    TRY(dalloc(b, &r.ref, W * 3 * AKMC_RES_FREE));
-    TRY(dalloc(b, &r.eout, W * 4));
-    TRY(dalloc(b, &r.eok, W));
-    for (int p = 0; p < 2; ++p) {
-        TRY(dalloc(b, &r.base_rho[p], A));
-        TRY(dalloc(b, &r.base_ep[p], A));
+    auto alloc = [&]() {
+        TRY(dalloc(b, &r.n, W));
+        TRY(dalloc(b, &r.slot, W * AKMC_RES_SLOTS));
+        TRY(dalloc(b, &r.mask, W * AKMC_RES_SLOTS * 4));
+        TRY(dalloc(b, &r.task, W * AKMC_RES_SLOTS));
+        TRY(dalloc(b, &r.fslot, W * AKMC_RES_FREE));
+        TRY(dalloc(b, &r.flist, W * AKMC_RES_FREE * r.fcap));
+        TRY(dalloc(b, &r.fcnt, W * AKMC_RES_FREE));
+        TRY(dalloc(b, &r.ref, W * 3 * AKMC_RES_FREE));
+        TRY(dalloc(b, &r.eout, W * 4));
+        TRY(dalloc(b, &r.eok, W));
+        for (int p = 0; p < 2; ++p) {
+            TRY(dalloc(b, &r.base_rho[p], A));
+            TRY(dalloc(b, &r.base_ep[p], A));
+        }
+        return dalloc(b, &b->res_args, 1);
+    };
+    if (alloc() != AKMC_SUCCESS) {
+        (void)hipGetLastError();
+        for (size_t k = had; k < b->allocs.size(); ++k) (void)hipFree(b->allocs[k]);
+        b->allocs.resize(had);
+        b->res_args = nullptr;
+        b->res_none = true;
+        return AKMC_SUCCESS;
     }
-    TRY(dalloc(b, &b->res_args, 1));
     r.on = 1;
     b->r = r;
     return AKMC_SUCCESS;
@@ -1298,7 +1299,7 @@ int sync_res_args(akmc_batch_t b)
 // and the resident kernel, 2 every running walker is resident
 int resident_mode(akmc_batch_t b)
 {
-    if (!b->r.on || b->res_off) return 0;
+    if (!b->r.on) return 0;
     int res = 0, other = 0;
     for (int w = 0; w < b->W; ++w) {
         const WalkerState &ws = b->hws[w];
@@ -1339,7 +1340,7 @@ BatchDev step_dev(akmc_batch_t b)
     }
     if (zone_usable(b) && (b->zone_on || b->r.on)) {
         d.zone_off = b->zone_on ? 0 : 1;
-        if (!b->res_off) d.r = b->r;
+        d.r = b->r;
         d.zfrozen = b->s.frozen;
         d.zflag = b->zflag;
         d.zmark = b->zmark;
@@ -1445,6 +1446,7 @@ int start_walkers(akmc_batch_t b, const int *walkers, int kind, double dt0, doub
 {
     TRY(wait_staging(b->st_ev, b->st_pending));
     int k = 0;
+    bool resident = false;
     for (int w = 0; w < b->W; ++w) {
         if (walkers && !walkers[w]) continue;
         WalkerState ws{};
@@ -1462,11 +1464,11 @@ int start_walkers(akmc_batch_t b, const int *walkers, int kind, double dt0, doub
         const int m = b->hnact[w];
         StartItem &it = b->st_pin[k++];
         it.walker = w;
-        it.zflag = (m > 0 && m < b->hw[w].n) ? (AKMC_ZONE_ON | AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64 | AKMC_ZONE_RESET)
-                                             : 0;
-        if (resident_walker(b, w)) {
-            TRY(ensure_resident(b));
+        it.zflag = (m > 0 && m < b->hw[w].n) ? AKMC_ZONE_FRESH : 0;
+        if (resident_walker(b, w)) TRY(ensure_resident(b));
+        if (resident_walker(b, w)) {  // (not without memory)
             it.zflag |= AKMC_ZONE_RES;
+            resident = true;
         }
         it.active = batch_mode(b);
         it.pad = 0;
@@ -1478,11 +1480,19 @@ int start_walkers(akmc_batch_t b, const int *walkers, int kind, double dt0, doub
     HIPCHK(hipMemcpyAsync(b->st_dev, b->st_pin, k * sizeof(StartItem), hipMemcpyHostToDevice, b->stream));
     HIPCHK(hipEventRecord(b->st_ev, b->stream));
     b->st_pending = true;
-    akmc_launch_start_walkers(b->d, b->s, b->st_dev, k, b->zflag, b->hv_on ? b->harvested : nullptr, b->r.on ? b->r.n : nullptr,
-                              b->stream);
+    akmc_launch_start_walkers(b->d, b->s, b->st_dev, k, b->zflag, b->hv_on ? b->harvested : nullptr,
+                              b->r.on ? b->r.n : nullptr, b->stream);
     akmc_launch_probe_init(b->d, b->s, b->stream);
+    if (resident) {
+        TRY(sync_res_args(b));
+        akmc_launch_res_admit(b->W, b->f->host, b->res_args, b->stream);
+    }
     HIPCHK(hipGetLastError());
-    if (!b->inflight) HIPCHK(hipStreamSynchronize(b->stream));
+    HIPCHK(hipMemcpyAsync(b->zf_pin, b->zflag, b->W * sizeof(int), hipMemcpyDeviceToHost, b->stream));
+    if (!b->inflight) {  // else the chunk's wait reads them
+        HIPCHK(hipStreamSynchronize(b->stream));
+        std::copy(b->zf_pin, b->zf_pin + b->W, b->hzflag.begin());
+    }
     return AKMC_SUCCESS;
 }
 
@@ -1985,17 +1995,20 @@ int akmc_batch_set_frozen(akmc_batch_t b, const int *frozen)
     // a search under way whose free atoms change starts over with its zone,
     // and on the chain: the resident kernel's lists and fixed parts are those
     // of its old free atoms, and its buffers hold AKMC_RES_FREE of them
-    const int fresh = AKMC_ZONE_ON | AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64 | AKMC_ZONE_RESET, one = 1;
+    const int fresh = AKMC_ZONE_FRESH, one = 1;
+    std::vector<int> changed;
     for (int w = 0; w < b->W; ++w) {
         const int off = b->hw[w].off, n = b->hw[w].n;
         if (!(b->hzflag[w] & AKMC_ZONE_ON) || std::equal(frozen + off, frozen + off + n, b->hfrozen.begin() + off))
             continue;
-        b->hzflag[w] = fresh;
+        changed.push_back(w);
         HIPCHK(hipMemcpyAsync(b->zflag + w, &fresh, sizeof(int), hipMemcpyHostToDevice, b->stream));
         HIPCHK(hipMemcpyAsync(b->d.rebuild + w, &one, sizeof(int), hipMemcpyHostToDevice, b->stream));
     }
     std::copy(frozen, frozen + b->A, b->hfrozen.begin());
-    return upload_active(b, nullptr);
+    TRY(upload_active(b, nullptr));  // (waits for the stream)
+    for (int w : changed) b->hzflag[w] = b->zf_pin[w] = fresh;
+    return AKMC_SUCCESS;
 }
 
 static int check_relax_method(const akmc_relax_params *p)
@@ -2187,23 +2200,18 @@ int akmc_batch_run_wait(akmc_batch_t b, int *steps_done, int *running)
                 b->klaunches += 1;
             }
         std::memcpy(b->hws.data(), b->hws_pin, b->W * sizeof(WalkerState));
+        for (int w = 0; w < b->W; ++w)  // its lists have outgrown the resident kernel
+            if (b->hws[w].left) b->hzflag[w] &= ~AKMC_ZONE_RES;
         if (b->hv_on) b->hv_last = b->hv_inflight;
     } else {
         HIPCHK(hipStreamSynchronize(b->stream));  // starts queued since the launch
     }
     // walkers started behind the chunk have not run yet
-    for (const auto &p : b->started_inflight) b->hws[p.first] = p.second;
-    b->started_inflight.clear();
-    // a walker that does not fit the resident kernel takes every walker of
-    // the batch back to the chain
-    bool too_big = false;
-    for (int w = 0; w < b->W; ++w) too_big |= b->hws[w].too_big != 0;
-    if (too_big && !b->res_off) {
-        akmc_launch_leave_resident(step_dev(b), b->stream);
-        HIPCHK(hipGetLastError());
-        b->res_off = true;
-        for (int &f : b->hzflag) f &= ~AKMC_ZONE_RES;
+    for (const auto &p : b->started_inflight) {
+        b->hws[p.first] = p.second;
+        b->hzflag[p.first] = b->zf_pin[p.first];  // whether it fits the resident kernel
     }
+    b->started_inflight.clear();
     for (int w = 0; w < b->W; ++w) run += b->hws[w].kind != WK_IDLE && b->hws[w].state != ST_DONE;
     if (steps_done) *steps_done = k;
     if (running) *running = run;

@@ -669,9 +669,21 @@ __device__ __attribute__((noinline)) void res_step(const ResArgs *args, int nf)
     if (threadIdx.x == 0) L.ws = w;
 }
 
+// the walker goes over to the chain: a fresh zone, full evaluations first
+__device__ inline void leave(const BatchDev &b, const SearchDev &s, int w)
+{
+    b.zflag[w] = AKMC_ZONE_FRESH;
+    b.rebuild[w] = 1;
+    s.ws[w].left = 1;
+}
+
 // Micro-steps of resident walkers, one workgroup each.  service: the chain
 // has just run, and with it k_res_base for the walkers on their first
-// micro-step; from then on a walker needs nothing from outside.
+// micro-step; from then on a walker needs nothing from outside.  nsteps 0:
+// only the first list build of the walkers just started, at the probes of
+// their first micro-step, so that a walker that does not fit is on the chain
+// before that step.  (Not a kernel of its own: LDS that out-of-line functions
+// share between kernels is no longer addressed directly.)
 template <int KIND>
 __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *args, int nsteps, int logic, int service)
 {
@@ -695,6 +707,18 @@ __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *ar
         res_offsets<KIND>(b.r.fcnt + wid * kFree, nf);
     }
     for (int f = tid; f < nf; f += kBlock) L.fid[f] = uint16_t(s.act[W.off + f] - W.off);
+    if (nsteps == 0) {
+        if (nz >= 0) return;
+        for (int f = tid; f < nf; f += kBlock) {
+            const int i = s.act[W.off + f];
+            L.fx[f] = b.x[i];
+            L.fy[f] = b.y[i];
+            L.fz[f] = b.z[i];
+        }
+        __syncthreads();
+        if (!res_build<KIND>(args, nf) && tid == 0) leave(b, s, wid);
+        return;
+    }
     bool loaded = false, too_big = false;  // loaded: the zone's records are in the pool
     for (int step = 0; step < nsteps; ++step) {
         __syncthreads();
@@ -776,9 +800,9 @@ __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *ar
     if (tid == 0) {
         b.zflag[wid] = flags;
         b.r.eok[wid] = eok;
-        if (too_big) L.ws.too_big = 1;
-        if (logic || too_big) s.ws[wid] = L.ws;
+        if (logic) s.ws[wid] = L.ws;
         s.evals32[wid] += evals32;
+        if (too_big) leave(b, s, wid);
     }
 }
 
@@ -849,14 +873,6 @@ __global__ void __launch_bounds__(kBaseBlock) k_res_base(BatchDev b)
     res_base_atoms<double, KIND>(b, W, tab);
 }
 
-__global__ void k_leave_resident(BatchDev b)
-{
-    const int w = blockIdx.x * blockDim.x + threadIdx.x;
-    if (w >= b.W || !(b.zflag[w] & AKMC_ZONE_RES)) return;
-    b.zflag[w] = AKMC_ZONE_ON | AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64 | AKMC_ZONE_RESET;
-    b.rebuild[w] = 1;
-}
-
 }  // namespace
 
 void akmc_launch_res_base(const BatchDev &b, const FieldDev &hf, hipStream_t st)
@@ -879,7 +895,7 @@ void akmc_launch_search_resident(int nwalkers, const FieldDev &hf, const ResArgs
     }
 }
 
-void akmc_launch_leave_resident(const BatchDev &b, hipStream_t st)
+void akmc_launch_res_admit(int nwalkers, const FieldDev &hf, const ResArgs *args, hipStream_t st)
 {
-    k_leave_resident<<<(b.W + 255) / 256, 256, 0, st>>>(b);
+    akmc_launch_search_resident(nwalkers, hf, args, 0, 0, 0, st);
 }

@@ -65,3 +65,78 @@ def test_two_separated_clusters_are_resident():
     f, b = _relax([c], [frozen], 64)
     assert b.zone()[2][0] & 16
     _check(f, b, [c], [frozen], 64)
+
+
+def _scattered(c, n, seed):
+    frozen = np.ones(c.n, np.int32)
+    frozen[np.random.default_rng(seed).choice(c.n, n, replace=False)] = 0
+    return frozen
+
+
+def test_a_walker_that_does_not_fit_leaves_the_others_alone():
+    """A small search beside one whose 200 scattered free atoms reach more
+    than 2048 atoms, and beside a cell past 16383 atoms: the same bits as
+    alone, at the first start and after a restart; only the others are on the
+    chain, and they make a force call a step from their first step on."""
+    from akmc_amd import lib as L
+    small = W.sc_cell(4, 4, 5, n_vac=1, jitter=0.02, seed=1)
+    wide = W.sc_cell(9, 9, 9, n_vac=1, jitter=0.02, seed=2)
+    huge = W.sc_cell(16, 16, 17, n_vac=1, jitter=0.02, seed=3)
+    cells = [small, wide, huge]
+    frozen = [_nearest(small, 60), _scattered(wide, 200, 1), _nearest(huge, 60)]
+    f, alone = _relax([small], [frozen[0]], 32, run=9, sync=9)
+    f, b = _relax(cells, frozen, 32, run=9, sync=9)
+    for again in range(2):
+        st, one = b.status(), alone.status()
+        assert [int(v) & 16 for v in b.zone()[2]] == [16, 0, 0] and alone.zone()[2][0] & 16
+        assert [s["force_calls"] for s in st] == [9, 9, 9]
+        for bb in (b, alone):
+            bb.run(400, sync_every=9)
+        st, one = b.status(), alone.status()
+        assert st[0] == one[0] and st[0]["done"] == 1
+        assert np.array_equal(b.positions()[0], alone.positions()[0])
+        if again == 0:
+            _check(f, b, cells, frozen, 32)
+            for bb in (b, alone):
+                bb.start_relax(L.relax_defaults(maxIter=25, maxTimeStep=0.004, initTimeStep=0.003))
+                bb.run(9, sync_every=9)
+
+
+def _zone(c, pos, frozen, reach):
+    free = np.nonzero(frozen == 0)[0]
+    inz = frozen == 0
+    for i in free:
+        inz |= W.site_distances(W.Cell(pos, c.types, c.lat), pos[:, i]) <= reach
+    return int(inz.sum())
+
+
+def _outgrowing(seed):
+    """16 scattered free atoms of a perfect lattice, displaced: (cell, mask,
+    zone at the start, zone when the farthest one has come back by half the
+    skin, skin)"""
+    c = W.sc_cell(10, 10, 10, n_vac=1, jitter=0.0, seed=4)
+    skin = 1.2
+    frozen = _scattered(c, 16, seed)
+    disp = np.where(frozen == 0, np.random.default_rng(seed).uniform(-0.6, 0.6, (3, c.n)), 0.0)
+    t = 1 - skin / 2 / np.sqrt((disp ** 2).sum(0)).max()
+    reach = 2 * CU["a"] + skin / 2
+    return (W.Cell(c.pos + disp, c.types, c.lat, vacancies=c.vacancies), frozen,
+            _zone(c, c.pos + disp, frozen, reach + 0.01), _zone(c, c.pos + t * disp, frozen, reach - 0.01), skin)
+
+
+def test_a_zone_that_outgrows_the_kernel_goes_on_in_the_chain():
+    """16 scattered free atoms whose zone has at most 2048 atoms at the start
+    of a relax and more when they have come back."""
+    cell, frozen, z0, z1, skin = _outgrowing(20)
+    assert z0 <= 2044 and z1 >= 2060
+    from akmc_amd import lib as L
+    f = L.Field(L.sc_potentials_text(ONE, 2 * CU["a"]))
+    f.set_precision(64)
+    f.set_skin(skin)
+    b = L.Batch(f, [cell])
+    b.set_frozen([frozen])
+    b.start_relax(L.relax_defaults(maxIter=400, maxTimeStep=0.004, initTimeStep=0.003))
+    assert b.zone()[2][0] & 16
+    b.run(3000, sync_every=10)
+    assert not b.zone()[2][0] & 16
+    _check(f, b, [cell], [frozen], 64)
