@@ -169,6 +169,7 @@ struct akmc_batch_s {
     // memory for them, so every walker takes the chain)
     ResidentDev r{};
     bool res_none = false;
+    bool res_on = true;               // akmc_batch_set_resident
     int *zf_pin = nullptr;            // zflag after the last starts (pinned)
     ResArgs *res_args = nullptr;      // device copy of the descriptors its kernel
     ResArgs res_host{};               // reads, and what it holds
@@ -1236,7 +1237,7 @@ bool zone_usable(akmc_batch_t b)
 bool resident_walker(akmc_batch_t b, int w)
 {
     const int m = b->hnact[w], n = b->hw[w].n;
-    return zone_usable(b) && !b->res_none && b->f->host.nspec <= 4 && m > 0 && m < n && m <= AKMC_RES_FREE &&
+    return zone_usable(b) && b->res_on && !b->res_none && b->f->host.nspec <= 4 && m > 0 && m < n && m <= AKMC_RES_FREE &&
            n <= AKMC_RES_ATOMS;
 }
 
@@ -2322,6 +2323,13 @@ int akmc_batch_set_search_zone(akmc_batch_t b, int enable)
     if (!b) return fail(AKMC_EINVAL, "null batch");
     b->zone_on = enable != 0;
     drop_graph(b);
+    return AKMC_SUCCESS;
+}
+
+int akmc_batch_set_resident(akmc_batch_t b, int enable)
+{
+    if (!b) return fail(AKMC_EINVAL, "null batch");
+    b->res_on = enable != 0;
     return AKMC_SUCCESS;
 }
 

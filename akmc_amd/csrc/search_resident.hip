@@ -23,12 +23,16 @@
 // chain's kernels took 293 us (91 us with four wavefronts and lists in
 // global memory); 12 walkers: 41 us against 104 us.
 //
-// Results do not depend on the batch or on when the lists were built.  The
-// FP32 terms summed here span fewer than 2^29 in magnitude and count, so
-// their FP64 sums are exact in any order; the FP64 fixed parts are summed in
-// twice the working precision.  With zones off the chain evaluates every
-// atom on every step and the same kernel follows, so both modes agree bit
-// for bit.
+// A walker's results do not depend on its batch: whether it is resident, when
+// its lists are built and every order of summation follow from the walker
+// alone.  The terms are the chain's, in another order: FP32 density and energy
+// terms span less than 2^29 in magnitude and count at any distance a search
+// meets, so their FP64 sums are the chain's bit for bit; force sums (products
+// with FP64 displacements) and FP64 sums differ in their last bits, and a list
+// built elsewhere along the way would change them too.  The FP64 fixed parts
+// are summed in twice the working precision.  With zones off the chain
+// evaluates every atom on every step and this kernel still advances the
+// walker, so both modes agree bit for bit.
 #define AKMC_LOGIC_BLOCK 512
 #include "search_logic.h"
 #include "sc_pair.h"

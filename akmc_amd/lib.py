@@ -191,6 +191,7 @@ def load() -> C.CDLL:
     L.akmc_batch_set_variant.argtypes = [C.c_void_p, C.c_int, C.c_int]
     L.akmc_batch_set_graphs.argtypes = [C.c_void_p, C.c_int]
     L.akmc_batch_set_search_zone.argtypes = [C.c_void_p, C.c_int]
+    L.akmc_batch_set_resident.argtypes = [C.c_void_p, C.c_int]
     L.akmc_batch_set_logic_block.argtypes = [C.c_void_p, C.c_int]
     L.akmc_batch_time_search_phases.argtypes = [C.c_void_p, C.c_int, C.POINTER(C.c_double)]
     L.akmc_batch_get_zone.argtypes = [C.c_void_p] + [C.POINTER(C.c_int)] * 4
@@ -552,6 +553,10 @@ class Batch:
         """Active zones of the search micro-steps (on by default)."""
         check(load().akmc_batch_set_search_zone(self._h, int(bool(enable))))
 
+    def set_resident(self, enable: bool):
+        """The resident kernel for searches started from now on (on by default)."""
+        check(load().akmc_batch_set_resident(self._h, int(bool(enable))))
+
     def time_search_phases(self, nrep):
         """per-phase ms of one evaluation of the search walkers as the micro-steps run it"""
         ms = np.zeros(4)
@@ -580,7 +585,8 @@ class Batch:
         return tuple(int(x) for x in best), table
 
     def zone(self):
-        """(member [A], size [W], flags [W], active [W]) of the active zones"""
+        """(member [A], size [W], flags [W], active [W]) of the active zones;
+        flags & 16: in the resident kernel"""
         member, size = np.zeros(self.A, np.int32), np.zeros(self.W, np.int32)
         flags, active = np.zeros(self.W, np.int32), np.zeros(self.W, np.int32)
         check(load().akmc_batch_get_zone(self._h, _ip(member), _ip(size), _ip(flags), _ip(active)))

@@ -20,8 +20,8 @@ kmcevents of the reference's example control file), each basin with its
 own de-duplication catalogue, so the rate is a steady state rather than a
 catalogue that saturates as the run goes on.
 Searches evaluate their active zones (the free atoms' forces, the
-densities and energies within the list radius of a free atom), bit for bit
-the results of full evaluations.
+densities and energies within the list radius of a free atom); every other
+atom keeps its values, which no free atom can change.
 Also reported: the plain unbatched GPU dimer (one walker, host-driven
 micro-steps) on the same cells, force evaluations per second, the roofline
 of the search micro-steps' resident kernel, one evaluation of every search

@@ -321,12 +321,23 @@ int akmc_batch_set_graphs(akmc_batch_t b, int enable);
  * steps evaluate forces on the free atoms and densities and energies on the
  * atoms within the list radius of a free atom; every other atom keeps the
  * values of the walker's first full evaluation since its start, which no
- * free atom can change.  The searches' forces on free atoms, energies and
- * trajectories are bit for bit those of full evaluations; forces on frozen
- * atoms are not re-evaluated during a search (the optimizers zero them), so
- * akmc_batch_download after a search returns their values from its start:
- * call akmc_batch_forces first for fresh ones. */
+ * free atom can change.  Searches have the same bits with zones on and off;
+ * with zones off the pair kernels evaluate every atom on every micro-step.
+ * Forces on frozen atoms are not re-evaluated during a search with zones on
+ * (the optimizers zero them), so akmc_batch_download after a search returns
+ * their values from its start: call akmc_batch_forces first for fresh ones. */
 int akmc_batch_set_search_zone(akmc_batch_t b, int enable);
+/* enable (default) or disable the resident kernel for searches started from
+ * now on (no counterpart in the reference).  It advances searches on the same
+ * fields whose walker has at most 16383 atoms, at most 256 of them free, at
+ * most 2048 atoms in their reach and 4096 around their bounding box, on
+ * fields of at most 4 species; a walker that does not fit, or outgrows it,
+ * takes the batch's pair kernels.  The rule looks at the walker and its field
+ * alone.  Resident searches take energies and free-atom forces from the
+ * resident kernel with zones on and off: the same terms as the pair kernels'
+ * (FP32 or FP64 alike) added in another order.  With it off, searches with
+ * zones off are full evaluations throughout, and zones on gives their bits. */
+int akmc_batch_set_resident(akmc_batch_t b, int enable);
 /* Workgroup size of the walker state machines: 256 threads, or 1024 (the
  * default for batches whose largest walker has at least 16 384 atoms).  No
  * counterpart in the reference; the two differ only in the order of their
@@ -342,7 +353,7 @@ int akmc_batch_time_search_phases(akmc_batch_t b, int nrep, double ms[4]);
 /* The active zones (no counterpart in the reference: inspection): member[A]
  * 1 for the atoms in their walker's zone, size[W] zone sizes, flags[W] the
  * zone bits (1 on, 2 / 4 a full FP32 / FP64 evaluation pending, 8 reset
- * pending), active[W] the walkers' evaluation modes (0 none, 1 FP32 pair
+ * pending, 16 in the resident kernel), active[W] the walkers' evaluation modes (0 none, 1 FP32 pair
  * terms, 2 FP64); any pointer may be NULL. */
 int akmc_batch_get_zone(akmc_batch_t b, int *member, int *size, int *flags, int *active);
 /* Kernel variants of the search micro-steps' Sutton-Chen passes (no
