@@ -2354,7 +2354,39 @@ int akmc_batch_set_search_variant(akmc_batch_t b, const int v[9])
     return AKMC_SUCCESS;
 }
 
-static int time_search_phases_prec(akmc_batch_t b, int prec, int nrep, double ms[4]);
+static int time_search_phases_prec(akmc_batch_t b, int prec, int nrep, bool chain, double ms[4]);
+
+// The variants are those of the chain's pair kernels.  What they do for a
+// resident walker is the evaluation of all its atoms on its first micro-step,
+// so that is what they are timed on: the flags that ask for it are set while
+// the object lives.
+struct FullEvaluations {
+    akmc_batch_t b;
+    std::vector<int> flags;
+    explicit FullEvaluations(akmc_batch_t b_) : b(b_) {}
+    int set()
+    {
+        flags.resize(b->W);
+        HIPCHK(hipMemcpyAsync(flags.data(), b->zflag, b->W * sizeof(int), hipMemcpyDeviceToHost, b->stream));
+        HIPCHK(hipStreamSynchronize(b->stream));
+        std::vector<int> full = flags;
+        for (int &f : full)
+            if (f & AKMC_ZONE_RES) f |= AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64;
+        HIPCHK(hipMemcpyAsync(b->zflag, full.data(), b->W * sizeof(int), hipMemcpyHostToDevice, b->stream));
+        HIPCHK(hipStreamSynchronize(b->stream));
+        return AKMC_SUCCESS;
+    }
+    // resident walkers' flags as they were (the chain keeps the others')
+    ~FullEvaluations()
+    {
+        std::vector<int> now(flags.size());
+        const size_t n = now.size() * sizeof(int);
+        if (!n || hipMemcpy(now.data(), b->zflag, n, hipMemcpyDeviceToHost) != hipSuccess) return;
+        for (size_t w = 0; w < now.size(); ++w)
+            if (now[w] & AKMC_ZONE_RES) now[w] = flags[w];
+        (void)hipMemcpy(b->zflag, now.data(), n, hipMemcpyHostToDevice);
+    }
+};
 
 int akmc_batch_autotune_search(akmc_batch_t b, int nrep, int best[9], double ms1[AKMC_NVARIANTS],
                                double ms2[AKMC_NVARIANTS], double ms64[AKMC_NVARIANTS])
@@ -2364,13 +2396,15 @@ int akmc_batch_autotune_search(akmc_batch_t b, int nrep, int best[9], double ms1
     static const int lanes[4] = {1, 2, 4, 8}, unroll[4] = {1, 2, 4, 8};
     const int nv = b->stage_ok ? AKMC_NVARIANTS : AKMC_NVARIANTS / 2;
     double t1[AKMC_NVARIANTS], t2[AKMC_NVARIANTS], ms[4];
+    FullEvaluations full(b);
+    TRY(full.set());
     for (int v = 0; v < AKMC_NVARIANTS; ++v) {
         t1[v] = t2[v] = -1.0;
         if (v >= nv) continue;
         const int sv[9] = {lanes[v / 4 % 4], unroll[v % 4], v / 16, lanes[v / 4 % 4], unroll[v % 4], v / 16, 0, 0, 0};
         TRY(akmc_batch_set_search_variant(b, sv));
-        TRY(akmc_batch_time_search_phases(b, 1, ms));  // first launch of this instantiation
-        TRY(akmc_batch_time_search_phases(b, nrep, ms));
+        TRY(time_search_phases_prec(b, batch_mode(b), 1, true, ms));  // first launch of this instantiation
+        TRY(time_search_phases_prec(b, batch_mode(b), nrep, true, ms));
         t1[v] = ms[1];
         t2[v] = ms[2];
     }
@@ -2388,8 +2422,8 @@ int akmc_batch_autotune_search(akmc_batch_t b, int nrep, int best[9], double ms1
         if (v >= nv) continue;
         const int sv[9] = {0, 0, 0, 0, 0, 0, lanes[v / 4 % 4], unroll[v % 4], v / 16};
         TRY(akmc_batch_set_search_variant(b, sv));
-        TRY(time_search_phases_prec(b, 2 | 4, 1, ms));
-        TRY(time_search_phases_prec(b, 2 | 4, nrep, ms));
+        TRY(time_search_phases_prec(b, 2 | 4, 1, true, ms));
+        TRY(time_search_phases_prec(b, 2 | 4, nrep, true, ms));
         t64[v] = ms[1] + ms[2];
         if (t64[v] < t64[k64]) k64 = v;
     }
@@ -2586,17 +2620,18 @@ int akmc_batch_time_search_phases(akmc_batch_t b, int nrep, double ms[4])
 {
     if (!b || nrep <= 0 || !ms) return fail(AKMC_EINVAL, "bad arguments");
     if (!b->search_alloc) return fail(AKMC_EINVAL, "no search has been started");
-    return time_search_phases_prec(b, batch_mode(b), nrep, ms);
+    return time_search_phases_prec(b, batch_mode(b), nrep, false, ms);
 }
 
 // per-phase times of nrep evaluations of the search walkers of precision
-// mask prec (2 | 4: the FP64 passes of mixed steps) at their probes
-static int time_search_phases_prec(akmc_batch_t b, int prec, int nrep, double ms[4])
+// mask prec (2 | 4: the FP64 passes of mixed steps) at their probes; chain:
+// by the pair kernels alone
+static int time_search_phases_prec(akmc_batch_t b, int prec, int nrep, bool chain, double ms[4])
 {
     for (auto &e : b->evp)
         if (!e) HIPCHK(hipEventCreate(&e));
     const BatchDev d = step_dev(b);
-    const int res = resident_mode(b);
+    const int res = chain ? 0 : resident_mode(b);
     TRY(sync_res_args(b));
     for (int ph = 0; ph < 4; ++ph) ms[ph] = 0.0;
     for (int r = 0; r < nrep; ++r) {

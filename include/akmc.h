@@ -365,8 +365,11 @@ int akmc_batch_get_zone(akmc_batch_t b, int *member, int *size, int *flags, int 
  * summation order of the sums they split. */
 int akmc_batch_set_search_variant(akmc_batch_t b, const int v[9]);
 /* Times every variant of each pass on the search walkers at their current
- * probes (akmc_batch_time_search_phases, nrep evaluations each; the FP64
- * variants on the walkers under FP64 verification), keeps the fastest per
+ * probes (nrep evaluations each, as akmc_batch_time_search_phases; walkers in
+ * the resident kernel by the evaluation of all their atoms that the pair
+ * kernels make on their first micro-step, so their frozen atoms' forces are
+ * current afterwards; the FP64 variants on the walkers under FP64
+ * verification), keeps the fastest per
  * part and returns it in best[9] (may be NULL) with the per-variant ms of
  * pass 1, pass 2 and the FP64 passes, indexed like akmc_batch_autotune (any
  * of them NULL).  Call it with searches under way. */

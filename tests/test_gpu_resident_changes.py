@@ -105,3 +105,35 @@ def test_refused_start_leaves_masks_alone():
         moved = np.abs(pos[w] - c.pos).max(0) > 0
         assert np.array_equal(moved, frozen[w] == 0)
         _check(f, c, pos[w], frc[w], st[w]["energy"], frozen[w] == 0)
+
+
+def test_variants_are_timed_on_the_pair_kernels():
+    """autotune_search under resident searches times the pair kernels'
+    evaluation of all the walkers' atoms (the forces it leaves are those of a
+    force call at the probes, frozen atoms included) and changes no search."""
+    from akmc_amd import lib as L
+    f = L.Field(L.sc_potentials_text(ONE, 2 * CU["a"]))
+    cells = [W.sc_cell(4, 4, 6, n_vac=1, jitter=0.02, seed=s) for s in (1, 2)]
+    frozen = [_frozen(c, 60) for c in cells]
+    ends = []
+    for tune in (True, False):
+        b = L.Batch(f, cells)
+        b.set_frozen(frozen)
+        b.start_relax(L.relax_defaults(maxIter=60, maxTimeStep=0.003, initTimeStep=0.002))
+        b.run(30, sync_every=10)
+        flags = b.zone()[2]
+        assert (flags & 16).all()
+        if tune:
+            best, ms = b.autotune_search(2)
+            assert np.array_equal(b.zone()[2], flags) and all(v[0] > 0 and v[1] > 0 for v in ms.values())
+            pos, frc = b.download()
+            for w, c in enumerate(cells):
+                ref = f.calculate_forces(pos[w].copy(), c.types, c.lat, stress=False)
+                assert np.abs(frc[w] - ref["force"]).max() < 2e-5
+        b.run(300, sync_every=10)
+        ends.append((b.positions(), b.status_array()))
+    assert (ends[0][1]["done"] == 1).all()
+    for k in ends[0][1].dtype.names:
+        assert np.array_equal(ends[0][1][k], ends[1][1][k], equal_nan=True), k
+    for p, q in zip(ends[0][0], ends[1][0]):
+        assert np.array_equal(p, q)
