@@ -49,6 +49,7 @@ struct SCCoef {
     T rho_coef;  // (eps c)^2
     T fs_coef;   // n eps
     T fm_coef;   // 0.5 m (eps c)^2
+    T ha2;       // 1 / (2 a^2)
 };
 struct SCPairDev {
     SCCoef<float> f;
@@ -108,7 +109,7 @@ struct FieldDev {
     int dsf_n;
     double dsf_del, dsf_rfld0, dsf_rfld1;
     SCPairDev sc[AKMC_MAXPAIR];
-    int all96;       // every species pair has a Sutton-Chen potential with n = 9, m = 6
+    int all96;       // every species pair has a Sutton-Chen potential with n = 9, m = 6, a > 0
     IonPairDev ion[AKMC_MAXPAIR];
     // tabulated EAM (kind 0 with eam = 1): species pair -> table (-1 none)
     int eam;
@@ -392,7 +393,7 @@ void akmc_launch_search_resident(int nwalkers, const FieldDev &hf, const ResArgs
 // fit goes over to the chain
 void akmc_launch_res_admit(int nwalkers, const FieldDev &hf, const ResArgs *args, hipStream_t st);
 // 0 general pair table, 1 one species pair with n = 9, m = 6, 2 every
-// species pair present with n = 9, m = 6
+// species pair present with n = 9, m = 6, a > 0
 int akmc_sc_kind(const FieldDev &hf);
 // FIRE iterations of the walkers relaxing with every atom free
 void akmc_launch_relax_fire(const BatchDev &b, const SearchDev &s, hipStream_t st);

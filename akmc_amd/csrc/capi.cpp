@@ -458,9 +458,9 @@ void build_tables(akmc_field_t f)
                 const SCPot &s = f->sc[k];
                 p.on = 1;
                 p.d = {s.a, s.n, s.m, s.eps, (s.eps * s.c) * (s.eps * s.c), s.n * s.eps,
-                       0.5 * s.m * (s.eps * s.c) * (s.eps * s.c)};
+                       0.5 * s.m * (s.eps * s.c) * (s.eps * s.c), 0.5 / (s.a * s.a)};
                 p.f = {(float)p.d.a, (float)p.d.n, (float)p.d.m, (float)p.d.eps, (float)p.d.rho_coef,
-                       (float)p.d.fs_coef, (float)p.d.fm_coef};
+                       (float)p.d.fs_coef, (float)p.d.fm_coef, (float)p.d.ha2};
                 auto as_int = [](double e) { return (e >= 0 && e <= 64 && std::floor(e) == e) ? (int)e : -1; };
                 p.n_int = as_int(s.n);
                 p.m_int = as_int(s.m);
@@ -483,7 +483,8 @@ void build_tables(akmc_field_t f)
             }
         }
     h.all96 = f->kind == 0 && f->eam.empty() ? 1 : 0;
-    for (int k = 0; k < ns * ns; ++k) h.all96 &= h.sc[k].on && h.sc[k].n_int == 9 && h.sc[k].m_int == 6;
+    for (int k = 0; k < ns * ns; ++k)
+        h.all96 &= h.sc[k].on && h.sc[k].n_int == 9 && h.sc[k].m_int == 6 && h.sc[k].d.a > 0.0;
 }
 
 // lanes per atom and gathers in flight of the pair kernels for one cell of n

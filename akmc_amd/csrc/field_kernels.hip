@@ -1227,7 +1227,7 @@ __device__ __forceinline__ void sc_density_atom(const BatchDev &b, const FieldDe
             for (int u = 0; u < U; ++u) {
                 const SCCoef<T> &c = sc_coef<T>(tab[row + (int)pj[u].w]);
                 T ir2, un, um;
-                table_9_6<T>(r2[u], c.a, ir2, un, um);
+                table_9_6<T>(r2[u], c, ir2, un, um);
                 T rh = in[u] ? c.rho_coef * um : T(0);
                 if constexpr (sizeof(T) == 4) asm("" : "+v"(rh));
                 rho += double(rh);
@@ -1411,7 +1411,7 @@ __device__ __forceinline__ void sc_force_atom(const BatchDev &b, const FieldDev 
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const SCCoef<T> &c = sc_coef<T>(tab[row + (int)pj[u].w]);
-                    table_9_6<T>(r2[u], c.a, ir2[u], un[u], um[u]);
+                    table_9_6<T>(r2[u], c, ir2[u], un[u], um[u]);
                     const T fs = c.fs_coef * un[u];
                     T fm;
                     if constexpr (sizeof(T) == 8)
@@ -2308,7 +2308,7 @@ int akmc_sc_kind(const FieldDev &hf)
 {
     if (sc_one(hf)) return 1;
     for (int k = 0; k < hf.nspec * hf.nspec; ++k)
-        if (!hf.sc[k].on || hf.sc[k].n_int != 9 || hf.sc[k].m_int != 6) return 0;
+        if (!hf.sc[k].on || hf.sc[k].n_int != 9 || hf.sc[k].m_int != 6 || !(hf.sc[k].d.a > 0.0)) return 0;
     return 2;
 }
 

@@ -43,6 +43,7 @@ constexpr int kFree = AKMC_RES_FREE, kSlots = AKMC_RES_SLOTS, kCand = AKMC_RES_C
 constexpr int kBitWords = 6784;  // hit words of a list build's strip: free atoms x candidate wavefronts
 constexpr int kFreeLanes = 16;   // lanes per free atom's list
 constexpr int kFreeIlp = 5;      // list entries in flight per lane: two batches for a bulk list of 155
+constexpr int kFreeIlp64 = 2;    // FP64 entries: five spill 356 bytes of registers (alloy searches 33.3 -> 29.6 ms)
 constexpr int kFzLanes = 4;      // lanes (mask words) per frozen slot
 constexpr int kFzIlp = 2;        // free atoms of a mask word in flight per lane
 constexpr int kClass = 8;        // frozen slots are served in classes of similar reach
@@ -132,7 +133,7 @@ __device__ inline void pair_terms(const double (&r2)[U], const bool (&in)[U], co
         pow_9_6<T, U>(u2, rt, un, um);
     } else if constexpr (KIND == 2) {
 #pragma unroll
-        for (int u = 0; u < U; ++u) table_9_6<T>(r2[u], sc_coef<T>(*p[u]).a, ir2[u], un[u], um[u]);
+        for (int u = 0; u < U; ++u) table_9_6<T>(r2[u], sc_coef<T>(*p[u]), ir2[u], un[u], um[u]);
     } else {
 #pragma unroll
         for (int u = 0; u < U; ++u) {
@@ -482,6 +483,7 @@ __device__ __attribute__((noinline)) void res_eval(const ResArgs *args, int nf, 
     const BatchDev b = load_uniform(&args->b);
     const WalkerDev W = load_uniform(b.walkers + blockIdx.x);
     constexpr int prec = sizeof(T) == 8 ? 1 : 0;
+    constexpr int kIlp = sizeof(T) == 8 ? kFreeIlp64 : kFreeIlp;
     const int w = blockIdx.x, tid = threadIdx.x;
     const SCCoef<T> c1 = sc_coef<T>(load_uniform(&b.field->sc[0]));
     const double rc2 = load_uniform(&b.field->rc2);
@@ -540,14 +542,14 @@ __device__ __attribute__((noinline)) void res_eval(const ResArgs *args, int nf, 
     }
     // free atoms: kFreeLanes lanes per list, entries strided over the lanes
     const int g = tid / kFreeLanes, sub = tid % kFreeLanes;
-    constexpr int kGroups = kBlock / kFreeLanes, kBatch = kFreeLanes * kFreeIlp;
+    constexpr int kGroups = kBlock / kFreeLanes, kBatch = kFreeLanes * kIlp;
     const uint16_t *glist = R.flist + (size_t)w * kFree * R.fcap;
     const uint16_t *llist = reinterpret_cast<const uint16_t *>(L.pool + 4 * S);
     const bool lists = lists_fit(L.fofs[nf], S);
     // the slots of entries k, k + kFreeLanes, ... of free atom f (-1: none)
-    auto fetch = [&](int f, int k, int cnt, int (&e)[kFreeIlp]) {
+    auto fetch = [&](int f, int k, int cnt, int (&e)[kIlp]) {
 #pragma unroll
-        for (int u = 0; u < kFreeIlp; ++u) {
+        for (int u = 0; u < kIlp; ++u) {
             const int kk = k + u * kFreeLanes;
             e[u] = -1;
             if (kk < cnt) e[u] = lists ? int(llist[L.fofs[f] + kk]) : int(glist[(size_t)f * R.fcap + kk]);
@@ -559,13 +561,13 @@ __device__ __attribute__((noinline)) void res_eval(const ResArgs *args, int nf, 
         const double xi = L.fx[f], yi = L.fy[f], zi = L.fz[f];
         double rho = 0.0, ep = 0.0;
         for (int k = sub; k < cnt; k += kBatch) {
-            int e[kFreeIlp];
+            int e[kIlp];
             fetch(f, k, cnt, e);
-            double px[kFreeIlp], py[kFreeIlp], pz[kFreeIlp];
-            bool ok[kFreeIlp];
-            const SCPairDev *p[kFreeIlp];
+            double px[kIlp], py[kIlp], pz[kIlp];
+            bool ok[kIlp];
+            const SCPairDev *p[kIlp];
 #pragma unroll
-            for (int u = 0; u < kFreeIlp; ++u) {
+            for (int u = 0; u < kIlp; ++u) {
                 ok[u] = e[u] >= 0;
                 const int j = ok[u] ? e[u] : sl;
                 px[u] = rx[j];
@@ -573,7 +575,7 @@ __device__ __attribute__((noinline)) void res_eval(const ResArgs *args, int nf, 
                 pz[u] = rz[j];
                 p[u] = KIND == 1 ? nullptr : L.tab + zt * ns + L.zt[j];
             }
-            add_density<T, KIND, kFreeIlp>(W, rc2, c1, p, xi, yi, zi, px, py, pz, ok, rho, ep);
+            add_density<T, KIND, kIlp>(W, rc2, c1, p, xi, yi, zi, px, py, pz, ok, rho, ep);
         }
         rho = row_sum<kFreeLanes>(rho);
         ep = row_sum<kFreeLanes>(ep);
@@ -598,14 +600,14 @@ __device__ __attribute__((noinline)) void res_eval(const ResArgs *args, int nf, 
         const T isi = rw[kRw * sl];
         double fx = 0.0, fy = 0.0, fz = 0.0;
         for (int k = sub; k < cnt; k += kBatch) {
-            int e[kFreeIlp];
+            int e[kIlp];
             fetch(f, k, cnt, e);
-            double dx[kFreeIlp], dy[kFreeIlp], dz[kFreeIlp], r2[kFreeIlp];
-            T isj[kFreeIlp];
-            bool in[kFreeIlp];
-            const SCPairDev *p[kFreeIlp];
+            double dx[kIlp], dy[kIlp], dz[kIlp], r2[kIlp];
+            T isj[kIlp];
+            bool in[kIlp];
+            const SCPairDev *p[kIlp];
 #pragma unroll
-            for (int u = 0; u < kFreeIlp; ++u) {
+            for (int u = 0; u < kIlp; ++u) {
                 const int j = e[u] >= 0 ? e[u] : sl;
                 dx[u] = xi - rx[j];
                 dy[u] = yi - ry[j];
@@ -616,10 +618,10 @@ __device__ __attribute__((noinline)) void res_eval(const ResArgs *args, int nf, 
                 r2[u] = dx[u] * dx[u] + dy[u] * dy[u] + dz[u] * dz[u];
                 in[u] = e[u] >= 0 && r2[u] <= rc2 && r2[u] > 1.0e-16;
             }
-            T ir2[kFreeIlp], un[kFreeIlp], um[kFreeIlp];
-            pair_terms<T, KIND, kFreeIlp>(r2, in, c1, p, ir2, un, um);
+            T ir2[kIlp], un[kIlp], um[kIlp];
+            pair_terms<T, KIND, kIlp>(r2, in, c1, p, ir2, un, um);
 #pragma unroll
-            for (int u = 0; u < kFreeIlp; ++u) {
+            for (int u = 0; u < kIlp; ++u) {
                 const SCCoef<T> &c = coef_of<T, KIND>(c1, p[u]);
                 const T fs = c.fs_coef * un[u];
                 const T fm = (isi >= T(0) && isj[u] >= T(0)) ? c.fm_coef * (isi + isj[u]) * um[u] : T(0);

@@ -1,0 +1,53 @@
+"""Alloy pairs with n = 9, m = 6 (straight products) in FP64: the error of a
+pair's energy and density against extended precision is that of the same
+products with a correctly rounded division and square root.
+
+A cell of two atoms of different species holds one pair: its vdw energy is
+eps (a/r)^9, its many-body energy -2 sqrt((eps c)^2 (a/r)^6).
+"""
+import numpy as np
+import pytest
+
+from akmc_amd import workloads as W
+
+pytestmark = pytest.mark.gpu
+RC = 7.22
+
+
+def _reference(r2, eps, a, c, T):
+    """the kernels' products in the number type T"""
+    r2, a, eps, c = T(1) * r2.astype(T), T(a), T(eps), T(c)
+    ir2 = T(1) / r2
+    u2 = a * a * ir2
+    u4 = u2 * u2
+    rho = (eps * c) * (eps * c) * (u2 * u4)
+    return T(2) * (T(0.5) * eps * (u4 * u4 * np.sqrt(u2))), -(np.sqrt(rho) + np.sqrt(rho))
+
+
+def test_fp64_table_pairs_round_like_division_and_square_root():
+    from akmc_amd import lib as L
+    rng = np.random.default_rng(8)
+    n = 600
+    r = rng.uniform(2.0, 7.2, n)
+    lat = np.diag([20.0] * 3).reshape(9)
+    cells = []
+    for k in range(n):
+        pos = np.array([[6.0, 6.0 + r[k]], [10.0, 10.0], [10.0, 10.0]])  # r^2 is one rounded product
+        cells.append(W.Cell(np.ascontiguousarray(pos), np.array([0, 1], np.int32), lat, ["Cu", "Ni"]))
+    f = L.Field(L.sc_potentials_text(W.ALLOY_POTS, RC, species=["Cu", "Ni"]))
+    f.set_precision(64)
+    f.set_list_density(0.01)
+    e = L.Batch(f, cells).forces()
+    eps, a, c = [(p[2], p[3], p[6]) for p in W.ALLOY_POTS if {p[0], p[1]} == {"Cu", "Ni"}][0]
+    d = np.array([cl.pos[0, 0] - cl.pos[0, 1] for cl in cells])
+    ld = np.longdouble
+    r2 = d * d
+    exact, plain = _reference(r2, eps, a, c, ld), _reference(r2, eps, a, c, np.float64)
+    for name, k in (("vdw", 0), ("many", 1)):
+        got = np.array([x[name] for x in e])
+        unit = np.spacing(np.abs(exact[k]).astype(np.float64)) / 2
+        err = ((got.astype(ld) - exact[k]) / unit).astype(np.float64)
+        ref = ((plain[k].astype(ld) - exact[k]) / unit).astype(np.float64)
+        print(f"{name}: rms {np.sqrt((err ** 2).mean()):.2f} half-units, plain products {np.sqrt((ref ** 2).mean()):.2f}; "
+              f"worst {np.abs(err).max():.1f}, {np.abs(ref).max():.1f}; {np.mean(got == plain[k]):.3f} equal", flush=True)
+        assert np.sqrt((err ** 2).mean()) <= 1.1 * np.sqrt((ref ** 2).mean())
