@@ -1405,9 +1405,10 @@ __device__ __forceinline__ void sc_force_atom(const BatchDev &b, const FieldDev 
             }
             continue;
         }
-        if constexpr (!ONE && !STRESS) {
+        if constexpr (!ONE) {
             if (F.all96) {
-                // a table of n = 9, m = 6 pairs: straight products, branch-free
+                // a table of n = 9, m = 6 pairs: straight products, branch-free;
+                // with stress too, so that asking for it changes no force
 #pragma unroll
                 for (int u = 0; u < U; ++u) {
                     const SCCoef<T> &c = sc_coef<T>(tab[row + (int)pj[u].w]);
@@ -1429,6 +1430,15 @@ __device__ __forceinline__ void sc_force_atom(const BatchDev &b, const FieldDev 
                     fy += dft * dy[u];
                     fz += dft * dz[u];
                     if constexpr (!WL) ep += double(eh);
+                    if constexpr (STRESS) {
+                        const double h = -0.5 * dft;  // one ordered pair: -(fs-fm)/(2 r^2) r r
+                        s0 += h * dx[u] * dx[u];
+                        s1 += h * dy[u] * dy[u];
+                        s2 += h * dz[u] * dz[u];
+                        s3 += h * dy[u] * dz[u];
+                        s4 += h * dx[u] * dz[u];
+                        s5 += h * dx[u] * dy[u];
+                    }
                 }
                 continue;
             }

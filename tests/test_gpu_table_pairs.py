@@ -51,3 +51,22 @@ def test_fp64_table_pairs_round_like_division_and_square_root():
         print(f"{name}: rms {np.sqrt((err ** 2).mean()):.2f} half-units, plain products {np.sqrt((ref ** 2).mean()):.2f}; "
               f"worst {np.abs(err).max():.1f}, {np.abs(ref).max():.1f}; {np.mean(got == plain[k]):.3f} equal", flush=True)
         assert np.sqrt((err ** 2).mean()) <= 1.1 * np.sqrt((ref ** 2).mean())
+
+
+@pytest.mark.parametrize("bits", [32, 64])
+@pytest.mark.parametrize("shape", [(4, 4, 5), (5, 6, 7), (16, 16, 17)])
+def test_asking_for_stress_changes_no_force(shape, bits):
+    """A wavefront per atom, and 8 lanes; the stress itself against that of
+    the FP64 pair terms (FP32 terms within a few 2^-24: 2e-6 of the largest)."""
+    from akmc_amd import lib as L
+    c = W.sc_cell(*shape, n_vac=2, jitter=0.05, seed=3, two_species=True, a=3.65)
+    f = L.Field(L.sc_potentials_text(W.ALLOY_POTS, RC, species=["Cu", "Ni"]))
+    f.set_precision(bits)
+    plain = f.calculate_forces(c.pos.copy(), c.types, c.lat, stress=False)
+    with_s = f.calculate_forces(c.pos.copy(), c.types, c.lat, stress=True)
+    assert np.array_equal(plain["force"], with_s["force"])
+    for k in ("vdw", "many"):  # (the walker sums with stress add in another order)
+        assert abs(plain["energy"][k] / with_s["energy"][k] - 1) < 1e-13
+    f.set_precision(64)
+    ref = f.calculate_forces(c.pos.copy(), c.types, c.lat, stress=True)
+    assert np.abs(with_s["stress"] - ref["stress"]).max() <= (0 if bits == 64 else 2e-6) * np.abs(ref["stress"]).max()
