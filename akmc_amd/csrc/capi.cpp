@@ -130,6 +130,7 @@ struct akmc_batch_s {
     // the overflow flag.  Small batches move each part in one transfer through
     // pinned memory.
     char *io = nullptr, *io_pin = nullptr;
+    size_t io_pin_n = 0;
     size_t io_q = 0, io_in = 0, io_out = 0, io_end = 0;
     // LDS staging of the many-body pair kernels is possible when every
     // walker's gather records fit one workgroup's LDS
@@ -1029,12 +1030,40 @@ void host_wrap(bool min_image, const double *lat, int n, double *x, double *y, d
     }
 }
 
+// up to this much goes through pinned memory: a 255-atom call is seven
+// pageable copies of 5-15 us otherwise; past it a pageable copy streams as
+// fast as the host can fill a pinned buffer
+constexpr size_t kPinnedIo = (size_t)4 << 20;
+
+// the batch's force calls move their data through its pinned buffer
+bool pinned_io(akmc_batch_t b) { return b->io_end <= kPinnedIo && !b->search_alloc; }
+
+int ensure_io_pin(akmc_batch_t b)
+{
+    if (b->io_pin && b->io_pin_n >= b->io_end) return AKMC_SUCCESS;
+    if (b->io_pin) HIPCHK(hipHostFree(b->io_pin));
+    b->io_pin = nullptr;
+    b->io_pin_n = 0;
+    HIPCHK(hipHostMalloc((void **)&b->io_pin, b->io_end, hipHostMallocDefault));
+    b->io_pin_n = b->io_end;
+    return AKMC_SUCCESS;
+}
+
 int ensure_single(akmc_field_t f, int n, const double *lat)
 {
     bool same = f->single && f->single_n == n && std::memcmp(f->single_lat, lat, sizeof f->single_lat) == 0;
     if (same) return AKMC_SUCCESS;
-    if (f->single) batch_free(f->single);
+    // the pinned buffer (at most kPinnedIo) passes from cell to cell
+    char *pin = nullptr;
+    size_t pin_n = 0;
+    if (f->single) {
+        std::swap(pin, f->single->io_pin);
+        std::swap(pin_n, f->single->io_pin_n);
+        batch_free(f->single);
+    }
     f->single = new akmc_batch_s();
+    f->single->io_pin = pin;
+    f->single->io_pin_n = pin_n;
     int rc = batch_build(f, 1, &n, lat, f->single);
     if (rc != AKMC_SUCCESS) {
         batch_free(f->single);
@@ -1047,17 +1076,6 @@ int ensure_single(akmc_field_t f, int n, const double *lat)
     return AKMC_SUCCESS;
 }
 
-// up to this much goes through pinned memory: a 255-atom call is seven
-// pageable copies of 5-15 us otherwise; past it a pageable copy streams as
-// fast as the host can fill a pinned buffer
-constexpr size_t kPinnedIo = (size_t)4 << 20;
-
-int ensure_io_pin(akmc_batch_t b)
-{
-    if (!b->io_pin) HIPCHK(hipHostMalloc((void **)&b->io_pin, b->io_end, hipHostMallocDefault));
-    return AKMC_SUCCESS;
-}
-
 // wait: returns with the host arrays and the pinned buffer free for reuse (a
 // caller that synchronises the stream itself need not)
 int upload(akmc_batch_t b, const double *x, const double *y, const double *z, const int *type, const double *q,
@@ -1067,7 +1085,7 @@ int upload(akmc_batch_t b, const double *x, const double *y, const double *z, co
     int ns = (int)b->f->species.size();
     for (size_t i = 0; i < A; ++i)
         if (type[i] < 0 || type[i] >= ns) return fail(AKMC_EINVAL, "atom %zu: species %d out of range", i, type[i]);
-    if (b->io_end <= kPinnedIo && !b->search_alloc) {
+    if (pinned_io(b)) {
         TRY(ensure_io_pin(b));
         double *px = (double *)b->io_pin;
         std::memcpy(px, x, A * sizeof(double));
@@ -1736,7 +1754,7 @@ int akmc_field_forces(akmc_field_t f, double *x, double *y, double *z, double *f
     akmc_batch_t b = f->single;
     TRY(upload(b, x, y, z, type, charge, false));
     TRY(run_forces(b, stress != nullptr));
-    if (b->io_pin) {
+    if (pinned_io(b)) {
         TRY(fetch_all(b));
         const double *pf = (const double *)(b->io_pin + b->io_out);
         std::memcpy(fx, pf, n * sizeof(double));
@@ -1772,7 +1790,7 @@ int akmc_field_energy(akmc_field_t f, double *x, double *y, double *z, const dou
     d.energy_only = 1;
     akmc_launch_forces_impl(d, f->host, batch_mode(b), 0, b->stream);
     HIPCHK(hipGetLastError());
-    if (b->io_pin) {
+    if (pinned_io(b)) {
         TRY(fetch_all(b));
     } else {
         TRY(check_overflow(b));
