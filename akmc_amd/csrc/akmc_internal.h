@@ -448,6 +448,9 @@ void akmc_mlp_launch_grad(const float *X, const float *T, const int *idx, int M,
 void akmc_mlp_launch_update(const float *P, int M, float *g, float *p, float *m1, float *m2, uint16_t *w1t,
                             uint16_t *w2t, uint16_t *w3t, uint16_t *w2r, uint16_t *w3r, int step, float lr, int t,
                             const double *part, double *acc, hipStream_t s);
+// neighbours within the angular cutoff that a descriptor takes at most (more:
+// AKMC_OV_LIST, possible only with longer lists)
+#define AKMC_DESC_CAP 4096
 // descriptors of nq queries (atom, site, mover): the terms of the na distinct
 // atoms into G [na][32], then the rows X [nq][48] (qslot: a query's atom in
 // the list of distinct ones)

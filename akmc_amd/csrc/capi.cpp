@@ -3170,7 +3170,8 @@ int akmc_batch_descriptors(akmc_batch_t b, int nq, const int *atom, const double
     if (e == hipSuccess) e = hipMemcpyAsync(X, qx, 48 * n * sizeof(float), hipMemcpyDeviceToHost, b->stream);
     if (e == hipSuccess) e = hipStreamSynchronize(b->stream);
     if (e != hipSuccess) return fail(AKMC_EHIP, "descriptors: %s", hipGetErrorString(e));
-    return check_overflow(b);
+    // an overflow of an earlier force call has been reported there
+    return b->d.maxnb > AKMC_DESC_CAP ? check_overflow(b) : AKMC_SUCCESS;
 }
 
 }  // extern "C"

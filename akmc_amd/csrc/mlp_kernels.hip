@@ -415,7 +415,7 @@ __device__ inline float fcut(float r, float rc) { return r < rc ? 0.5f * (__cosf
 // atoms with every mover, so k_atom_descriptors computes them once per atom
 // and k_query_descriptors assembles the queries.
 constexpr float kDescRc = 7.22f, kDescRca = 5.0f;
-constexpr int kDescCap = 4096;  // neighbours inside kDescRca kept in LDS at most
+constexpr int kDescCap = AKMC_DESC_CAP;  // neighbours inside kDescRca kept in LDS at most
 
 // sum over the wavefront, the same bits on every lane
 __device__ inline float wave_sum(float v)
