@@ -729,12 +729,12 @@ __global__ void __launch_bounds__(kBlock) k_nbr_build_cells(BatchDev b)
 // Explicit-image lists (fields without the image convention) hold every
 // (j, S) with |r_i - r_j - S L| <= rc + skin except j == i, S == 0; the shell
 // loop is centred on the nearest image so unwrapped positions are handled.
-// image_hits: one candidate j of atom i over those shells; calls put(entry)
-// for each image inside the list radius and on the pass's side of the near
-// shell, in (sa, sb, sc) ascending order
+// image_hits: one candidate j of atom i over those shells; calls
+// put(entry, near) for each image inside the list radius, in (sa, sb, sc)
+// ascending order; near: inside the near shell
 template <typename Put>
 __device__ inline void image_hits(const BatchDev &b, const WalkerDev &W, int i, int jl, double xi, double yi,
-                                  double zi, double rl2, double rn2, int pass, Put put)
+                                  double zi, double rl2, double rn2, Put put)
 {
     const int j = W.off + jl;
     const double bx = xi - b.x[j], by = yi - b.y[j], bz = zi - b.z[j];
@@ -748,12 +748,13 @@ __device__ inline void image_hits(const BatchDev &b, const WalkerDev &W, int i, 
                 const double dz = bz - sc * W.L[2];
                 const double r2 = dx * dx + dy * dy + dz * dz;
                 const bool near = r2 <= rn2;
-                if (r2 <= rl2 && (pass == 0 ? near : !near)) {
+                if (r2 <= rl2 && !(near && !(rn2 > 0.0))) {
                     if (sa < -7 || sa > 7 || sb < -7 || sb > 7 || sc < -7 || sc > 7) {
                         *b.overflow = 1;
                         continue;
                     }
-                    put(uint32_t(jl) | (uint32_t(sa + 7) << 20) | (uint32_t(sb + 7) << 24) | (uint32_t(sc + 7) << 28));
+                    put(uint32_t(jl) | (uint32_t(sa + 7) << 20) | (uint32_t(sb + 7) << 24) | (uint32_t(sc + 7) << 28),
+                        near);
                 }
             }
         }
@@ -798,7 +799,11 @@ __device__ inline void image_masks(const BatchDev &b, const WalkerDev &W, int i,
 // order, the order of a serial scan, so the list does not depend on
 // scheduling.  Bound by the FP64 distances to 27 images: the 510-ion cell
 // takes 14 us (116 us with one wavefront per atom, whose near and other
-// entries were separate passes, each evaluating every image twice).
+// entries were separate passes, each evaluating every image twice).  Cells
+// that reach more shells hold one candidate per lane or two: its hits are
+// kept from the first sweep (upload and force call of 200 cells of 63 ions:
+// 0.64 ms, 0.95 ms counting near and other hits apart in both sweeps, 0.70 ms
+// before the workgroup per atom).
 __global__ void __launch_bounds__(kBlock) k_nbr_build_images(BatchDev b)
 {
     constexpr int kWaves = kBlock / 64;
@@ -812,7 +817,7 @@ __global__ void __launch_bounds__(kBlock) k_nbr_build_images(BatchDev b)
     const bool one = W.shells[0] == 1 && W.shells[1] == 1 && W.shells[2] == 1;
     const int nchunk = (W.n + 63) / 64;
     const int c0 = wave * nchunk / kWaves, c1 = (wave + 1) * nchunk / kWaves;
-    int at[2] = {0, 0};
+    int at[2] = {0, 0}, first[2] = {0, 0};  // first: the hits of this lane's first candidate
 #pragma unroll 1  // one copy of the distances: both sweeps see the same hits
     for (int sweep = 0; sweep < 2; ++sweep) {
         int sum[2] = {0, 0};
@@ -825,10 +830,17 @@ __global__ void __launch_bounds__(kBlock) k_nbr_build_images(BatchDev b)
                     image_masks(b, W, i, jl, xi, yi, zi, rl2, rn2, hit[0], hit[1], m);
                     cnt[0] = __popc(hit[0]);
                     cnt[1] = __popc(hit[1]);
+                } else if (sweep == 1 && ch == c0) {
+                    cnt[0] = first[0];
+                    cnt[1] = first[1];
                 } else {
-                    for (int p = 0; p < 2; ++p) {
-                        if (p == 0 && !(rn2 > 0.0)) continue;
-                        image_hits(b, W, i, jl, xi, yi, zi, rl2, rn2, p, [&](uint32_t) { ++cnt[p]; });
+                    image_hits(b, W, i, jl, xi, yi, zi, rl2, rn2, [&](uint32_t, bool nr) {
+                        cnt[0] += nr;
+                        cnt[1] += !nr;
+                    });
+                    if (ch == c0) {
+                        first[0] = cnt[0];
+                        first[1] = cnt[1];
                     }
                 }
             }
@@ -837,25 +849,29 @@ __global__ void __launch_bounds__(kBlock) k_nbr_build_images(BatchDev b)
                 sum[1] += cnt[1];
                 continue;
             }
+            int slot[2];
+#pragma unroll
             for (int p = 0; p < 2; ++p) {
                 int incl = cnt[p];
                 for (int o = 1; o < 64; o <<= 1) {
                     const int t = __shfl_up(incl, o);
                     if (lane >= o) incl += t;
                 }
-                int slot = at[p] + incl - cnt[p];
+                slot[p] = at[p] + incl - cnt[p];
                 at[p] += __shfl(incl, 63);
-                if (cnt[p] == 0) continue;
-                if (one) {
+            }
+            if (one) {
+#pragma unroll
+                for (int p = 0; p < 2; ++p)
                     for (uint32_t h = hit[p]; h; h &= h - 1u) {
                         const int k = __ffs((int)h) - 1;
                         const int sa = m[0] + k / 9 - 1, sb = m[1] + k / 3 % 3 - 1, sc = m[2] + k % 3 - 1;
-                        put_nbr(b, i, slot++, uint32_t(jl) | (uint32_t(sa + 7) << 20) | (uint32_t(sb + 7) << 24) |
-                                                  (uint32_t(sc + 7) << 28));
+                        put_nbr(b, i, slot[p]++, uint32_t(jl) | (uint32_t(sa + 7) << 20) | (uint32_t(sb + 7) << 24) |
+                                                     (uint32_t(sc + 7) << 28));
                     }
-                } else {
-                    image_hits(b, W, i, jl, xi, yi, zi, rl2, rn2, p, [&](uint32_t e) { put_nbr(b, i, slot++, e); });
-                }
+            } else if (cnt[0] + cnt[1] > 0) {
+                image_hits(b, W, i, jl, xi, yi, zi, rl2, rn2,
+                           [&](uint32_t e, bool nr) { put_nbr(b, i, nr ? slot[0]++ : slot[1]++, e); });
             }
         }
         if (sweep == 0) {
