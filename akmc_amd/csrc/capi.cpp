@@ -2974,6 +2974,18 @@ int akmc_mlp_forward(akmc_mlp_t m, const float *X, int M, float *Y)
 int akmc_mlp_forward_scaled(akmc_mlp_t m, const float *X, const float *mean, const float *scale, int M, float *Y)
 {
     if (!m || !X || !Y || M < 0 || !mean != !scale) return fail(AKMC_EINVAL, "bad arguments");
+    // a few rows are standardised here: two more copies and a launch take
+    // longer than their arithmetic (1 row 38 us so, 45 us on the device, 1024
+    // rows 53 and 63 us)
+    constexpr int kHostRows = 1024;
+    std::vector<float> few;
+    if (mean && M <= kHostRows) {
+        few.resize((size_t)M * 48);
+        for (int r = 0; r < M; ++r)
+            for (int c = 0; c < 48; ++c) few[(size_t)r * 48 + c] = (X[(size_t)r * 48 + c] - mean[c]) * scale[c];
+        X = few.data();
+        mean = scale = nullptr;
+    }
     TRY(mlp_scaling(m, mean, scale));
     for (int r0 = 0; r0 < M; r0 += m->rows) {
         int n = std::min(m->rows, M - r0);
