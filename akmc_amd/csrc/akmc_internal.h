@@ -373,7 +373,9 @@ struct SearchDev {
     int final64;                      // relaxes end with one FP64 energy evaluation
     int fire_on;                      // k_relax_fire runs (the logic kernel leaves its walkers alone)
 };
-// atoms of a walker that k_relax_fire takes at most
+// atoms of a walker that k_relax_fire takes at most: four per thread of its
+// 1024 (eight would need 96 of a thread's 128 registers for their forces and
+// velocities alone)
 #define AKMC_FIRE_ATOMS 4096
 
 // after pass 1 of the chain: what frozen neighbours contribute to the

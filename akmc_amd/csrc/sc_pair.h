@@ -39,22 +39,6 @@ __device__ inline float pow_general(float u, float x)
     return r * exp2f((x - xi) * log2f(u));
 }
 
-// u2^(k/2) for an integer k >= 0 by repeated squaring; with k uniform across
-// the wavefront the loop is scalar control flow around the multiplications
-template <typename T>
-__device__ inline T pow_int(T u2, int k)
-{
-    T r = T(1), base = u2;
-    int p = k >> 1;
-    while (p) {
-        if (p & 1) r *= base;
-        base *= base;
-        p >>= 1;
-    }
-    if (k & 1) r *= sqrt(u2);
-    return r;
-}
-
 // square root for the integer powers: the hardware instruction (1 ulp) on
 // the FP32 path, whose arguments (a/r)^2 are normal numbers far from the
 // denormal range the correctly rounded expansion guards; libm on FP64
@@ -201,6 +185,5 @@ __device__ inline void stage_sc_table(const FieldDev &F, SCPairDev *tab)
     for (int w = threadIdx.x; w < nw; w += blockDim.x) dst[w] = src[w];
     __syncthreads();
 }
-
 
 }  // namespace

@@ -5,9 +5,9 @@
 // inside the walker-resident search kernel (search_resident.hip).
 //
 // One workgroup owns one walker.  Every vector operation of the walker is a
-// strided loop of its 256 threads over the walker's atoms (relax) or free
+// strided loop of its threads (kBlock) over the walker's atoms (relax) or free
 // atoms (saddle searches) followed by a fixed-order reduction (wavefront
-// butterfly, then the four wavefront partials in order), so a walker's
+// butterfly, then the wavefronts' partials in order), so a walker's
 // trajectory is bitwise the same whether it runs alone or in a batch of
 // hundreds.  Vectors are FP64 [3][A] arrays (component c of atom i at
 // c*A + i).
@@ -18,16 +18,17 @@
 
 namespace {
 
-// workgroup size of the walker state machines: 256 threads, or 1024 in the
-// wide build of this file (search_kernels_wide.hip) for batches of walkers
-// so large that the strided loops of 256 threads dominate a micro-step
+// workgroup size of the walker state machines: 256 threads in the logic
+// kernel, 1024 in its wide build (search_kernels_wide.hip) for batches of
+// walkers so large that the strided loops of 256 threads dominate a
+// micro-step, 512 in the resident kernel (search_resident.hip)
 #ifndef AKMC_LOGIC_BLOCK
 #define AKMC_LOGIC_BLOCK 256
 #endif
 constexpr int kBlock = AKMC_LOGIC_BLOCK;
 
 // Block-wide sums and maxima in a fixed order: a butterfly over the 64
-// lanes of each wavefront, then the four wavefront partials in order, so
+// lanes of each wavefront, then the wavefronts' partials in order, so
 // every thread gets the same bits and a walker's result does not depend on
 // the rest of the batch.
 constexpr int kWaves = kBlock / 64;
@@ -686,7 +687,7 @@ __device__ __attribute__((always_inline)) double tridiag_kth(int n, const double
 // Full re-orthogonalisation of the Lanczos residual T against q_0 .. q_k
 // with the vectors in LDS: the free atoms' components of q_0 .. q_k and T
 // are loaded once (all loads in flight together), then classical
-// Gram-Schmidt runs twice, each wavefront taking every fourth projection
+// Gram-Schmidt runs twice, the wavefronts taking the projections in turn
 // (a wavefront sum, no block barrier per projection), and T goes back to
 // global memory.  Element e of a vector is component e / nact of free atom
 // e % nact.  Modified Gram-Schmidt in global memory, with k + 1 block

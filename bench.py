@@ -579,8 +579,6 @@ def main():
     ap.add_argument("--sync-every", type=int, default=25,
                     help="micro-steps per device chunk between host checks (refills)")
     ap.add_argument("--walkers", type=int, default=512)
-    ap.add_argument("--roofline-window", type=int, default=100,
-                    help="micro-steps of the eagerly launched window that times the dominant kernel")
     ap.add_argument("--plain", type=int, default=32, help="plain GPU dimer searches")
     ap.add_argument("--no-cpu", action="store_true")
     ap.add_argument("--skin", type=float, default=None, help="Verlet skin of the device lists (A)")
@@ -708,21 +706,8 @@ def main():
         if r >= args.warmup:
             t_timed += st.search_time
             tot.add(st)
-    # ---- the dominant kernel timed with HIP events on the batch's stream over a
-    # window of the same searches that follows the timed ones (events inside
-    # replayed graphs cannot be timed, so this window launches eagerly), with
-    # the FP32 evaluations each walker consumed there
     camp.drain()
-    counts0 = camp.batch.eval_counts()
-    camp.batch.kernel_timer(True)
-    rst = camp.advance(args.roofline_window, sync_every=25)
-    k_ms, k_launches = camp.batch.kernel_time()
-    evals = camp.batch.eval_counts() - counts0
-    camp.batch.kernel_timer(False)
-    timed_ms = k_ms / max(k_launches, 1)
-    print(f"[bench] pass 2 in the roofline window: {k_launches} launches, {timed_ms:.4f} ms per launch "
-          f"({int(evals.sum())} walker evaluations)", file=sys.stderr, flush=True)
-    # ---- the pass kernels as the search micro-steps run them (active zones),
+    # ---- one evaluation of every search walker as the micro-steps run it,
     # timed with HIP events on the batch's stream at the searches' current
     # probes, after one warm evaluation that does any pending full one; the
     # algorithmic work from the device's zones and the free-atom masks
@@ -832,7 +817,6 @@ def main():
                      "flops_per_launch": round(SEARCH_PAIR_FLOP * zw["pairs_free"]),
                      "flop_per_pair": SEARCH_PAIR_FLOP,
                      "zones": zw,
-                     "window_k_sc_force_ms_per_launch": round(timed_ms, 4),
                      "full_evaluation": {"kernel": "k_sc_force over every atom of every walker at the basins",
                                          "ms_per_launch": round(force_ms, 4), "flops_per_launch": 40 * Ptot,
                                          "tflops": round(achieved_tf, 3),

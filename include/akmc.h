@@ -171,7 +171,9 @@ long long akmc_batch_rebuilds(akmc_batch_t b);
  * Each walker advances by "micro-steps": one batched force evaluation at
  * the walker's probe positions followed by one update of its state
  * machine.  All walkers of a batch move together; finished walkers are
- * skipped by the force kernels. */
+ * skipped by the force kernels.  (One exception: a search whose zone
+ * outgrows the resident kernel in a chunk in which every walker is resident
+ * makes its next step in the next chunk; akmc_batch_set_resident.) */
 
 /* RelaxCntrl (Common/RelaxCntrl.h:15-48).  Relax::RelaxStructure
  * (optim/Relax.cpp:19-42) dispatches on method: AKMC_RELAX_FIRE is

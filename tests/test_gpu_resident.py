@@ -1,7 +1,7 @@
 """Resident searches (search_resident.hip) at the edges of their ranges: one
 free atom, the most free atoms a resident walker takes and one more (the
-chain), a scattered free set past the list-build capacity (the walker goes
-back to the chain), cells smaller and larger than the zone, and the three
+chain), a scattered free set that reaches more atoms than one holds (the
+chain), cells smaller and larger than the zone, and the three
 kinds of pair table (one species; n = 9, m = 6 throughout; any exponents),
 in both precisions.
 
@@ -56,6 +56,7 @@ def test_resident_evaluation_equals_force_call(kind, shape, nfree, scattered, bi
     b.set_frozen([frozen, frozen])
     b.start_relax(L.relax_defaults(maxIter=30, maxTimeStep=0.003, initTimeStep=0.002))
     b.run(400, sync_every=13)
+    assert (((b.zone()[2] & 16) != 0) == (nfree <= 256 and not scattered)).all()  # which path it was
     st = b.status()
     pos = b.positions()
     frc = b.download()[1]

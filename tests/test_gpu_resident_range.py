@@ -56,6 +56,14 @@ def test_compact_region_is_resident(shape, nfree, bits):
     _check(f, b, [c], [frozen], bits)
 
 
+def test_one_free_atom_more_takes_the_chain():
+    c = W.sc_cell(8, 8, 8, n_vac=1, jitter=0.02, seed=5)
+    frozen = _nearest(c, 257)
+    f, b = _relax([c], [frozen], 64)
+    assert not b.zone()[2][0] & 16
+    _check(f, b, [c], [frozen], 64)
+
+
 def test_two_separated_clusters_are_resident():
     c = W.sc_cell(10, 10, 10, n_vac=1, jitter=0.02, seed=6)
     frozen = _nearest(c, 60)
