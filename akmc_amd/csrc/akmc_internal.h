@@ -378,9 +378,17 @@ struct SearchDev {
 // velocities alone)
 #define AKMC_FIRE_ATOMS 4096
 
-// after pass 1 of the chain: what frozen neighbours contribute to the
-// density and pair energy of every atom of the resident walkers it serves
-void akmc_launch_res_base(const BatchDev &b, const FieldDev &hf, hipStream_t st);
+// precisions (AKMC_ZONE_FULL bits) that the searches may evaluate in: FP64
+// when they are verified or relaxes end with an FP64 energy
+inline __host__ __device__ int akmc_res_precisions(const SearchDev &s)
+{
+    return (s.default_mode != 2 ? AKMC_ZONE_FULL32 : 0) |
+           (s.default_mode == 2 || s.verify_nl > 0 || s.final64 ? AKMC_ZONE_FULL64 : 0);
+}
+// after pass 1 of the chain: what frozen neighbours contribute to the density
+// and pair energy of every atom of the resident walkers for which it is
+// pending, in those precisions and the walkers' current ones
+void akmc_launch_res_base(const BatchDev &b, const FieldDev &hf, int precisions, hipStream_t st);
 // up to nsteps micro-steps of every resident walker (evaluation and state
 // machine), those waiting for the chain's full evaluation among them when
 // service is set; logic 0: one evaluation each, nothing else

@@ -1382,7 +1382,7 @@ void enqueue_chain(akmc_batch_t b, const BatchDev &d, bool base, bool sums, int 
     const int prec = batch_mode(b) | ((b->s.verify_nl > 0 || b->s.final64) ? 2 : 0);
     const FieldDev &hf = b->f->host;
     for (int ph = 0; ph < 2; ++ph) akmc_launch_phase(d, hf, prec, 0, ph, b->stream);
-    if (base) akmc_launch_res_base(d, hf, b->stream);
+    if (base) akmc_launch_res_base(d, hf, akmc_res_precisions(b->s), b->stream);
     if (b->ktimer && (prec & 1) && hf.kind == 0) {
         (void)hipEventRecord(b->kev[0][j], b->stream);
         akmc_launch_phase(d, hf, 1, 0, 2, b->stream);
@@ -2659,7 +2659,7 @@ static int time_search_phases_prec(akmc_batch_t b, int prec, int nrep, bool chai
             akmc_launch_phase(d, b->f->host, prec, 0, ph, b->stream);
             // resident walkers: their whole evaluation is timed with pass 1
             if (ph == 1 && res) {
-                akmc_launch_res_base(d, b->f->host, b->stream);
+                akmc_launch_res_base(d, b->f->host, akmc_res_precisions(b->s), b->stream);
                 akmc_launch_search_resident(b->W, b->f->host, b->res_args, 1, 0, 1, b->stream);
             }
             HIPCHK(hipEventRecord(b->evp[ph + 1], b->stream));

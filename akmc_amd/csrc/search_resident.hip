@@ -7,7 +7,7 @@
 // frozen neighbours, fixed for the whole search, and a part from the free
 // atoms in reach.  The chain (list build, all-atom passes) evaluates a
 // walker once, on its first micro-step, and k_res_base keeps the fixed parts
-// of both precisions; from then on an evaluation visits
+// in the precisions it may come to; from then on an evaluation visits
 //   - the free atoms' own neighbours (densities, then forces), and
 //   - per frozen atom of the zone, the free atoms in reach (a bit mask),
 // about 35,000 pairs for the 75 free atoms of a 6 A region against 160,000
@@ -733,11 +733,14 @@ __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *ar
         const int mode = step == 0 ? b.active[wid]
                                    : (L.ws.kind == WK_VERIFY || L.ws.state == ST_R_E64) ? 2 : s.default_mode;
         const int prec = mode == 2 ? 1 : 0;
-        if (flags & (AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64)) {
-            if (step > 0 || !service) break;
-            flags &= ~(AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64);
-            eok = 0;
+        const int full = prec ? AKMC_ZONE_FULL64 : AKMC_ZONE_FULL32;
+        if (step == 0 && service) {  // the fixed parts that k_res_base has just made
+            const int made = flags & (akmc_res_precisions(s) | full);
+            flags &= ~made;
+            if (made & AKMC_ZONE_FULL32) eok &= ~1;
+            if (made & AKMC_ZONE_FULL64) eok &= ~2;
         }
+        if (flags & full) break;
         bool moved = nz < 0;
         for (int f = tid; f < nf; f += kBlock) {
             const int i = W.off + L.fid[f];
@@ -825,69 +828,89 @@ struct Sum2 {
 
 constexpr int kBaseLanes = 4, kBaseSplit = 16, kBaseBlock = 256;
 
-template <typename T, int KIND>
+// (one pass over the lists for both precisions: the list and position loads
+// bound it)
+template <int KIND, bool F32, bool F64>
 __device__ inline void res_base_atoms(const BatchDev &b, const WalkerDev &W, const SCPairDev *tab)
 {
-    constexpr int prec = sizeof(T) == 8 ? 1 : 0;
     const FieldDev &F = *b.field;
-    const SCCoef<T> c1 = sc_coef<T>(F.sc[0]);
+    const SCCoef<float> c32 = sc_coef<float>(F.sc[0]);
+    const SCCoef<double> c64 = sc_coef<double>(F.sc[0]);
     const int sub = threadIdx.x % kBaseLanes;
     constexpr int per = kBaseBlock / kBaseLanes;
     for (int l = blockIdx.y * per + (int)threadIdx.x / kBaseLanes; l < W.n; l += kBaseSplit * per) {
         const int i = W.off + l, cnt = b.nnb[i];
         const double xi = b.x[i], yi = b.y[i], zi = b.z[i];
-        Sum2 rho{0.0, 0.0}, ep{0.0, 0.0};
+        Sum2 sum[4] = {};  // density, half pair energy; FP32, FP64
         for (int k = sub; k < cnt; k += kBaseLanes) {
             const int j = W.off + int(nbr_entry(b, k, i) & AKMC_NB_JMASK);
             const bool ok[1] = {b.zfrozen[j] != 0};
             const double px[1] = {b.x[j]}, py[1] = {b.y[j]}, pz[1] = {b.z[j]};
             const SCPairDev *p[1] = {KIND == 1 ? nullptr : tab + b.type[i] * F.nspec + b.type[j]};
-            double r = 0.0, e = 0.0;
-            add_density<T, KIND, 1>(W, F.rc2, c1, p, xi, yi, zi, px, py, pz, ok, r, e);
-            rho.add(r);
-            ep.add(e);
+            if constexpr (F32) {
+                double r = 0.0, e = 0.0;
+                add_density<float, KIND, 1>(W, F.rc2, c32, p, xi, yi, zi, px, py, pz, ok, r, e);
+                sum[0].add(r);
+                sum[1].add(e);
+            }
+            if constexpr (F64) {
+                double r = 0.0, e = 0.0;
+                add_density<double, KIND, 1>(W, F.rc2, c64, p, xi, yi, zi, px, py, pz, ok, r, e);
+                sum[2].add(r);
+                sum[3].add(e);
+            }
         }
-        for (int o = kBaseLanes / 2; o > 0; o >>= 1) {
-            const double rh = __shfl_xor(rho.h, o), rl = __shfl_xor(rho.l, o);
-            const double eh = __shfl_xor(ep.h, o), el = __shfl_xor(ep.l, o);
-            rho.add(rh);
-            rho.l += rl;
-            ep.add(eh);
-            ep.l += el;
-        }
+#pragma unroll
+        for (int v = F32 ? 0 : 2; v < (F64 ? 4 : 2); ++v)
+            for (int o = kBaseLanes / 2; o > 0; o >>= 1) {
+                const double h = __shfl_xor(sum[v].h, o), lo = __shfl_xor(sum[v].l, o);
+                sum[v].add(h);
+                sum[v].l += lo;
+            }
         if (sub == 0) {
-            b.r.base_rho[prec][i] = rho.h + rho.l;
-            b.r.base_ep[prec][i] = ep.h + ep.l;
+            if constexpr (F32) {
+                b.r.base_rho[0][i] = sum[0].h + sum[0].l;
+                b.r.base_ep[0][i] = sum[1].h + sum[1].l;
+            }
+            if constexpr (F64) {
+                b.r.base_rho[1][i] = sum[2].h + sum[2].l;
+                b.r.base_ep[1][i] = sum[3].h + sum[3].l;
+            }
         }
     }
 }
 
 // The parts of every atom's density and pair energy that come from frozen
-// neighbours, in both precisions, for the resident walkers on their first
-// micro-step (kBaseSplit workgroups per walker).  A search goes over to FP64
-// at its verification; with these parts at hand it does so without waiting
-// for an evaluation of the chain.
+// neighbours, for the resident walkers on their first micro-step (kBaseSplit
+// workgroups per walker), in every precision that the searches may come to: a
+// search goes over to FP64 at its verification, and with these parts at hand
+// it does so without waiting for an evaluation of the chain.  (When
+// verification is turned on under running searches the FP64 parts follow with
+// the next chunk, from the same lists: frozen atoms do not move.)
 template <int KIND>
-__global__ void __launch_bounds__(kBaseBlock) k_res_base(BatchDev b)
+__global__ void __launch_bounds__(kBaseBlock) k_res_base(BatchDev b, int precisions)
 {
     __shared__ SCPairDev tab[KIND == 1 ? 1 : kResSpec * kResSpec];
     const int w = blockIdx.x, mode = b.active[w], f = b.zflag[w];
-    if (mode == 0 || !(f & AKMC_ZONE_RES) || !(f & (AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64))) return;
+    const int todo = f & (precisions | (mode == 2 ? AKMC_ZONE_FULL64 : AKMC_ZONE_FULL32)) &
+                     (AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64);
+    if (mode == 0 || !(f & AKMC_ZONE_RES) || !todo) return;
     if constexpr (KIND != 1) stage_sc_table(*b.field, tab);
     const WalkerDev W = b.walkers[w];
-    res_base_atoms<float, KIND>(b, W, tab);
-    res_base_atoms<double, KIND>(b, W, tab);
+    if (!(todo & AKMC_ZONE_FULL64)) res_base_atoms<KIND, true, false>(b, W, tab);
+    else if (!(todo & AKMC_ZONE_FULL32)) res_base_atoms<KIND, false, true>(b, W, tab);
+    else res_base_atoms<KIND, true, true>(b, W, tab);
 }
 
 }  // namespace
 
-void akmc_launch_res_base(const BatchDev &b, const FieldDev &hf, hipStream_t st)
+void akmc_launch_res_base(const BatchDev &b, const FieldDev &hf, int precisions, hipStream_t st)
 {
     const dim3 g(b.W, kBaseSplit);
     switch (akmc_sc_kind(hf)) {
-    case 1: k_res_base<1><<<g, kBaseBlock, 0, st>>>(b); break;
-    case 2: k_res_base<2><<<g, kBaseBlock, 0, st>>>(b); break;
-    default: k_res_base<0><<<g, kBaseBlock, 0, st>>>(b);
+    case 1: k_res_base<1><<<g, kBaseBlock, 0, st>>>(b, precisions); break;
+    case 2: k_res_base<2><<<g, kBaseBlock, 0, st>>>(b, precisions); break;
+    default: k_res_base<0><<<g, kBaseBlock, 0, st>>>(b, precisions);
     }
 }
 

@@ -73,3 +73,31 @@ def test_steps_are_steps(searches):
             for a, b in zip(pos, pos2):
                 assert np.array_equal(a, b), (steps, kw)
     assert len(kinds) > 1 and (st["verified"] == 1).any()  # searches caught in their verification too
+
+
+def test_verification_turned_on_under_running_searches(searches):
+    """The FP64 fixed parts follow with the next chunk: the same bits, step by
+    step, as with verification on from the start."""
+    L, f = _field()
+    cells, (frozen, modes, x0) = searches
+    out = []
+    for late in (False, True):
+        b = L.Batch(f, cells)
+        if not late:
+            b.set_verify(16, 0.01)
+        b.start_dimer(modes, params=L.dimer_defaults(maxParIter=400), x0_per_walker=x0, frozen_per_walker=frozen)
+        b.run(100, sync_every=25)
+        assert (b.zone()[2] == (21 if late else 17)).all()  # the FP64 parts are pending
+        if late:
+            b.set_verify(16, 0.01)
+        b.run(160, sync_every=20)
+        part = b.status_array()
+        assert (part["kind"] == 3).any() and (part["force_calls"][part["done"] == 0] == 260).all()
+        b.run(400, sync_every=20)
+        out.append((part, b.status_array(), b.positions()))
+    for k in out[0][0].dtype.names:
+        assert np.array_equal(out[0][0][k], out[1][0][k], equal_nan=True), k
+        assert np.array_equal(out[0][1][k], out[1][1][k], equal_nan=True), k
+    assert (out[0][1]["verified"] == 1).any()
+    for p, q in zip(out[0][2], out[1][2]):
+        assert np.array_equal(p, q)
