@@ -345,6 +345,7 @@ struct WalkerState {
     int b2_new, b2_status, b2_calls, b2_iters;
     int fire_done;  // k_relax_fire advanced the walker on this micro-step
     int left;  // its lists do not fit the resident kernel: the chain advances it
+    int waits;  // it needs fixed parts that its last chunk did not bring
 };
 
 struct SearchDev {

@@ -1398,27 +1398,47 @@ void enqueue_chain(akmc_batch_t b, const BatchDev &d, bool base, bool sums, int 
 // relax kernel (part of SearchDev, so that a captured graph is for one answer)
 bool relax_fire(akmc_batch_t b) { return b->s.fire_on != 0; }
 
-// The kernels of a chunk of micro-steps, res as resident_mode.  A resident
-// walker needs the chain once, on its first micro-step, and a walker starts
-// between chunks: one chain evaluation serves those of a chunk, one resident
-// launch takes all its micro-steps, and the chain goes on for the other
-// walkers alone.  With zones off the chain evaluates every atom on every
-// step; the kernel timer times a chain launch of every step.
-void enqueue_steps(akmc_batch_t b, int steps, int res)
+// some running resident walker waits for its fixed parts (the host's flags
+// hold every bit that the device's do)
+bool parts_pending(akmc_batch_t b)
+{
+    const int want = akmc_res_precisions(b->s);
+    for (int w = 0; w < b->W; ++w) {
+        const WalkerState &ws = b->hws[w];
+        if (ws.kind == WK_IDLE || ws.state == ST_DONE || !(b->hzflag[w] & AKMC_ZONE_RES)) continue;
+        if ((b->hzflag[w] & want) || ws.waits) return true;
+    }
+    return false;
+}
+
+// what a chunk's kernels depend on beside the descriptors
+struct ChunkPlan {
+    int res;       // resident_mode
+    bool service;  // parts_pending
+};
+
+// The kernels of a chunk of micro-steps.  A resident walker needs the chain
+// once, on its first micro-step, and a walker starts between chunks: where one
+// has started, one chain evaluation serves the chunk; one resident launch takes
+// all the chunk's micro-steps, and the chain goes on for the other walkers
+// alone.  With zones off the chain evaluates every atom on every step; the
+// kernel timer times a chain launch of every step.
+void enqueue_steps(akmc_batch_t b, int steps, const ChunkPlan &p)
 {
     const BatchDev d = step_dev(b);
     const bool fire = relax_fire(b), every = !b->zone_on || b->ktimer;
+    const int chain = p.res < 2 || every ? steps : p.service ? 1 : 0;
     for (int j = 0; j < steps; ++j) {
-        if (res == 2 && j > 0 && !every) break;
-        enqueue_chain(b, d, res && j == 0, res < 2, j);
+        if (j < chain) enqueue_chain(b, d, p.res && j == 0 && p.service, p.res < 2, j);
         // walkers of tens of thousands of atoms: 1024-thread state machines
-        if (res < 2) {
+        if (p.res < 2) {
             if (fire) akmc_launch_relax_fire(d, b->s, b->stream);
             if (b->logic_wide) akmc_launch_search_logic_wide(d, b->s, b->stream);
             else akmc_launch_search_logic(d, b->s, b->stream);
         }
-        if (res && (j == 0 || every))
-            akmc_launch_search_resident(b->W, b->f->host, b->res_args, every ? 1 : steps, 1, j == 0, b->stream);
+        if (p.res && (j == 0 || every))
+            akmc_launch_search_resident(b->W, b->f->host, b->res_args, every ? 1 : steps, 1, j == 0 && p.service,
+                                        b->stream);
     }
 }
 
@@ -1619,18 +1639,18 @@ int load_walkers(akmc_batch_t b, const int *walkers, const double *x0, const dou
 int copy_walkers_out(akmc_batch_t b, const double *src, int nw, const int *walkers, double *out);
 int copy_walkers_out3(akmc_batch_t b, const double *const src[3], int nw, const int *walkers, double *out);
 
-int capture_graph(akmc_batch_t b, int steps, int res)
+int capture_graph(akmc_batch_t b, int steps, const ChunkPlan &plan)
 {
     drop_graph(b);
     HIPCHK(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-    enqueue_steps(b, steps, res);
+    enqueue_steps(b, steps, plan);
     hipGraph_t g = nullptr;
     hipError_t e = hipStreamEndCapture(b->stream, &g);
     if (e != hipSuccess) return fail(AKMC_EHIP, "graph capture failed: %s", hipGetErrorString(e));
     b->graph = g;
     HIPCHK(hipGraphInstantiate(&b->gexec, g, nullptr, nullptr, 0));
     b->graph_steps = steps;
-    b->graph_res = res;
+    b->graph_res = 2 * plan.res + plan.service;
     b->graph_args = b->s;
     b->graph_d = step_dev(b);
     b->graph_prec = batch_mode(b);
@@ -2145,7 +2165,7 @@ int launch_chunk(akmc_batch_t b, int steps, int running)
     }
     // HIP events recorded inside a replayed graph cannot be timed, so the
     // kernel timer launches the micro-steps one by one
-    const int res = resident_mode(b);
+    const ChunkPlan plan{resident_mode(b), parts_pending(b)};
     b->s.fire_on = 0;
     if (b->s.rp.method == AKMC_RELAX_FIRE && !b->s.rp.verlet)
         for (int w = 0; w < b->W && !b->s.fire_on; ++w)
@@ -2154,15 +2174,20 @@ int launch_chunk(akmc_batch_t b, int steps, int running)
     TRY(sync_res_args(b));
     if (b->use_graphs && !b->ktimer) {
         const BatchDev bd = step_dev(b);
-        if (!b->gexec || b->graph_steps != steps || b->graph_res != res || b->graph_prec != batch_mode(b) ||
+        if (!b->gexec || b->graph_steps != steps || b->graph_res != 2 * plan.res + plan.service || b->graph_prec != batch_mode(b) ||
             std::memcmp(&b->graph_args, &b->s, sizeof(SearchDev)) != 0 ||
             std::memcmp(&b->graph_d, &bd, sizeof(BatchDev)) != 0)
-            TRY(capture_graph(b, steps, res));
+            TRY(capture_graph(b, steps, plan));
         HIPCHK(hipGraphLaunch(b->gexec, b->stream));
     } else {
-        enqueue_steps(b, steps, res);
+        enqueue_steps(b, steps, plan);
         HIPCHK(hipGetLastError());
     }
+    // the running resident walkers get their parts (the device clears the same
+    // bits, and their current mode's)
+    for (int w = 0; w < b->W; ++w)
+        if ((b->hzflag[w] & AKMC_ZONE_RES) && b->hws[w].kind != WK_IDLE && b->hws[w].state != ST_DONE)
+            b->hzflag[w] &= ~akmc_res_precisions(b->s);
     if (b->hv_on) {
         // the buffer the host read two waits ago
         b->hv_cur ^= 1;
@@ -2279,7 +2304,8 @@ int akmc_batch_run(akmc_batch_t b, int max_steps, int sync_every, int *steps_don
     int done = 0, running = 1;
     while (running > 0 && done < max_steps) {
         int k = std::min(sync_every, max_steps - done), got = 0;
-        TRY(akmc_batch_run_async(b, k));
+        // nothing but the chunks changes the walkers from here on
+        TRY(done == 0 ? akmc_batch_run_async(b, k) : akmc_batch_run_next(b, k));
         TRY(akmc_batch_run_wait(b, &got, &running));
         if (got == 0) break;
         done += got;

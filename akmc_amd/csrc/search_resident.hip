@@ -699,7 +699,10 @@ __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *ar
     const int wid = blockIdx.x, tid = threadIdx.x;
     int flags = b.zflag[wid];
     if (!(flags & AKMC_ZONE_RES) || b.active[wid] == 0) return;
-    if (tid == 0) L.ws = s.ws[wid];
+    if (tid == 0) {
+        L.ws = s.ws[wid];
+        L.ws.waits = 0;
+    }
     if constexpr (KIND != 1) stage_sc_table(*b.field, L.tab);
     __syncthreads();
     if (L.ws.kind == WK_IDLE || L.ws.state == ST_DONE) return;
@@ -740,7 +743,10 @@ __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *ar
             if (made & AKMC_ZONE_FULL32) eok &= ~1;
             if (made & AKMC_ZONE_FULL64) eok &= ~2;
         }
-        if (flags & full) break;
+        if (flags & full) {
+            if (tid == 0) L.ws.waits = 1;
+            break;
+        }
         bool moved = nz < 0;
         for (int f = tid; f < nf; f += kBlock) {
             const int i = W.off + L.fid[f];
