@@ -19,9 +19,9 @@
 // of the rate of two on a CU), so a workgroup has eight wavefronts, two fit
 // a CU, the functions are out of line for 128 registers each, lists and
 // records are in LDS, and sums go by DPP moves.  512 walkers of 500-4000
-// atoms: 63 us per micro-step for evaluations and state machines, where the
+// atoms: 65 us per micro-step for evaluations and state machines, where the
 // chain's kernels took 293 us (91 us with four wavefronts and lists in
-// global memory); 12 walkers: 41 us against 104 us.
+// global memory); 12 walkers: 37 us against 104 us.
 //
 // A walker's results do not depend on its batch: whether it is resident, when
 // its lists are built and every order of summation follow from the walker
