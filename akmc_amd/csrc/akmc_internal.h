@@ -49,7 +49,6 @@ struct SCCoef {
     T rho_coef;  // (eps c)^2
     T fs_coef;   // n eps
     T fm_coef;   // 0.5 m (eps c)^2
-    T ha2;       // 1 / (2 a^2)
 };
 struct SCPairDev {
     SCCoef<float> f;

@@ -459,9 +459,9 @@ void build_tables(akmc_field_t f)
                 const SCPot &s = f->sc[k];
                 p.on = 1;
                 p.d = {s.a, s.n, s.m, s.eps, (s.eps * s.c) * (s.eps * s.c), s.n * s.eps,
-                       0.5 * s.m * (s.eps * s.c) * (s.eps * s.c), 0.5 / (s.a * s.a)};
+                       0.5 * s.m * (s.eps * s.c) * (s.eps * s.c)};
                 p.f = {(float)p.d.a, (float)p.d.n, (float)p.d.m, (float)p.d.eps, (float)p.d.rho_coef,
-                       (float)p.d.fs_coef, (float)p.d.fm_coef, (float)p.d.ha2};
+                       (float)p.d.fs_coef, (float)p.d.fm_coef};
                 auto as_int = [](double e) { return (e >= 0 && e <= 64 && std::floor(e) == e) ? (int)e : -1; };
                 p.n_int = as_int(s.n);
                 p.m_int = as_int(s.m);

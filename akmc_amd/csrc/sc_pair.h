@@ -129,7 +129,8 @@ __device__ inline void table_9_6(double r2, const SCCoef<T> &c, T &ir2, T &un, T
         const double ir = rsqrt_fp64(r2), q = ir * ir, s = c.a * ir;
         ir2 = fma(q, fma(-r2, q, 1.0), q);
         u2 = c.a * c.a * ir2;
-        rt = fma(fma(-s, s, u2), s * r2 * c.ha2, s);  // s r2 / (2 a^2) = 1 / (2 s)
+        // (the residual is a few units of s: 1 / (2 s) to FP32's bits is enough)
+        rt = fma(fma(-s, s, u2), double(0.5f * __builtin_amdgcn_rsqf(float(u2))), s);
     } else {
         ir2 = recip<T>(T(r2));
         u2 = c.a * c.a * ir2;
