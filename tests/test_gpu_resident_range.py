@@ -148,3 +148,40 @@ def test_a_zone_that_outgrows_the_kernel_goes_on_in_the_chain():
     b.run(3000, sync_every=10)
     assert not b.zone()[2][0] & 16
     _check(f, b, [cell], [frozen], 64)
+
+
+def test_starts_behind_a_chunk_in_flight():
+    """Two walkers started while a chunk runs, one that fits the resident
+    kernel and one that does not: both take a step with every micro-step of
+    the next chunk, and end as they do when started before it."""
+    from akmc_amd import lib as L
+    cells = [W.sc_cell(4, 4, 5, n_vac=1, jitter=0.02, seed=1), W.sc_cell(5, 4, 5, n_vac=1, jitter=0.02, seed=4),
+             W.sc_cell(9, 9, 9, n_vac=1, jitter=0.02, seed=2)]
+    frozen = [_nearest(cells[0], 60), _nearest(cells[1], 70), _scattered(cells[2], 200, 1)]
+    f = L.Field(L.sc_potentials_text(ONE, 2 * CU["a"]))
+    modes, x0 = [], []
+    for w, c in enumerate(cells):
+        disp, mode = W.local_displacement(c, W.neighbours_of_site(c, c.vacancies[0], 12), 0.1, w)
+        modes.append(mode)
+        x0.append(c.pos + disp)
+    modes[2] = np.random.default_rng(1).standard_normal((3, cells[2].n))  # its free atoms are everywhere
+    ends = []
+    for behind in (True, False):
+        b = L.Batch(f, cells)
+        kw = dict(x0_per_walker=x0, frozen_per_walker=frozen)
+        b.start_dimer(modes, walkers=[0], **kw)
+        if behind:
+            b.run_async(20)
+            b.start_dimer(modes, walkers=[1, 2], **kw)
+            b.run_wait()
+        else:
+            b.run(20, sync_every=20)
+            b.start_dimer(modes, walkers=[1, 2], **kw)
+        assert [int(v) & 16 for v in b.zone()[2]] == [16, 16, 0]
+        for _ in range(2):
+            b.run_next(15) if behind else b.run_async(15)
+            b.run_wait()
+        assert [s["force_calls"] for s in b.status()] == [50, 30, 30]
+        ends.append(b.positions())
+    for p, q in zip(*ends):
+        assert np.array_equal(p, q)
