@@ -28,6 +28,10 @@
 #define AKMC_ZONE_RES 16
 // a search walker's flags at its start on the chain
 #define AKMC_ZONE_FRESH (AKMC_ZONE_ON | AKMC_ZONE_FULL32 | AKMC_ZONE_FULL64 | AKMC_ZONE_RESET)
+// what the resident kernel reports of a walker: its lists do not fit (the
+// chain advances it), it needs fixed parts that its last chunk did not bring
+#define AKMC_RES_LEFT 1
+#define AKMC_RES_WAITS 2
 // capacities of a resident walker: free atoms, zone atoms, atoms of the
 // cell, candidates of its list build
 #define AKMC_RES_FREE 256
@@ -343,8 +347,7 @@ struct WalkerState {
     double eb2, eb2_64, b2_maxd2;
     int b2_new, b2_status, b2_calls, b2_iters;
     int fire_done;  // k_relax_fire advanced the walker on this micro-step
-    int left;  // its lists do not fit the resident kernel: the chain advances it
-    int waits;  // it needs fixed parts that its last chunk did not bring
+    int res;  // AKMC_RES_LEFT, AKMC_RES_WAITS
 };
 
 struct SearchDev {

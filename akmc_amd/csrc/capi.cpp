@@ -1119,7 +1119,7 @@ int upload(akmc_batch_t b, const double *x, const double *y, const double *z, co
         HIPCHK(hipMemcpyAsync(b->s.X + 2 * A, z, A * sizeof(double), hipMemcpyHostToDevice, b->stream));
     }
     HIPCHK(hipStreamSynchronize(b->stream));
-    if (b->zflag)
+    if (b->search_alloc)
         for (int w = 0; w < b->W; ++w) b->hzflag[w] = b->zf_pin[w] = 0;
     return AKMC_SUCCESS;
 }
@@ -1406,7 +1406,7 @@ bool parts_pending(akmc_batch_t b)
     for (int w = 0; w < b->W; ++w) {
         const WalkerState &ws = b->hws[w];
         if (ws.kind == WK_IDLE || ws.state == ST_DONE || !(b->hzflag[w] & AKMC_ZONE_RES)) continue;
-        if ((b->hzflag[w] & want) || ws.waits) return true;
+        if ((b->hzflag[w] & want) || (ws.res & AKMC_RES_WAITS)) return true;
     }
     return false;
 }
@@ -2246,7 +2246,7 @@ int akmc_batch_run_wait(akmc_batch_t b, int *steps_done, int *running)
             }
         std::memcpy(b->hws.data(), b->hws_pin, b->W * sizeof(WalkerState));
         for (int w = 0; w < b->W; ++w)  // its lists have outgrown the resident kernel
-            if (b->hws[w].left) b->hzflag[w] &= ~AKMC_ZONE_RES;
+            if (b->hws[w].res & AKMC_RES_LEFT) b->hzflag[w] &= ~AKMC_ZONE_RES;
         if (b->hv_on) b->hv_last = b->hv_inflight;
     } else {
         HIPCHK(hipStreamSynchronize(b->stream));  // starts queued since the launch

@@ -680,7 +680,7 @@ __device__ inline void leave(const BatchDev &b, const SearchDev &s, int w)
 {
     b.zflag[w] = AKMC_ZONE_FRESH;
     b.rebuild[w] = 1;
-    s.ws[w].left = 1;
+    s.ws[w].res |= AKMC_RES_LEFT;
 }
 
 // Micro-steps of resident walkers, one workgroup each.  service: the chain
@@ -701,7 +701,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *ar
     if (!(flags & AKMC_ZONE_RES) || b.active[wid] == 0) return;
     if (tid == 0) {
         L.ws = s.ws[wid];
-        L.ws.waits = 0;
+        L.ws.res &= ~AKMC_RES_WAITS;
     }
     if constexpr (KIND != 1) stage_sc_table(*b.field, L.tab);
     __syncthreads();
@@ -744,7 +744,7 @@ __global__ void __launch_bounds__(kBlock, 4) k_search_resident(const ResArgs *ar
             if (made & AKMC_ZONE_FULL64) eok &= ~2;
         }
         if (flags & full) {
-            if (tid == 0) L.ws.waits = 1;
+            if (tid == 0) L.ws.res |= AKMC_RES_WAITS;
             break;
         }
         bool moved = nz < 0;
